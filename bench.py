@@ -682,7 +682,8 @@ def bench_adi(torch, n=256, iters=20):
         step_ms, incl = timed(lambda k: adi.run(1.0, u, ws, k, graph=True, sync=True))
         out[key] = {"step_ms": round(step_ms, 4), "gpts_s": round(n ** 3 / step_ms / 1e6, 2),
                     "step_ms_incl_capture": round(incl, 4), "steps": iters,
-                    "bytes_per_point_step": 168 if key == "fp64" else 84}
+                    "bytes_per_point_step": 56 if key == "fp64" else 28,
+                    "bytes_per_point_call": 24 if key == "fp64" else 12}
         # matrix-free step: coefficients and right-hand side computed in the
         # sweeps, 56 (28) B/pt
         du = ws.du

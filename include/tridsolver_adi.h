@@ -26,7 +26,9 @@ EXTERN_C tridStatus_t tridAdiPreprocS(float lambda, const float *u, float *du, f
 
 /* One timestep (reference loop body apps/adi/src/adi_cuda.cu:283-325) with one
  * shared coefficient set a, b, c. ctx as for the solves (opts are hints for
- * the three sweeps); ctx->sync != 0 or ctx == NULL waits for completion. */
+ * the three sweeps); ctx->sync != 0 or ctx == NULL waits for completion. du
+ * and the coefficient arrays end as the reference's preproc and x, y solves
+ * leave them, also where the sweeps compute the coefficients themselves. */
 EXTERN_C tridStatus_t tridAdiStepD(const TridParams *ctx, double lambda, double *u,
                                    double *du, double *a, double *b, double *c, int nx,
                                    int ny, int nz);
@@ -48,8 +50,8 @@ EXTERN_C tridStatus_t tridAdiRunS(const TridParams *ctx, float lambda, float *u,
  * coefficient arrays, apps/adi/src/preproc.cu:77-85, from values fixed by
  * position, :59-73). The ADI coefficients depend only on the grid position,
  * so each sweep computes a, b, c from (i, j, k), and the x sweep computes its
- * right-hand side from u: 56 B per point per step at FP64 instead of 168,
- * same results bit for bit as tridAdiStep. du is workspace. */
+ * right-hand side from u: 56 B per point per step at FP64 instead of 168 with
+ * arrays read back, same results bit for bit as tridAdiStep. du is workspace. */
 EXTERN_C tridStatus_t tridAdiStepFusedD(double lambda, double *u, double *du, int nx, int ny,
                                         int nz);
 EXTERN_C tridStatus_t tridAdiStepFusedS(float lambda, float *u, float *du, int nx, int ny,

@@ -204,6 +204,45 @@ def test_fused_256_20_steps_equals_array(dtype):
     assert torch.equal(u, uf)
 
 
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 3, 3), (2, 5, 4), (33, 17, 9), (255, 6, 5),
+                                   (64, 32, 16), (7, 3, 8200)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_array_step_matrix_free_equals_preproc_and_solves(dtype, shape, shift):
+    """tridAdiRun's arrays written once, then matrix-free sweeps, against preproc
+    and the per-lane array solves (opts 1) of the same call: a, b, c bit for
+    bit; du and u normwise at the parity bars (1e-12 / 1e-5 against the exact
+    solve for either). Sizes that are no multiple of a 16-byte vector, arrays
+    one element off 16-byte alignment (shift), and a z line longer than a
+    strided workgroup holds (which keeps the array solves)."""
+    nx, ny, nz = shape
+    n = nx * ny * nz
+    tol = 1e-12 if dtype == torch.float64 else 1e-5
+
+    def fields():
+        class WS:
+            pass
+        ws = WS()
+        ws.shape = shape
+        for k in ("du", "a", "b", "c"):
+            setattr(ws, k, torch.full((n + 2,), 7.0, dtype=dtype, device="cuda")[shift:shift + n])
+        u = torch.empty(n + 2, dtype=dtype, device="cuda")[shift:shift + n]
+        u.copy_(torch.rand(n, dtype=dtype, device="cuda",
+                           generator=torch.Generator(device="cuda").manual_seed(21)))
+        return u, ws
+
+    (u, ws), (v, wv) = fields(), fields()
+    adi.run(0.9, u, ws, 2, graph=False, sync=True)
+    adi.run(0.9, v, wv, 2, graph=False, opts=(1, 1, 1), sync=True)
+    for k in ("a", "b", "c"):
+        assert torch.equal(getattr(ws, k), getattr(wv, k)), k
+    # after a step du is the y solve's output, u the field
+    for got, want in ((u, v), (ws.du, wv.du)):
+        scale = want.double().abs().max().item()
+        err = (got.double() - want.double()).abs().max().item()
+        assert err <= 2 * tol * max(scale, 1.0), (err, scale)
+
+
 def test_fused_rejects_bad_arguments():
     from tridsolver_amd import _lib
     L = _lib.lib()
