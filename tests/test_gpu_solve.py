@@ -198,6 +198,26 @@ def test_forced_wide_variant(G, inc, seg, dtype):
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("inc", [False, True])
+@pytest.mark.parametrize("dims,sd,seg", [
+    ([64, 33, 512], 1, 256),     # aligned rows (nontemporal), last wave partly past N
+    ([61, 300, 520], 1, 256),    # misaligned rows (plain access), partial last group
+    ([64, 512, 300], 2, 256), ([256, 8, 512], 2, 128),
+    ([16, 512, 2], 1, 128), ([16, 513, 2], 1, 128), ([40, 1023, 1], 1, 128),
+    ([17, 2, 1024], 2, 128), ([7, 1000, 1], 1, 128)])
+def test_default_strided_shapes(dims, sd, seg, inc, dtype):
+    """The default strided shapes at the edges of their ranges: 256-byte rows
+    for systems up to 512 rows in many workgroups, 128-byte rows else, up to 1024
+    rows; waves whose rows all lie inside their systems beside waves with rows
+    past N or systems past n0. FP32 may take 128-byte rows where FP64 takes
+    256."""
+    cfg = run_case(dims, sd, dtype, inc, (0, 0, 0), seed=sum(dims))
+    esize = np.dtype(dtype).itemsize
+    assert cfg[0] == 8
+    assert cfg[3] * esize in ((seg,) if dtype == np.float64 else (128, 256))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("inc", [False, True])
 @pytest.mark.parametrize("G", [1, 8])
 def test_forced_long32_contiguous(G, inc, dtype):
     """Contiguous systems of 4097-8192 rows, one per 256-thread workgroup at

@@ -631,6 +631,39 @@ __device__ __forceinline__ int64_t wave_uniform(int64_t v) {
   return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
+// Byte address of an LDS object inside the workgroup's LDS.
+__device__ __forceinline__ uint32_t lds_address(const void *p) {
+  return (uint32_t)(uintptr_t)(lds_void *)p;
+}
+
+// One global->LDS wave instruction: lane l's dword at base + off goes to LDS
+// byte lds + 4 l (lds wave-uniform). Written in asm because the compiler waits
+// for every outstanding load (vmcnt(0)) before a register load issued behind
+// the builtin is used; it does not see this one. It has no register
+// output. Loads complete in order, so the caller waits for it through a
+// register load that it issues after the staging: loads whose address passed
+// through loads_after_stage() come behind it, and stage_done(v) waits until v,
+// one of them, has arrived.
+__device__ __forceinline__ void stage_dword(uint32_t lds, const void *base, uint32_t off) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+               :
+               : "s"(lds), "v"(off), "s"(base)
+               : "m0", "memory");
+}
+__device__ __forceinline__ uint32_t loads_after_stage(uint32_t off) {
+  asm volatile("" : "+v"(off) : : "memory");
+  return off;
+}
+template <typename X>
+__device__ __forceinline__ void stage_done(X &v) {
+  asm volatile("" : "+v"(v) : : "memory");
+}
+// Waits for every load of the wave, staging included.
+__device__ __forceinline__ void stage_wait_all() {
+  __builtin_amdgcn_s_waitcnt(0);
+  asm volatile("" : : : "memory");
+}
+
 // `fetched()` runs once b is in chunk order (after a barrier that follows
 // the loads); a persistent caller decodes its next item there.
 template <typename REAL, bool INC, int T, typename OnFetched>

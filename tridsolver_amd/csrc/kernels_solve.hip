@@ -338,21 +338,36 @@ bool hybrid_plain_cfg(const Geom &g, HybridCfg *cfg) {
 template <typename REAL>
 bool hybrid_default_cfg(const Geom &g, HybridCfg *cfg) {
   if (g.stride != 1) {
-    // Strided systems: the variant with a staged in LDS, shapes measured
-    // at 256^3-512^3. Rows at least 64 KiB apart (z) lie in different pages:
-    // FP64 takes 256-byte rows (M = 32 above 256 rows) in plain workgroup
-    // order, FP32 128-byte rows. Rows close together (y) take 128-byte rows,
-    // XCD-grouped.
+    // Strided systems: the wide variant (kernels_wide.hip). The lines below
+    // lie where both sides were measured, in three sets of arrays used in
+    // turn (so that no call finds its data in a cache), on 40 grids from
+    // 33 x 80 x 50 to 512^3:
+    //  - rows of 256 bytes where such a workgroup holds the system (N <= 512)
+    //    and there are at least two of them per CU: fewer row segments and
+    //    fewer misaligned edges per byte (FP64 777 x 300 x 250 y 504 against
+    //    532 us, 256^3 z 127 against 155). 128-byte rows otherwise: 60 x 64 x
+    //    512 z 17.2 against 19.3 us with half the workgroups.
+    //  - FP64 at 16 rows per lane (512^3 z 0.94 against 0.95 ms at 32, 251 x
+    //    300 x 300 y 213 against 222 us). FP32 at 32 rows per lane on 256-byte
+    //    rows of 257-512 (512^3 y 0.466 against 0.484 ms for 16 on 128-byte
+    //    rows) and above 512, else at 16 on 128-byte rows (203 x 170 x 300 y 52
+    //    against 55 us).
+    //  - workgroups dealt to the XCDs in 8 ranges (G), so that neighbouring
+    //    segments, which share lines where rows are misaligned, pass through
+    //    one L2 (777 x 300 x 250 z 494 against 544 us at G = 1); in plain order
+    //    where rows lie a power of two of at least 64 KiB apart (512^3 z 0.94
+    //    against 1.04 ms at G = 8, 256^3 z 127 against 140 us).
     HybridCfg c;
     const bool fp64 = sizeof(REAL) == 8;
     const int64_t row_bytes = g.stride * (int64_t)sizeof(REAL);
-    const bool far = row_bytes >= (64 << 10);
-    c.M = (far && fp64 && g.N > 256) ? 32 : 16;
-    c.W = ((far && fp64) ? 256 : 128) / (int)sizeof(REAL);
+    const int64_t wide_groups = (g.n0 * (int64_t)sizeof(REAL) + 255) / 256 * g.n1;
+    const bool wide = g.N <= 512 && (fp64 ? wide_groups >= 512 : g.N > 256 && wide_groups >= 1024);
+    c.M = fp64 || (!wide && g.N <= 512) ? 16 : 32;
+    c.W = (wide ? 256 : 128) / (int)sizeof(REAL);
     const int per_wave = std::max(1, 64 / c.W);
     c.P = (int)((g.N + c.M - 1) / c.M);
     c.P = (c.P + per_wave - 1) / per_wave * per_wave;
-    c.G = !far ? 8 : (fp64 || row_bytes >= (1 << 20)) ? 1 : 8;
+    c.G = row_bytes >= (64 << 10) && (row_bytes & (row_bytes - 1)) == 0 ? 1 : 8;
     c.V = 3;
     if (hybrid_cfg_valid<REAL>(g, c)) {
       *cfg = c;
