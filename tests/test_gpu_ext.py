@@ -466,6 +466,42 @@ def test_adjoint_long_vs_oracle(dims, sd, dtype):
     assert np.array_equal(lam_only[0].cpu().numpy(), out[0].cpu().numpy())
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("M,seg", [(16, 128), (16, 256), (32, 128), (32, 256)])
+@pytest.mark.parametrize("dims,sd", [
+    ([16, 64, 3], 1), ([37, 65, 2], 1), ([64, 2, 128], 2), ([33, 3, 31], 2), ([5, 1, 1], 1),
+    ([32, 256, 2], 1), ([70, 2, 255], 2)])
+def test_adjoint_wide(dims, sd, M, seg, dtype):
+    """The wide adjoint kernel against the oracle at the parity bars: rows that
+    fill the workgroup's chunks exactly (no row past the last is read) and not,
+    waves with and without rows past N or systems past n0, one-row systems,
+    aligned and misaligned rows, each gradient alone."""
+    esize = np.dtype(dtype).itemsize
+    W = seg // esize
+    per_wave = max(1, 64 // W)
+    P = -(-dims[sd] // M)
+    P = -(-P // per_wave) * per_wave
+    rng = np.random.default_rng(sum(dims) + M)
+    n = int(np.prod(dims))
+    a, b, c, d = H.diag_dominant(rng, n)
+    w = rng.standard_normal(n)
+    x = d.copy()
+    oracle.batch(a, b, c, x, ndim=len(dims), solvedim=sd, dims=dims)
+    a, b, c, x, w = (v.astype(dtype) for v in (a, b, c, x, w))
+    ref = oracle.adjoint(*(v.astype(np.float64) for v in (a, b, c, x, w)), ndim=len(dims),
+                         solvedim=sd, dims=dims)
+    tol = 1e-12 if dtype == np.float64 else 1e-5
+    t = [dev(v) for v in (a, b, c, x, w)]
+    with api.forced_hybrid(M, P, W, 8, 3):
+        for want in ((True, True, True), (True, None, None), (None, True, None),
+                     (None, None, True), (None, None, None)):
+            out = api.adjoint_strided_batch(*t, solvedim=sd, dims=dims, grad_a=want[0],
+                                            grad_b=want[1], grad_c=want[2], sync=True)
+            for got, exact in zip(out, ref):
+                if got is not None:
+                    H.assert_norm_close(got.cpu().numpy(), exact, tol=tol)
+
+
 def test_adjoint_long_autotune():
     """Tuning a geometry the adjoint kernel does not hold records the
     transposed path (nothing to time) and succeeds; the solve then runs it."""

@@ -26,6 +26,7 @@
 #include "../../include/tridsolver_hip.h"
 #include "hybrid_core.hpp"
 #include "trid_internal.h"
+#include "wide_core.hpp"
 
 namespace trid {
 namespace {
@@ -107,6 +108,138 @@ __global__ __launch_bounds__((AdjBounds<REAL, M>::threads)) void adjoint_kernel(
   }
   hyb::to_fetch<M, CONTIG>(L, l, tile);
   hyb::store<M, CONTIG, NT>(L, lam, l);
+}
+
+// The strided adjoint with the operand below the transpose's diagonal, c[n-1],
+// staged in LDS and the sweep following the loads (wide_core.hpp; what bounds a
+// strided solve and why this split: kernels_wide.hip). x's rows take c's place
+// in the tile during the PCR, so that the gradients' operands arrive while
+// nothing else is loaded and hold no registers; the rows next to the chunk's
+// come in two registers. The four outputs are written one array after the other
+// (256^3 FP64 y 231 against 237 us with all four row by row). Every output
+// stream is as long as an input's: with all gradients, nine streams at 256^3
+// FP64, y / z run at 5.2 / 4.9 TB/s, 231 / 246 us, against 251 / 261 with every
+// operand in registers (adjoint_kernel); lam alone at 5.9 TB/s (z 115 us).
+template <typename REAL, int M, int SEG, bool GRAD, bool NT>
+__global__ __launch_bounds__((wide::WideBounds<REAL, M>::threads)) void adjoint_wide_kernel(
+    Geom g, int P, int G, int slots, const REAL *__restrict__ a, const REAL *__restrict__ b,
+    const REAL *__restrict__ c, const REAL *__restrict__ x, const REAL *__restrict__ w,
+    REAL *__restrict__ lam, REAL *__restrict__ ga, REAL *__restrict__ gb,
+    REAL *__restrict__ gc) {
+  constexpr int W = wide::WideShape<REAL, SEG>::W;
+  constexpr int CH = 64 / W;  // chunks per wave
+  constexpr int PITCH = wide::wide_chunk_bytes(M, SEG);
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const hyb::Lane L = hyb::lane_of<false>(g, P, W, G);
+  hyb::Ring ring{smem_raw + (size_t)P * PITCH, (int)(3 * sizeof(REAL) * L.T), 0, slots};
+  const int lane = L.t & 63, wv = __builtin_amdgcn_readfirstlane(L.t >> 6);
+  const int N = (int)L.N;
+  const uint32_t tile = hyb::lds_address(smem_raw) + wv * CH * PITCH;
+  const int64_t first = hyb::wave_uniform(L.i0 - L.w);
+  const int64_t base0 = first + hyb::wave_uniform(L.i1) * g.st1, nsys = g.n0 - first;
+  const uint32_t os = (uint32_t)(L.stride * (int64_t)sizeof(REAL));
+  const int row0 = L.p * M;
+  const int rows = L.active ? N - row0 : 0;
+  const uint32_t ob = (uint32_t)(L.base + row0 * L.stride) * (uint32_t)sizeof(REAL);
+  REAL *xs = reinterpret_cast<REAL *>(reinterpret_cast<char *>(smem_raw) + L.p * PITCH) + L.w;
+  const bool whole = __all(rows >= M);
+  REAL rb[M], rc[M], rd[M], f_d, f_a, f_g;
+  if (whole)
+    wide::wide_sweep<REAL, M, SEG, CH, true, NT, 1>(c + base0, tile, wv * CH * M, lane, N, nsys,
+                                                    os, ob, row0, rows, xs, b, a, w, rb, rc, rd,
+                                                    f_d, f_a, f_g);
+  else
+    wide::wide_sweep<REAL, M, SEG, CH, false, NT, 1>(c + base0, tile, wv * CH * M, lane, N, nsys,
+                                                     os, ob, row0, rows, xs, b, a, w, rb, rc, rd,
+                                                     f_d, f_a, f_g);
+  REAL xprev = 0, xnext = 0;
+  uint32_t obs = ob;
+  asm volatile("" : "+v"(obs));  // offsets formed here, not held from the loads
+  if (GRAD) {
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    if (whole)
+      wide::wide_stage<REAL, M, SEG, CH, true>(x + base0, tile, wv * CH * M, ln, os, N, nsys);
+    else
+      wide::wide_stage<REAL, M, SEG, CH, false>(x + base0, tile, wv * CH * M, ln, os, N, nsys);
+    const char *xb = reinterpret_cast<const char *>(x);
+    if (row0 > 0 && rows > 0) xprev = *reinterpret_cast<const REAL *>(xb + (obs - os));
+    if (rows > M) xnext = *reinterpret_cast<const REAL *>(xb + (obs + (uint32_t)M * os));
+  }
+  REAL y, ym;
+  hyb::reduced_solve<REAL>(L, ring, rb[M - 1], rc[M - 1], rd[M - 1], f_d, f_a, f_g, y, ym);
+  if (GRAD) {
+    // every wave has its x rows before any wave stores (an output may be one
+    // of the inputs)
+    hyb::stage_wait_all();
+    __syncthreads();
+  }
+  if (!L.active) return;
+  rd[M - 1] = y;
+#pragma unroll
+  for (int r = M - 2; r >= 0; --r) rd[r] = rd[r] - rb[r] * ym - rc[r] * rd[r + 1];
+  auto put = [&](REAL *p, uint32_t off, REAL v) {
+    hyb::st<NT>(reinterpret_cast<REAL *>(reinterpret_cast<char *>(p) + off), v);
+  };
+#pragma unroll
+  for (int r = 0; r < M; ++r)
+    if (r < rows) put(lam, obs + (uint32_t)r * os, rd[r]);
+  if (GRAD) {
+    if (ga) {
+#pragma unroll
+      for (int r = 0; r < M; ++r)
+        if (r < rows)
+          put(ga, obs + (uint32_t)r * os,
+              row0 + r == 0 ? REAL(0) : -rd[r] * (r > 0 ? xs[(r - 1) * W] : xprev));
+    }
+    if (gb) {
+#pragma unroll
+      for (int r = 0; r < M; ++r)
+        if (r < rows) put(gb, obs + (uint32_t)r * os, -rd[r] * xs[r * W]);
+    }
+    if (gc) {
+#pragma unroll
+      for (int r = 0; r < M; ++r)
+        if (r < rows)
+          put(gc, obs + (uint32_t)r * os,
+              r + 1 < rows ? -rd[r] * (r + 1 < M ? xs[(r + 1) * W] : xnext) : REAL(0));
+    }
+  }
+}
+
+template <typename REAL, int M, int SEG, bool GRAD, bool NT>
+hipError_t launch_adjoint_wide_nt(const Geom &g, const HybridCfg &cfg, const REAL *a,
+                                  const REAL *b, const REAL *c, const REAL *x, const REAL *w,
+                                  REAL *lam, REAL *ga, REAL *gb, REAL *gc, hipStream_t st) {
+  const int slots = wide::wide_slots<REAL>(M, cfg.P, SEG);
+  const size_t lds = wide::wide_lds_bytes<REAL>(M, cfg.P, SEG, slots);
+  auto kern = adjoint_wide_kernel<REAL, M, SEG, GRAD, NT>;
+  static LdsGrant lds_granted;
+  {
+    hipError_t e = ensure_lds(reinterpret_cast<const void *>(kern), lds, lds_granted);
+    if (e != hipSuccess) return e;
+  }
+  const int64_t blocks = (g.n0 + cfg.W - 1) / cfg.W * g.n1;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(cfg.W * cfg.P), lds, st, g, cfg.P, cfg.G,
+                     slots, a, b, c, x, w, lam, ga, gb, gc);
+  return hipGetLastError();
+}
+
+template <typename REAL, int M, int SEG>
+hipError_t launch_adjoint_wide(const Geom &g, const HybridCfg &cfg, const REAL *a, const REAL *b,
+                               const REAL *c, const REAL *x, const REAL *w, REAL *lam, REAL *ga,
+                               REAL *gb, REAL *gc, hipStream_t st) {
+  const bool grad = ga || gb || gc;
+  uintptr_t low = (uintptr_t)a | (uintptr_t)b | (uintptr_t)w | (uintptr_t)lam;
+  if (grad) low |= (uintptr_t)x | (uintptr_t)ga | (uintptr_t)gb | (uintptr_t)gc;
+  const bool nt = wide::wide_rows_aligned<REAL>(g, low);
+#define TRID_ADJ_WIDE(GRAD, NT)                                                          \
+  return launch_adjoint_wide_nt<REAL, M, SEG, GRAD, NT>(g, cfg, a, b, c, x, w, lam, ga, gb, gc, st)
+  if (grad && nt) TRID_ADJ_WIDE(true, true);
+  if (grad) TRID_ADJ_WIDE(true, false);
+  if (nt) TRID_ADJ_WIDE(false, true);
+  TRID_ADJ_WIDE(false, false);
+#undef TRID_ADJ_WIDE
 }
 
 // Nontemporal loads and stores except for strided systems whose rows are
@@ -219,8 +352,16 @@ hipError_t launch_adjoint_grads(const Geom &g, const REAL *x, const REAL *lam, R
   return hipGetLastError();
 }
 
+// Variant 3 on a shape that wide kernels hold takes adjoint_wide_kernel; every
+// other variant number, and variant 3 on another shape, adjoint_kernel.
+template <typename REAL>
+static bool adjoint_wide(const Geom &g, const HybridCfg &c) {
+  return c.V == 3 && wide::wide_shape_fits<REAL>(g, c);
+}
+
 template <typename REAL>
 bool adjoint_cfg_valid(const Geom &g, const HybridCfg &c) {
+  if (adjoint_wide<REAL>(g, c)) return true;
   // FP64 M = 16 on contiguous systems spills a few registers; not offered.
   if (sizeof(REAL) == 8 && c.M == 16 && g.stride == 1) return false;
   const int maxT = adj_max_threads<REAL>(c.M);
@@ -235,9 +376,22 @@ bool adjoint_cfg_valid(const Geom &g, const HybridCfg &c) {
 
 template <typename REAL>
 bool adjoint_default_cfg(const Geom &g, HybridCfg *cfg) {
-  // Same shapes as the forward solve where they fit the adjoint's register
-  // budget, else the next valid one.
+  // Strided systems: the forward solve's wide shape. Otherwise the same shapes
+  // as the forward solve where they fit the adjoint's register budget, else
+  // the next valid one.
   HybridCfg c;
+  if (g.stride != 1 && hybrid_default_cfg<REAL>(g, &c) && adjoint_wide<REAL>(g, c)) {
+    if (sizeof(REAL) == 4 && g.N <= 512 && wide::wide_many_groups<REAL>(g)) {
+      // nine streams of 128-byte rows want more bytes per row than the
+      // solve's five: 256-byte rows at every length (256^3 FP32 y / z 108 /
+      // 113 against 114 / 127 us, 203 x 170 x 300 z 117 against 128)
+      c.M = g.N > 256 ? 32 : 16;
+      c.W = 64;
+      c.P = (int)((g.N + c.M - 1) / c.M);
+    }
+    *cfg = c;
+    return true;
+  }
   if (hybrid_plain_cfg<REAL>(g, &c)) {
     for (int k = 0; k < 4 && !adjoint_cfg_valid<REAL>(g, c); ++k) {
       if (g.stride == 1 && c.W > 1) c.W /= 2;
@@ -262,6 +416,14 @@ hipError_t launch_adjoint(const Geom &g, const HybridCfg &cfg, const REAL *a, co
                           const REAL *c, const REAL *x, const REAL *w, REAL *lam, REAL *ga,
                           REAL *gb, REAL *gc, hipStream_t st) {
   const bool contig = g.stride == 1, grad = ga || gb || gc;
+  if (adjoint_wide<REAL>(g, cfg)) {
+    const bool s256 = cfg.W * (int)sizeof(REAL) == 256;
+    if (cfg.M == 16)
+      return s256 ? launch_adjoint_wide<REAL, 16, 256>(g, cfg, a, b, c, x, w, lam, ga, gb, gc, st)
+                  : launch_adjoint_wide<REAL, 16, 128>(g, cfg, a, b, c, x, w, lam, ga, gb, gc, st);
+    return s256 ? launch_adjoint_wide<REAL, 32, 256>(g, cfg, a, b, c, x, w, lam, ga, gb, gc, st)
+                : launch_adjoint_wide<REAL, 32, 128>(g, cfg, a, b, c, x, w, lam, ga, gb, gc, st);
+  }
 #define TRID_ADJ_CASE(MM)                                                                  \
   case MM:                                                                                 \
     if (grad)                                                                              \

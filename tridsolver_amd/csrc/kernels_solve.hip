@@ -55,6 +55,7 @@
 
 #include "hybrid_core.hpp"
 #include "trid_internal.h"
+#include "wide_core.hpp"
 
 namespace trid {
 namespace {
@@ -343,14 +344,14 @@ bool hybrid_default_cfg(const Geom &g, HybridCfg *cfg) {
     // turn (so that no call finds its data in a cache), on 40 grids from
     // 33 x 80 x 50 to 512^3:
     //  - rows of 256 bytes where such a workgroup holds the system (N <= 512)
-    //    and there are at least two of them per CU: fewer row segments and
-    //    fewer misaligned edges per byte (FP64 777 x 300 x 250 y 504 against
-    //    532 us, 256^3 z 127 against 155). 128-byte rows otherwise: 60 x 64 x
-    //    512 z 17.2 against 19.3 us with half the workgroups.
+    //    and there are enough of them (wide_many_groups): fewer row segments
+    //    and fewer misaligned edges per byte (FP64 777 x 300 x 250 y 504 against
+    //    532 us, 256^3 z 127 against 155). 128-byte rows otherwise.
     //  - FP64 at 16 rows per lane (512^3 z 0.94 against 0.95 ms at 32, 251 x
     //    300 x 300 y 213 against 222 us). FP32 at 32 rows per lane on 256-byte
     //    rows of 257-512 (512^3 y 0.466 against 0.484 ms for 16 on 128-byte
-    //    rows) and above 512, else at 16 on 128-byte rows (203 x 170 x 300 y 52
+    //    rows, given 1024 such workgroups: 200 x 300 x 150 y, 600, 56 against 48
+    //    us) and above 512, else at 16 on 128-byte rows (203 x 170 x 300 y 52
     //    against 55 us).
     //  - workgroups dealt to the XCDs in 8 ranges (G), so that neighbouring
     //    segments, which share lines where rows are misaligned, pass through
@@ -360,8 +361,8 @@ bool hybrid_default_cfg(const Geom &g, HybridCfg *cfg) {
     HybridCfg c;
     const bool fp64 = sizeof(REAL) == 8;
     const int64_t row_bytes = g.stride * (int64_t)sizeof(REAL);
-    const int64_t wide_groups = (g.n0 * (int64_t)sizeof(REAL) + 255) / 256 * g.n1;
-    const bool wide = g.N <= 512 && (fp64 ? wide_groups >= 512 : g.N > 256 && wide_groups >= 1024);
+    const bool wide = g.N <= 512 && (fp64 ? wide::wide_many_groups<REAL>(g)
+                                          : g.N > 256 && wide::wide_many_groups<REAL>(g, 1024));
     c.M = fp64 || (!wide && g.N <= 512) ? 16 : 32;
     c.W = (wide ? 256 : 128) / (int)sizeof(REAL);
     const int per_wave = std::max(1, 64 / c.W);

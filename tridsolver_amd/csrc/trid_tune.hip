@@ -542,6 +542,13 @@ tridStatus_t tune_adjoint(int dev, const Geom &g, bool grads, Choice *best) {
   static const int Ws[] = {1, 2, 4, 8, 16, 32, 64};
   static const int Gs[] = {1, 8, 16};
   std::vector<std::pair<float, HybridCfg>> timed;
+  auto try_cfg = [&](const HybridCfg &cfg) {
+    if (!adjoint_cfg_valid<REAL>(g, cfg)) return;
+    const float ms = time_on(st, [&] {
+      return launch_adjoint<REAL>(g, cfg, a, b, c, x, w, lam, ga, gb, gc, st);
+    });
+    if (std::isfinite(ms)) timed.emplace_back(ms, cfg);
+  };
   for (int M : Ms)
     for (int W : Ws)
       for (int G : Gs) {
@@ -553,12 +560,22 @@ tridStatus_t tune_adjoint(int dev, const Geom &g, bool grads, Choice *best) {
         if (g.stride != 1 && (int64_t)W * (int64_t)sizeof(REAL) < 64 && W < g.n0) continue;
         if ((int64_t)W > g.n0 && W > 1) continue;
         if ((int64_t)cfg.W * cfg.P < 32 && cfg.W < g.n0) continue;
-        if (!adjoint_cfg_valid<REAL>(g, cfg)) continue;
-        const float ms = time_on(st, [&] {
-          return launch_adjoint<REAL>(g, cfg, a, b, c, x, w, lam, ga, gb, gc, st);
-        });
-        if (std::isfinite(ms)) timed.emplace_back(ms, cfg);
+        try_cfg(cfg);
       }
+  if (g.stride != 1)  // the wide variant, whole waves of 128- or 256-byte rows
+    for (int M : {16, 32})
+      for (int seg : {128, 256})
+        for (int G : {1, 4, 8, 16, 32}) {
+          HybridCfg cfg;
+          cfg.M = M;
+          cfg.W = seg / (int)sizeof(REAL);
+          const int per_wave = std::max(1, 64 / cfg.W);
+          cfg.P = (int)((g.N + M - 1) / M);
+          cfg.P = (cfg.P + per_wave - 1) / per_wave * per_wave;
+          cfg.G = G;
+          cfg.V = 3;
+          if (wide_cfg_valid<REAL>(g, cfg)) try_cfg(cfg);
+        }
   std::sort(timed.begin(), timed.end(),
             [](const std::pair<float, HybridCfg> &p, const std::pair<float, HybridCfg> &q) {
               return p.first < q.first;
