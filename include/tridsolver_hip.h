@@ -118,6 +118,20 @@ EXTERN_C tridStatus_t tridHipAutotuneSave(const char *path);
 EXTERN_C tridStatus_t tridHipAutotuneLoad(const char *path);
 EXTERN_C tridStatus_t tridHipAutotuneClear(void);
 
+/* ---- solve into another array ---------------------------------------------
+ * No counterpart in the reference. tridXmtsvStridedBatch
+ * (scalar/include/tridsolver.h:38-48) with the solution written to x, an array of
+ * d's layout, and d left as it is: one pass over a, b, c, d and x where copying
+ * d first would be two. x may be d. */
+EXTERN_C tridStatus_t tridDmtsvStridedBatchTo(const TridParams *ctx, const double *a,
+                                              const double *b, const double *c, const double *d,
+                                              double *x, int ndim, int solvedim,
+                                              const int *dims, const int *pads);
+EXTERN_C tridStatus_t tridSmtsvStridedBatchTo(const TridParams *ctx, const float *a,
+                                              const float *b, const float *c, const float *d,
+                                              float *x, int ndim, int solvedim, const int *dims,
+                                              const int *pads);
+
 /* ---- FP32 sweeps with FP64 refinement ------------------------------------
  * No counterpart in the reference. Same arguments and layout as
  * tridDmtsvStridedBatch (scalar/include/tridsolver.h:38-42) plus the number

@@ -196,6 +196,50 @@ def test_forced_wide_variant(G, inc, seg, dtype):
     assert ran >= 8
 
 
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("dims,sd,force", [
+    ([64, 9, 5], 0, None), ([61, 9, 5], 0, None), ([5000, 3], 0, None), ([9000, 2], 0, None),
+    ([20000, 2], 0, None), ([40, 64, 3], 1, None), ([33, 5, 70], 2, None), ([9, 5000], 1, None),
+    ([40, 64, 3], 1, 1), ([40, 64, 3], 1, 2), ([40, 64, 3], 1, 0), ([40, 64, 3], 1, "lane")])
+def test_solve_to_equals_solve_in_place(dims, sd, force, dtype):
+    """The solution written to another array equals the solve in place bit for bit
+    (the same kernels and arithmetic) on every kernel family, inside a halo
+    whose cells neither form writes, and d is left as it is. force: a hybrid
+    variant at the rows per lane the streamed ones are built for, or the
+    per-lane kernel."""
+    import contextlib
+    if force in (0, 1, 2):
+        force = (8, 8, 16, 8, force) if dtype == torch.float64 else (16, 4, 16, 8, force)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    pads = [n + 2 for n in dims]
+    off = sum(int(np.prod(pads[:k])) for k in range(len(dims)))
+    a, b, c, d = (torch.rand(pads[::-1], dtype=dtype, device="cuda", generator=g) for _ in range(4))
+    b += 2
+    x = torch.full_like(d, 7.0)
+    ref, kept = d.clone(), d.clone()
+    args = dict(solvedim=sd, dims=dims, pads=pads, offset=off, sync=True)
+    if force == "lane":  # the algorithm a call's opts choose, as tridHipAutotuneLoad may record it
+        from tridsolver_amd import _lib
+        from tridsolver_amd._lib import int3
+        import ctypes as C
+        p = api.make_params((1, 1, 1), 1)
+        name = ("tridD" if dtype == torch.float64 else "tridS") + "mtsvStridedBatchTo"
+        api.use_torch_stream()
+        ptr = [C.c_void_p(t.data_ptr() + off * t.element_size()) for t in (a, b, c, d, x)]
+        assert getattr(_lib.lib(), name)(C.byref(p), *ptr, len(dims), sd, int3(dims),
+                                         int3(pads)) == 0
+        api.trid_strided_batch(a, b, c, ref, opts=(1, 1, 1), **args)
+    else:
+        with api.forced_hybrid(*force) if force else contextlib.nullcontext():
+            api.solve_to(a, b, c, d, x, **args)
+            api.trid_strided_batch(a, b, c, ref, **args)
+    inside = tuple(slice(1, 1 + n) for n in dims[::-1])
+    assert torch.equal(d, kept)
+    assert torch.equal(x[inside], ref[inside])
+    x[inside] = 7.0
+    assert bool((x == 7.0).all())
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("inc", [False, True])
 @pytest.mark.parametrize("dims,sd,seg", [

@@ -66,6 +66,8 @@ SIGNATURES = {
     "tridHipStreamCopy": ([P, P, SZ], I),
     "tridHipStreamCopyShape": ([P, P, SZ, I, I, I], I),
     "tridHipAccessProbe": ([P, P, P, P, I, P, I, I, I], I),
+    "tridDmtsvStridedBatchTo": ([P] * 6 + [I, I, P, P], I),
+    "tridSmtsvStridedBatchTo": ([P] * 6 + [I, I, P, P], I),
     "tridDmtsvStridedBatchMixed": ([P, P, P, P, P, I, I, P, P, I], I),
     "tridDmtsvStridedBatchMixedF32": ([P, P, P, P, P, P, I, I, P, P, I], I),
     "tridDmtsvStridedBatchAdjoint": ([P] * 10 + [I, I, P, P], I),

@@ -90,6 +90,22 @@ def trid_strided_batch(a, b, c, d, *, solvedim, dims=None, pads=None, u=None,
     return u if inc else d
 
 
+def solve_to(a, b, c, d, x, *, solvedim, dims=None, pads=None, offset=0, sync=False, stream=None):
+    """The solve along ``solvedim`` written to x, an array of d's layout; d is
+    left as it is (tridXmtsvStridedBatchTo). Returns x."""
+    dims = list(d.shape[::-1]) if dims is None else dims
+    pads = (list(d.shape[::-1]) if d.dim() == len(dims) else list(dims)) if pads is None else pads
+    arrs = [a, b, c, d, x]
+    _validate(arrs, dims, pads, offset)
+    use_torch_stream(stream)
+    name = ("tridD" if d.dtype == torch.float64 else "tridS") + "mtsvStridedBatchTo"
+    params = make_params((0, 0, 0), 1 if sync else 0)
+    st = getattr(_lib.lib(), name)(C.byref(params), *[_ptr(t, offset) for t in arrs], len(dims),
+                                   solvedim, int3(dims), int3(pads))
+    check(st, name)
+    return x
+
+
 def part_boundary(a, b, c, d, bnd, *, solvedim, shard, nshards, dims=None, pads=None,
                   offset=0, opts=(0, 0, 0), sync=False, stream=None):
     """Step 1 of a solve whose systems are split across shards

@@ -6,8 +6,9 @@ kernel (tridXmtsvStridedBatchAdjoint).
 
 a, b, c, d are dense tensors of one shape (x fastest = last torch dimension,
 so torch shape [nz, ny, nx] is the C API's dims [nx, ny, nz]); gradients are
-returned for every input that requires one. The forward leaves d untouched
-(it solves a copy); only the gradients the autograd graph needs are formed.
+returned for every input that requires one. The forward writes x to an array of
+its own and leaves d untouched; only the gradients the autograd graph needs are
+formed.
 """
 from __future__ import annotations
 
@@ -23,8 +24,7 @@ class TridSolve(torch.autograd.Function):
         a, b, c, d = tensors
         dims = list(d.shape[::-1])
         # torch dimension k is C dimension ndim-1-k
-        x = d.clone()
-        api.trid_strided_batch(a, b, c, x, solvedim=solvedim, dims=dims)
+        x = api.solve_to(a, b, c, d, torch.empty_like(d), solvedim=solvedim, dims=dims)
         ctx.solvedim = solvedim
         ctx.save_for_backward(a, b, c, x)
         return x

@@ -670,9 +670,8 @@ template <typename REAL, bool INC, int T, typename OnFetched>
 __device__ __forceinline__ void long32_solve(int64_t base, int N, unsigned char *smem_raw,
                                              const REAL *__restrict__ a,
                                              const REAL *__restrict__ b,
-                                             const REAL *__restrict__ c,
-                                             REAL *__restrict__ d, REAL *__restrict__ u,
-                                             OnFetched fetched) {
+                                             const REAL *__restrict__ c, const REAL *d,
+                                             REAL *u, OnFetched fetched) {
   constexpr int M = LONG32_M;
   static_assert(T % 64 == 0 && T <= LONG32_T_MAX, "whole waves, 32 T rows at most");
   const int t = threadIdx.x;
@@ -774,7 +773,7 @@ __device__ __forceinline__ void long32_solve(int64_t base, int N, unsigned char 
 #pragma unroll
   for (int r = 0; r < M; ++r) rd[r] = tile[fslot + (T + T / M) * r];
   __syncthreads();
-  REAL *dst = (INC ? u : d) + base;
+  REAL *dst = u + base;  // u == d for a solve in place
   // the store rows formed here from a thread index the compiler cannot
   // match with the loads' (an empty asm), so that the loads' row indices
   // are not held through the solve

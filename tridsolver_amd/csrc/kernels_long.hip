@@ -175,8 +175,7 @@ __global__ __launch_bounds__(256) void long_build_kernel(int64_t nsys, int64_t n
 template <typename REAL, bool CONTIG, bool INC>
 __global__ __launch_bounds__((LongShape<REAL, CONTIG>::T)) void long_subst_kernel(
     Geom g, int64_t nseg, const REAL *__restrict__ a, const REAL *__restrict__ b,
-    const REAL *__restrict__ c, REAL *__restrict__ d, REAL *__restrict__ u,
-    const REAL *__restrict__ y) {
+    const REAL *__restrict__ c, const REAL *d, REAL *u, const REAL *__restrict__ y) {
   using S = LongShape<REAL, CONTIG>;
   constexpr int M = LONG_M;
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -199,7 +198,7 @@ __global__ __launch_bounds__((LongShape<REAL, CONTIG>::T)) void long_subst_kerne
   hyb::substitute<REAL, M>(ra, rc, rd, yk, ym, x);
   hyb::to_fetch<M, CONTIG>(L, x, tile);
   if (INC) hyb::store_add<M, CONTIG>(L, u, x);
-  else hyb::store<M, CONTIG, true>(L, d, x);
+  else hyb::store<M, CONTIG, true>(L, u, x);  // u == d for a solve in place
 }
 
 template <typename REAL, bool CONTIG>
@@ -251,8 +250,8 @@ hipError_t launch_long_kernels(const Geom &g, int64_t nseg, const REAL *a, const
     static LdsGrant granted;
     hipError_t e = ensure_lds(reinterpret_cast<const void *>(kern), lds, granted);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(S::T), lds, st, g, nseg, a, b, c, d, u,
-                       y);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(S::T), lds, st, g, nseg, a, b, c, d,
+                       u ? u : d, y);
   }
   return hipGetLastError();
 }

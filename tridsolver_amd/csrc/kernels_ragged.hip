@@ -329,8 +329,8 @@ __global__ __launch_bounds__(RGL_T, 2) void rg_solve_split(
     };
     if (item < nlong)
       hyb::long32_solve<REAL, INC, RGL_T>(hyb::wave_uniform(cur.base),
-                                   __builtin_amdgcn_readfirstlane(cur.N), smem_raw, a, b, c, d, u,
-                                   fetched);
+                                   __builtin_amdgcn_readfirstlane(cur.N), smem_raw, a, b, c, d,
+                                   INC ? u : d, fetched);
     else rg_item<REAL, 16, INC, RGL_T>(cur, smem_raw, a, b, c, d, u, fetched);
     item = nxt;
     cur = next;

@@ -154,11 +154,12 @@ constexpr int hybrid_max_threads() {
   return HybridBounds<REAL, M>::threads;
 }
 
+// The solution goes to u: added to it (INC), or stored, with u == d for a solve
+// in place (every lane has loaded its rows before it stores any).
 template <typename REAL, int M, bool INC, bool CONTIG, bool VEC>
 __global__ __launch_bounds__((HybridBounds<REAL, M>::threads)) void hybrid_kernel(
     Geom g, int P, int W, int G, const REAL *__restrict__ a,
-    const REAL *__restrict__ b, const REAL *__restrict__ c, REAL *__restrict__ d,
-    REAL *__restrict__ u) {
+    const REAL *__restrict__ b, const REAL *__restrict__ c, const REAL *d, REAL *u) {
   constexpr int V = 16 / sizeof(REAL);
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const hyb::Lane L = hyb::lane_of<CONTIG>(g, P, W, G);
@@ -184,11 +185,11 @@ __global__ __launch_bounds__((HybridBounds<REAL, M>::threads)) void hybrid_kerne
   hyb::solve_chunk<REAL, M, CONTIG>(L, ring, ra, rb, rc, rd, x);
   if constexpr (VEC) {
     hyb::vto_fetch<M, V>(L, x, tile);
-    hyb::vstore<M, V, INC, true>(L, INC ? u : d, x);
+    hyb::vstore<M, V, INC, true>(L, u, x);
   } else {
     hyb::to_fetch<M, CONTIG>(L, x, tile);
     if (INC) hyb::store_add<M, CONTIG>(L, u, x);
-    else hyb::store<M, CONTIG, true>(L, d, x);
+    else hyb::store<M, CONTIG, true>(L, u, x);
   }
 }
 
@@ -208,7 +209,7 @@ hipError_t launch_hybrid_m(const Geom &g, const HybridCfg &cfg, const REAL *a,
   const int64_t nb0 = (g.n0 + cfg.W - 1) / cfg.W;
   const int64_t blocks = nb0 * g.n1;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(T), lds, st, g, cfg.P,
-                     cfg.W, cfg.G, a, b, c, d, u);
+                     cfg.W, cfg.G, a, b, c, d, u ? u : d);
   return hipGetLastError();
 }
 
@@ -221,7 +222,7 @@ hipError_t launch_hybrid_m(const Geom &g, const HybridCfg &cfg, const REAL *a,
 template <typename REAL, bool INC, int T>
 __global__ __launch_bounds__(T, 512 / T) void hybrid_long32_kernel(
     Geom g, int G, const REAL *__restrict__ a, const REAL *__restrict__ b,
-    const REAL *__restrict__ c, REAL *__restrict__ d, REAL *__restrict__ u) {
+    const REAL *__restrict__ c, const REAL *d, REAL *u) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const uint32_t n0 = (uint32_t)g.n0;
   const uint32_t sys = hyb::xcd_remap(blockIdx.x, gridDim.x, G);
@@ -239,7 +240,7 @@ hipError_t launch_long32_t(const Geom &g, const HybridCfg &cfg, const REAL *a, c
   hipError_t e = ensure_lds(reinterpret_cast<const void *>(kern), lds, lds_granted);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kern, dim3((unsigned)(g.n0 * g.n1)), dim3(T), lds, st, g, cfg.G, a, b, c,
-                     d, u);
+                     d, u ? u : d);
   return hipGetLastError();
 }
 
@@ -416,7 +417,7 @@ hipError_t launch_hybrid(const Geom &g, const HybridCfg &cfg, const REAL *a,
   auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   const bool vec = contig && cfg.M <= VEC_MAX_M && cfg.M % V == 0 && g.N % V == 0 &&
                    g.st0 % V == 0 && g.st1 % V == 0 && al16(a) && al16(b) && al16(c) &&
-                   al16(d) && (!INC || al16(u));
+                   al16(d) && (!u || al16(u));
 #define TRID_HYB_CASE(MM)                                                               \
   case MM:                                                                              \
     if (!contig) return launch_hybrid_m<REAL, MM, INC, false, false>(g, cfg, a, b, c, d, u, st); \

@@ -47,7 +47,7 @@ using namespace wide;
 template <typename REAL, int M, int SEG, bool INC, bool NT>
 __global__ __launch_bounds__((WideBounds<REAL, M>::threads)) void hybrid_wide_kernel(
     Geom g, int P, int G, int slots, const REAL *__restrict__ a, const REAL *__restrict__ b,
-    const REAL *__restrict__ c, REAL *__restrict__ d, REAL *__restrict__ u) {
+    const REAL *__restrict__ c, const REAL *d, REAL *u) {
   constexpr int W = WideShape<REAL, SEG>::W;
   constexpr int CH = 64 / W;  // chunks per wave
   constexpr int PITCH = wide_chunk_bytes(M, SEG);
@@ -96,7 +96,7 @@ __global__ __launch_bounds__((WideBounds<REAL, M>::threads)) void hybrid_wide_ke
   // across the whole kernel).
   uint32_t obs = ob;
   asm volatile("" : "+v"(obs));
-  char *dst = reinterpret_cast<char *>(INC ? u : d);
+  char *dst = reinterpret_cast<char *>(u);  // u == d for a solve in place
 #pragma unroll
   for (int r = 0; r < M; ++r) {
     if (r < rows) {
@@ -122,7 +122,7 @@ hipError_t launch_wide_nt(const Geom &g, const HybridCfg &cfg, const REAL *a, co
   }
   const int64_t blocks = (g.n0 + W - 1) / W * g.n1;
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(T), lds, st, g, cfg.P, cfg.G, slots, a,
-                     b, c, d, u);
+                     b, c, d, u ? u : d);
   return hipGetLastError();
 }
 
@@ -130,7 +130,7 @@ hipError_t launch_wide_nt(const Geom &g, const HybridCfg &cfg, const REAL *a, co
 template <typename REAL, int M, int SEG, bool INC>
 hipError_t launch_wide_m(const Geom &g, const HybridCfg &cfg, const REAL *a, const REAL *b,
                          const REAL *c, REAL *d, REAL *u, hipStream_t st) {
-  const uintptr_t low = (uintptr_t)b | (uintptr_t)c | (uintptr_t)d | (uintptr_t)(INC ? u : d);
+  const uintptr_t low = (uintptr_t)b | (uintptr_t)c | (uintptr_t)d | (uintptr_t)(u ? u : d);
   if (wide_rows_aligned<REAL>(g, low))
     return launch_wide_nt<REAL, M, SEG, INC, true>(g, cfg, a, b, c, d, u, st);
   return launch_wide_nt<REAL, M, SEG, INC, false>(g, cfg, a, b, c, d, u, st);

@@ -22,6 +22,7 @@
 
 #include "../../include/tridsolver.h"
 #include "../../include/tridsolver_hip.h"
+#include "hybrid_core.hpp"
 #include "trid_internal.h"
 #include "trid_tune.h"
 
@@ -161,6 +162,34 @@ void record_config(int algo, const HybridCfg *cfg) {
 
 const HybridCfg &forced_config() { return tl_forced; }
 
+namespace {
+
+// The batch's elements of src to dst, in the arrays' layout.
+template <typename REAL, bool CONTIG>
+__global__ __launch_bounds__(256) void copy_rows_kernel(Geom g, const REAL *__restrict__ src,
+                                                        REAL *__restrict__ dst) {
+  const int64_t total = g.nsys() * g.N;
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < total;
+       e += (int64_t)gridDim.x * 256) {
+    int64_t k;
+    const int64_t i = hyb::batch_elem<CONTIG>(g, e, &k);
+    dst[i] = src[i];
+  }
+}
+
+template <typename REAL>
+hipError_t launch_copy_rows(const Geom &g, const REAL *src, REAL *dst, hipStream_t st) {
+  if (g.stride == 1)
+    hipLaunchKernelGGL((copy_rows_kernel<REAL, true>), dim3(batch_elem_blocks(g)), dim3(256), 0,
+                       st, g, src, dst);
+  else
+    hipLaunchKernelGGL((copy_rows_kernel<REAL, false>), dim3(batch_elem_blocks(g)), dim3(256), 0,
+                       st, g, src, dst);
+  return hipGetLastError();
+}
+
+}  // namespace
+
 // Chooses and launches the kernel for one batched solve.
 template <typename REAL, bool INC>
 tridStatus_t solve(const TridParams *ctx, const REAL *a, const REAL *b, const REAL *c,
@@ -190,6 +219,16 @@ tridStatus_t solve(const TridParams *ctx, const REAL *a, const REAL *b, const RE
     const int algo = tuned_solve_algo<REAL, INC>(dev, g, &cfg);
     use_hybrid = algo == 3;
     use_long = algo == 12;
+  }
+
+  // Out of place, the kernels that only solve in place (per-lane Thomas, whose
+  // forward coefficients go through d, and the streamed variants) run in u
+  // on a copy of d.
+  if (!INC && u && (use_hybrid ? cfg.V == 1 || cfg.V == 2 : !use_long)) {
+    const hipError_t e = launch_copy_rows<REAL>(g, d, u, st);
+    if (e != hipSuccess) return finish(ctx, st, e);
+    d = u;
+    u = nullptr;
   }
 
   if (use_hybrid) {

@@ -171,6 +171,25 @@ tridStatus_t ragged_mixed32(const TridParams *ctx, const float *a, const float *
 
 using namespace trid;
 
+// d is read only where x is another array (solve() writes to x alone then).
+EXTERN_C tridStatus_t tridDmtsvStridedBatchTo(const TridParams *ctx, const double *a,
+                                              const double *b, const double *c, const double *d,
+                                              double *x, int ndim, int solvedim,
+                                              const int *dims, const int *pads) {
+  if (!x) return TRID_STATUS_INVALID_VALUE;
+  return solve<double, false>(ctx, a, b, c, const_cast<double *>(d), x == d ? nullptr : x, ndim,
+                              solvedim, dims, pads);
+}
+
+EXTERN_C tridStatus_t tridSmtsvStridedBatchTo(const TridParams *ctx, const float *a,
+                                              const float *b, const float *c, const float *d,
+                                              float *x, int ndim, int solvedim, const int *dims,
+                                              const int *pads) {
+  if (!x) return TRID_STATUS_INVALID_VALUE;
+  return solve<float, false>(ctx, a, b, c, const_cast<float *>(d), x == d ? nullptr : x, ndim,
+                             solvedim, dims, pads);
+}
+
 EXTERN_C tridStatus_t tridDmtsvStridedBatchMixed(const TridParams *ctx, const double *a,
                                                  const double *b, const double *c, double *d,
                                                  int ndim, int solvedim, const int *dims,

@@ -69,15 +69,19 @@ hipError_t launch_lane(const Geom &g, const REAL *a, const REAL *b, const REAL *
                        REAL *d, REAL *u, REAL *cws, REAL *dws, hipStream_t st);
 
 // Thomas-PCR hybrid; contiguous systems (stride == 1) use the LDS-staged
-// loader, strided systems load per lane with x-adjacent lanes.
+// loader, strided systems load per lane with x-adjacent lanes. u: the array the
+// solution is added to (INC); without INC the array it is written to, in d's
+// layout, or nullptr for d itself (the streamed variants, cfg.V 1 and 2, only
+// solve in place).
 template <typename REAL, bool INC>
 hipError_t launch_hybrid(const Geom &g, const HybridCfg &cfg, const REAL *a,
                          const REAL *b, const REAL *c, REAL *d, REAL *u,
                          hipStream_t st);
 
 // ---- shared host helpers (trid_api.hip) ---------------------------------
-// The batched solve behind tridXmtsvStridedBatch[Inc] (shape choice, launch,
-// ctx->sync).
+// The batched solve behind tridXmtsvStridedBatch[Inc] and its out-of-place form
+// (shape choice, launch, ctx->sync). Without INC, u is the array the solution is
+// written to (d is left as it is), or nullptr to solve in place.
 template <typename REAL, bool INC>
 tridStatus_t solve(const TridParams *ctx, const REAL *a, const REAL *b, const REAL *c,
                    REAL *d, REAL *u, int ndim, int solvedim, const int *dims,
@@ -97,7 +101,7 @@ void drop_stream_workspaces(int dev, hipStream_t st);
 
 // ---- systems longer than one workgroup holds (kernels_long.hip) -----------
 // The hybrid with its reduced system solved by a second batched solve;
-// workspace: long_workspace_bytes(g) bytes.
+// workspace: long_workspace_bytes(g) bytes. u as for launch_hybrid.
 template <typename REAL>
 size_t long_workspace_bytes(const Geom &g);
 template <typename REAL, bool INC>

@@ -91,8 +91,8 @@ __device__ __forceinline__ void wide_sweep(const REAL *a0, uint32_t tile, int wa
                                            int N, int64_t nsys, uint32_t os, uint32_t ob,
                                            int row0, int rows, REAL *as,
                                            const REAL *__restrict__ b,
-                                           const REAL *__restrict__ c,
-                                           const REAL *__restrict__ d, REAL (&rb)[M],
+                                           const REAL *__restrict__ c, const REAL *d,
+                                           REAL (&rb)[M],
                                            REAL (&rc)[M], REAL (&rd)[M], REAL &f_d, REAL &f_a,
                                            REAL &f_g) {
   constexpr int W = WideShape<REAL, SEG>::W;
