@@ -392,6 +392,17 @@ bool adjoint_default_cfg(const Geom &g, HybridCfg *cfg) {
     *cfg = c;
     return true;
   }
+  if (g.stride == 1 && sizeof(REAL) == 8 && g.N > 32 && g.N <= 256) {
+    // fewer rows per lane than the solve takes at these lengths: with nine
+    // streams the loads in flight matter more than the PCR (all gradients, 100
+    // / 200 rows: 125 / 85 against 137 / 89 us)
+    c.M = g.N <= 128 ? 2 : 4;
+    c.P = (int)((g.N + c.M - 1) / c.M);
+    c.W = std::max(1, 256 / c.P);
+    c.G = 1;
+    c.V = 0;
+    if (adjoint_cfg_valid<REAL>(g, c)) { *cfg = c; return true; }
+  }
   if (hybrid_plain_cfg<REAL>(g, &c)) {
     for (int k = 0; k < 4 && !adjoint_cfg_valid<REAL>(g, c); ++k) {
       if (g.stride == 1 && c.W > 1) c.W /= 2;

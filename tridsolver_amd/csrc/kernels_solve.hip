@@ -306,14 +306,32 @@ bool hybrid_plain_cfg(const Geom &g, HybridCfg *cfg) {
   const bool contig = g.stride == 1;
   static const int Ms[] = {1, 2, 4, 8, 16};
   if (contig) {
-    // One wave (or fewer lanes) per system when possible, 256-thread groups.
+    // Rows per lane: a lane more costs a PCR step's share (a division and two
+    // exchanges each), a row more a step of the serial sweep and registers.
+    // Measured with three sets of arrays used in turn, FP64 at 64 / 100 / 128 /
+    // 256 / 512 / 1000 / 2000 rows: 44.6 / 70 / 76 / 106 / 842 / 200 / 133 us at the
+    // rows below against 99 / 87 / 132 / 133 / 909 / 232 / 153 at the fewest rows
+    // that keep a system in one wave (1, 2, 2, 4, 8, 16, 16 with G = 8). FP32 stays
+    // at 4 rows (one vector) up to 256: 200 rows 49 against 54 us at 8.
+    // Workgroups of about 256 threads, except where the systems' lanes are no
+    // power of two and fill most of one wave: there one wave, whose PCR needs
+    // no barrier (100 / 400 rows: 70 / 81 against 76 / 85 us). Plain workgroup
+    // order: neighbouring systems share no lines, and all XCDs reading one
+    // region ran 4-8 % faster than eight regions at every length.
+    const int64_t n4 = sizeof(REAL) == 8 ? 112 : 256;
+    const int first = g.N <= 4 ? 1
+                      : sizeof(REAL) == 8 && g.N <= 32 ? 2
+                      : g.N <= n4 ? 4
+                      : g.N <= 2048 ? 8 : 16;
     for (int M : Ms) {
+      if (M < first) continue;
       const int64_t P = (g.N + M - 1) / M;
-      if (P > 64 && M < 16) continue;
       HybridCfg c;
       c.M = M;
       c.P = (int)P;
       c.W = (int)std::max<int64_t>(1, 256 / P);
+      if ((P & (P - 1)) != 0 && P <= 64 && 64 / P * P >= 48) c.W = (int)(64 / P);
+      c.G = 1;
       if (hybrid_cfg_valid<REAL>(g, c)) { *cfg = c; return true; }
     }
     return false;
