@@ -36,9 +36,10 @@ EXTERN_C tridStatus_t tridAdiStepS(const TridParams *ctx, float lambda, float *u
                                    float *a, float *b, float *c, int nx, int ny, int nz);
 
 /* `iters` timesteps (reference loop apps/adi/src/adi_cuda.cu:282-326). With
- * use_graph != 0 one step is captured into a hipGraph on a private stream and
- * replayed `iters` times on this thread's stream; the call then waits for the
- * replays before it returns (the executable graph is destroyed). */
+ * use_graph != 0, a step whose solves ctx->opts chooses is captured into a
+ * hipGraph on a private stream and replayed `iters` times on this thread's
+ * stream; matrix-free sweeps, which replays do not make faster, are launched.
+ * Either way the call waits for the steps before it returns. */
 EXTERN_C tridStatus_t tridAdiRunD(const TridParams *ctx, double lambda, double *u,
                                   double *du, double *a, double *b, double *c, int nx,
                                   int ny, int nz, int iters, int use_graph);

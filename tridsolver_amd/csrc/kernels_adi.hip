@@ -688,7 +688,7 @@ tridStatus_t run(const TridParams *ctx, REAL lambda, REAL *u, REAL *du, REAL *a,
                  REAL *c, int nx, int ny, int nz, int iters, int use_graph) {
   // a == NULL selects the matrix-free step. The array step's coefficient
   // arrays do not change from step to step: where its sweeps are matrix-free,
-  // they are written once before the steps. 256^3, per replayed step, against
+  // they are written once before the steps. 256^3, per step, against
   // preproc and the array solves in every step: FP64 0.178 against 0.605 ms,
   // FP32 0.104 against 0.276; a call of 20 FP64 steps 3.75 against 12.3 ms.
   if (iters < 0) return TRID_STATUS_INVALID_VALUE;
@@ -705,8 +705,17 @@ tridStatus_t run(const TridParams *ctx, REAL lambda, REAL *u, REAL *du, REAL *a,
     if (s != TRID_STATUS_SUCCESS) return s;
   }
   const bool sync = ctx == nullptr || ctx->sync != 0;
-  if (!use_graph || iters == 0) {
+  // use_graph: a step of array solves is captured once and replayed. The
+  // matrix-free sweeps are launched in either case: at three launches a step
+  // the replays are no faster (32^3 FP32, 200 steps: 4.54 ms with one step
+  // captured and replayed, 3.37 with graphs of 20 steps, 3.27 launched; 256^3
+  // FP64, 20 steps 3.66 against 3.47 ms), and capturing costs about 110 us a
+  // call. The call waits for the steps as it does for replays.
+  if (!use_graph || iters == 0 || !arrays) {
     for (int it = 0; it < iters && s == TRID_STATUS_SUCCESS; ++it) s = one_step();
+    if (use_graph && iters > 0 && hipStreamSynchronize(st) != hipSuccess &&
+        s == TRID_STATUS_SUCCESS)
+      s = TRID_STATUS_EXECUTION_FAILED;
   } else {
     // Capture one step on a private stream (the null stream cannot be
     // captured), replay it `iters` times on the caller's stream.
@@ -719,7 +728,7 @@ tridStatus_t run(const TridParams *ctx, REAL lambda, REAL *u, REAL *du, REAL *a,
     hipGraphExec_t exec = nullptr;
     void *prev = nullptr;
     tridHipGetStream(&prev);
-    if (arrays) {
+    {
       // Solves that take the per-lane path (ctx->opts 1 or 2, or systems
       // longer than one workgroup holds) need a workspace, which cannot be
       // allocated during capture: reserve it for the capture stream now.
