@@ -59,7 +59,8 @@ EXTERN_C size_t tridHipWorkspaceBytes(int fp64, int inc, int ndim, int solvedim,
  * for the hybrid its
  * rows per lane M, lanes per system P, systems per workgroup W and XCD
  * grouping G (consecutive system groups dealt to one XCD; 1 = plain order).
- * For the ragged solves: M, W = solve launches, G = workgroups per CU. */
+ * For the ragged solves: M, W = solve launches, G = workgroups per CU (0: one
+ * 256-thread workgroup per work item). */
 EXTERN_C tridStatus_t tridHipLastConfig(int *algorithm, int *M, int *P, int *W, int *G);
 
 /* Forces the hybrid shape for this thread's subsequent solves (M = 0 clears).
@@ -207,8 +208,8 @@ EXTERN_C tridStatus_t tridSmtsvStridedBatchAdjoint(const TridParams *ctx, const 
  * upper bound of every length, known to the caller (at most 8192); a longer
  * system found on the device is skipped and, for a synchronous call, reported
  * as TRID_STATUS_INVALID_VALUE (an asynchronous call cannot report it). Four
- * small planning kernels, then one persistent launch that takes every system
- * from a work queue (tridHipForceRaggedConfig can split it in two); capturable.
+ * small planning kernels, then one solve launch over every system
+ * (tridHipForceRaggedConfig can split it in two); capturable.
  * Needs tridHipRaggedWorkspaceBytes(nsys) of the stream's workspace (reserve
  * it before a hipGraph capture). */
 EXTERN_C tridStatus_t tridDmtsvRaggedBatch(const TridParams *ctx, const double *a,

@@ -741,6 +741,42 @@ def test_ragged_split_launch(per_cu, dtype):
                              sync=True)
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("said,longest,count", [(2048, 2048, 3000), (4096, 4096, 2000),
+                                                (2048, 1030, 17000), (2048, 8192, 400),
+                                                (4096, 8192, 400)])
+def test_ragged_default_shapes(said, longest, count, dtype):
+    """The untuned shapes, one workgroup per item: lengths at the edges of the
+    classes (8 and 16 rows per lane, up to 256 lanes), empty systems, more items
+    than the launch has workgroups (17,000 of 1025-1030 rows), and systems longer
+    than max_len says, which are solved up to 8192 rows; the arrays start at
+    different places inside a 128-byte line. Plain and Inc, against the oracle,
+    with the batch's tolerance."""
+    rng = np.random.default_rng(said + longest)
+    if count == 17000:
+        lens = rng.integers(1025, longest + 1, count)
+    else:
+        lens = np.round(np.exp(rng.uniform(0, np.log(longest), count))).astype(np.int64)
+        edges = [0, 1, 2, 8, 9, 16, 17, 511, 512, 513, 1023, 1024, 1025, longest - 1, longest, 0]
+        lens[:len(edges)] = edges
+    off, a, b, c, d = ragged_case(rng, lens, dtype)
+    u = rng.uniform(-1, 1, len(d)).astype(dtype)
+
+    def placed(v, k):
+        t = torch.zeros(len(v) + 32, dtype=dev(v).dtype, device="cuda")[k:k + len(v)]
+        return t.copy_(torch.from_numpy(v))
+
+    for inc in (False, True):
+        td = placed(d, 3)
+        tu = placed(u, 7) if inc else None
+        api.ragged_batch(placed(a, 0), placed(b, 1), placed(c, 5), td, dev(off), max_len=said,
+                         u=tu, sync=True)
+        got = (tu if inc else td).cpu().numpy()
+        if inc:
+            assert np.array_equal(td.cpu().numpy(), d)
+        check_ragged(off, a, b, c, d, got, dtype, u if inc else None)
+
+
 @pytest.mark.parametrize("launches", [0, 1, 2])
 @pytest.mark.parametrize("max_len", [2048, 8192])
 def test_ragged_mixed_f32_vs_oracle(max_len, launches):

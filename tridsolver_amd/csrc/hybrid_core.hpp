@@ -516,58 +516,53 @@ __device__ __forceinline__ void reduced_solve(const Lane &L, Ring &ring, TR al_e
   ym = ymv[0];
 }
 
-// Phases (i)-(iii) with the chunk's `a` kept in LDS: al_s[r * S] holds a of
-// the lane's row r (not read for the system's first row: first_chunk). The
-// forward sweep overwrites it with al, the backward sweep with ap; rc and rd
-// become gp and dp. y and ym as from reduced_solve. The arithmetic is
-// solve_chunk's; only where a lives differs. One row's LDS traffic at a time
-// (scheduling barriers), so the compiler does not hoist every LDS read.
-template <typename TR, int M, int S>
-__device__ __forceinline__ void sweep_lds_a(const Lane &L, Ring &ring, TR *al_s,
-                                            bool first_chunk, const TR (&rb)[M], TR (&rc)[M],
-                                            TR (&rd)[M], TR &y, TR &ym) {
-  // (i) forward sweep with left spike; al in the tile, ga in rc, de in rd
-  TR al_prev = 0;
+// Phases (i) and (ii) in one sweep. a_of(r) gives a of the chunk's row r (0 in
+// the system's first row). Row r becomes al_r x_{s-1} + x_r + ga_r x_{r+1} = de_r
+// with al in rb (a row's b is dead once its pivot is formed), ga in rc, de in rd;
+// the chunk's first unknown, x_s = f_d - f_a x_{s-1} - f_g x_{r+1} after row r,
+// is carried along, so that no backward sweep is needed for the reduced
+// system. substitute_back then solves the chunk from its end. One row at a time
+// (scheduling barriers), with the next row's a read ahead of it.
+template <typename TR, int M, typename A>
+__device__ __forceinline__ void sweep_carry(A a_of, TR (&rb)[M], TR (&rc)[M], TR (&rd)[M],
+                                            TR &f_d, TR &f_a, TR &f_g) {
+  f_d = 0; f_a = 0; f_g = -1;
+  TR ar = a_of(0), al = 0;
 #pragma unroll
   for (int r = 0; r < M; ++r) {
-    const TR ar = (r > 0 || !first_chunk) ? al_s[r * S] : TR(0);  // a[0] is not used
-    TR al;
+    TR anext = 0;
+    if (r + 1 < M) anext = a_of(r + 1);
     if (r == 0) {
       const TR inv = TR(1) / rb[0];
       al = ar * inv;
       rc[0] = rc[0] * inv;
       rd[0] = rd[0] * inv;
+      if (M >= 2) { f_d = rd[0]; f_a = al; f_g = rc[0]; }
     } else {
       const TR inv = TR(1) / (rb[r] - ar * rc[r - 1]);
-      al = -ar * al_prev * inv;
+      al = -ar * al * inv;
       rc[r] = rc[r] * inv;
       rd[r] = (rd[r] - ar * rd[r - 1]) * inv;
+      if (r < M - 1) {
+        f_d = f_d - f_g * rd[r];
+        f_a = f_a - f_g * al;
+        f_g = -f_g * rc[r];
+      }
     }
-    al_s[r * S] = al;
-    al_prev = al;
+    rb[r] = al;
+    ar = anext;
     __builtin_amdgcn_sched_barrier(0);
   }
-  const TR al_e = al_prev, ga_e = rc[M - 1], de_e = rd[M - 1];
-  // (ii) backward sweep; ap replaces al in the tile, gp and dp replace ga, de
-  TR ap_next = M >= 2 ? al_s[(M - 2) * S] : TR(0);
+}
+
+// (iv) after sweep_carry: x of the chunk's rows in rd, from y (x of its last row)
+// and ym (x of the previous chunk's).
+template <typename TR, int M>
+__device__ __forceinline__ void substitute_back(const TR (&rb)[M], const TR (&rc)[M],
+                                                TR (&rd)[M], TR y, TR ym) {
+  rd[M - 1] = y;
 #pragma unroll
-  for (int r = M - 3; r >= 0; --r) {
-    const TR gr = rc[r];
-    rd[r] = rd[r] - gr * rd[r + 1];
-    const TR ap = al_s[r * S] - gr * ap_next;
-    al_s[r * S] = ap;
-    ap_next = ap;
-    rc[r] = -gr * rc[r + 1];
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  TR f_d, f_a, f_g;
-  if (M >= 2) {
-    f_d = rd[0]; f_a = ap_next; f_g = rc[0];
-  } else {
-    f_d = TR(0); f_a = TR(0); f_g = TR(-1);
-  }
-  // (iii) reduced system across the P chunks
-  reduced_solve<TR>(L, ring, al_e, ga_e, de_e, f_d, f_a, f_g, y, ym);
+  for (int r = M - 2; r >= 0; --r) rd[r] = rd[r] - rb[r] * ym - rc[r] * rd[r + 1];
 }
 
 // (iv) x_r = dp_r - ap_r ym - gp_r y; x_{M-1} = y.
@@ -594,23 +589,170 @@ __device__ __forceinline__ void solve_chunk(const Lane &L, Ring &ring, TR (&ra)[
   substitute<TR, M>(ra, rc, rd, y, ym, x);
 }
 
+// v of lane 0, which the compiler then holds in scalar registers (a value
+// every lane of the wave has).
+__device__ __forceinline__ int64_t wave_uniform(int64_t v) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)v >> 32));
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+// ---- transposes inside one wave ----------------------------------------------
+// Where the system's lanes are P64 = min(P, 64) consecutive lanes of each wave (P
+// a power of two), a wave can load the rows its own lanes hold, P64 * M
+// consecutive ones per system, and transpose them in an LDS tile of its own
+// (64 * (M + 1) elements): LDS operations of a wave complete in order, so no
+// workgroup barrier is needed. lp: the lane's place among the P64; wt: the tile
+// of the lane's system. Fetch order: slot r holds row lp + P64 * r of the wave's
+// part. FULL: P64 = 64 (constant offsets from one address).
+__device__ __forceinline__ void wave_lds_order() { asm volatile("" : : : "memory"); }
+
+// Rows a lane fetches of its wave's M * P64: slot r holds row e + P64 * r, slot 0
+// row e0. Where a wave has one system (P64 = 64), e = lane - sh with sh the
+// system's first row past a 128-byte line, so that every slot but slot 0 reads
+// and writes whole lines of a system that starts anywhere; the sh lanes in front
+// take the wave's last sh rows in slot 0 instead. Ragged batches, whose systems start
+// anywhere (a misaligned wave access touches five lines for four in FP64, three for two
+// in FP32): 6000 systems of 2049-4096 rows, FP32, 79 us against 94, 40,000 of 8-8192
+// rows 252 against 291 (FP64: 443 against 456).
+struct Fetch {
+  int e, e0;
+};
+template <typename REAL, int M, bool FULL>
+__device__ __forceinline__ Fetch fetch_rows(const REAL *first, int lp) {
+  if (!FULL) return Fetch{lp, lp};
+  const int sh = (int)(((uintptr_t)first & 127) / sizeof(REAL));
+  const int e = lp - sh;
+  return Fetch{e, e < 0 ? e + 64 * M : e};
+}
+constexpr int ilog2(int v) { return v <= 1 ? 0 : 1 + ilog2(v / 2); }
+template <int M, bool FULL, typename TR>
+__device__ __forceinline__ TR *wave_slot(TR *wt, Fetch f, int P64, int r) {
+  static_assert(64 % M == 0, "rows per lane divide the wave");
+  const int e = r == 0 ? f.e0 : f.e;
+  // (M a power of two: the shift floors, for the negative e too)
+  return FULL ? wt + (e + (e >> ilog2(M))) + (64 + 64 / M) * r : wt + skew<M>(e + P64 * r);
+}
+template <int M, bool FULL, typename TR>
+__device__ __forceinline__ void wave_to_chunk(TR (&v)[M], TR *wt, int lp, Fetch f, int P64) {
+#pragma unroll
+  for (int r = 0; r < M; ++r) *wave_slot<M, FULL>(wt, f, P64, r) = v[r];
+  wave_lds_order();
+#pragma unroll
+  for (int r = 0; r < M; ++r) v[r] = wt[lp * (M + 1) + r];
+  wave_lds_order();
+}
+template <int M, bool FULL, typename TR>
+__device__ __forceinline__ void wave_to_fetch(TR (&v)[M], TR *wt, int lp, Fetch f, int P64) {
+#pragma unroll
+  for (int r = 0; r < M; ++r) wt[lp * (M + 1) + r] = v[r];
+  wave_lds_order();
+#pragma unroll
+  for (int r = 0; r < M; ++r) v[r] = *wave_slot<M, FULL>(wt, f, P64, r);
+  wave_lds_order();
+}
+
+// Barrier that orders LDS but leaves the wave's global loads in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("" : : : "memory");
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" : : : "memory");
+}
+
+// One workgroup's contiguous systems of P lanes each (P a power of two, M rows
+// per lane): loads, transposes inside the waves, solve, transposed store. L.base,
+// L.N and L.active are the lane's system; tile: 64 * (M + 1) elements per wave.
+// FULL: P >= 64, so that every lane of a wave has the same system (scalar base
+// address). Loads are unconditional, from rows clamped into the system; the
+// identity rows past N, and a of the first and c of the last row, are set once
+// the rows are in chunk order. issued() runs once the loads are issued,
+// loaded() once they have been transposed.
+template <typename REAL, int M, bool INC, bool FULL, typename OnIssued, typename OnLoaded>
+__device__ __forceinline__ void wave_solve(const Lane &L, REAL *tile, Ring &ring,
+                                           const REAL *__restrict__ a,
+                                           const REAL *__restrict__ b,
+                                           const REAL *__restrict__ c, const REAL *d, REAL *u,
+                                           OnIssued issued, OnLoaded loaded) {
+  const int P64 = FULL ? 64 : L.P, lane = L.t & 63;
+  const int lp = lane & (P64 - 1);
+  REAL *wt = tile + (L.t - lp) * (M + 1);  // the waves' tiles follow each other
+  const int w0 = (L.p - lp) * M;           // the wave's first row
+  const int N = (int)L.N;
+  const int64_t base = FULL ? wave_uniform(L.base) : L.base;
+  const Fetch f = fetch_rows<REAL, M, FULL>(d + base, lp);
+  REAL ra[M], rb[M], rc[M], rd[M];
+  if (L.active) {
+    const REAL *pa = a + base, *pb = b + base, *pc = c + base, *pd = d + base;
+    auto rows_of = [&](const REAL *p, REAL (&v)[M]) {
+#pragma unroll
+      for (int r = 0; r < M; ++r) {
+        const int row = w0 + (r == 0 ? f.e0 : f.e + P64 * r);
+        v[r] = ld<FULL>(p + (row < N ? row : N - 1));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    rows_of(pa, ra);
+    rows_of(pb, rb);
+    rows_of(pc, rc);
+    rows_of(pd, rd);
+  }
+  issued();
+  wave_to_chunk<M, FULL>(ra, wt, lp, f, P64);
+  wave_to_chunk<M, FULL>(rb, wt, lp, f, P64);
+  wave_to_chunk<M, FULL>(rc, wt, lp, f, P64);
+  wave_to_chunk<M, FULL>(rd, wt, lp, f, P64);
+  loaded();
+  const int row0 = L.p * M, rows = L.active ? N - row0 : 0;
+  if (row0 == 0) ra[0] = REAL(0);
+  if (rows <= M) {
+#pragma unroll
+    for (int r = 0; r < M; ++r) {
+      ra[r] = r < rows ? ra[r] : REAL(0);
+      rb[r] = r < rows ? rb[r] : REAL(1);
+      rc[r] = r + 1 < rows ? rc[r] : REAL(0);
+      rd[r] = r < rows ? rd[r] : REAL(0);
+    }
+  }
+  REAL f_d, f_a, f_g, y, ym;
+  sweep_carry<REAL, M>([&](int r) { return ra[r]; }, rb, rc, rd, f_d, f_a, f_g);
+  reduced_solve<REAL, true>(L, ring, rb[M - 1], rc[M - 1], rd[M - 1], f_d, f_a, f_g, y, ym);
+  substitute_back<REAL, M>(rb, rc, rd, y, ym);
+  // (the tile slots and rows from here on are formed again, not held through
+  // the solve: empty asm)
+  int lq = lp;
+  asm volatile("" : "+v"(lq));
+  const Fetch q = fetch_rows<REAL, M, FULL>(d + base, lq);
+  wave_to_fetch<M, FULL>(rd, tile + (L.t - lq) * (M + 1), lq, q, P64);
+  if (L.active) {
+    REAL *dst = u + base;  // u == d for a solve in place
+#pragma unroll
+    for (int r = 0; r < M; ++r) {
+      const int row = (L.p - lq) * M + (r == 0 ? q.e0 : q.e + P64 * r);
+      if (row < N) {
+        if (INC) dst[row] += rd[r];
+        else st<FULL>(&dst[row], rd[r]);
+      }
+    }
+  }
+}
+
 // ---- one long system in one workgroup, 32 rows per lane -----------------
 // 32 rows per lane, T lanes: systems of 4097-8192 rows in 256 threads, 8193-
-// 16384 in 512. b, c and d go to chunk order through the LDS tile; `a` then
-// goes from HBM into the same tile by global->LDS loads, in chunk order, and
-// stays there through the sweeps (sweep_lds_a), so the lane holds 32 rows of
-// b, c, d only (FP64: about 256 VGPRs, two waves per SIMD: two 256-thread
-// workgroups per CU or one of 512). The tile is skewed with one pad slot per
-// 32 rows (skew<32>, as the transposes use), so lane p reads its rows at
-// slots 33p + r. A global->LDS wave instruction writes 256 contiguous LDS
-// bytes (lane l: bytes 4l .. 4l+3 from its own source): FP64, rows 32k ..
-// 32k+31 to slots 33k ..; FP32, rows 64j .. 64j+63 by two instructions with
-// complementary lane masks, lanes 0-31 (chunk 2j) to slots 66j .. and lanes
-// 32-63 (chunk 2j+1) from base slot 66j + 1, which puts row 64j + l at slot
-// 66j + 1 + l = 33(2j+1) + (l - 32). base and N are the system's first
-// element and length (N <= 32 T), the same for every lane: callers pass them
-// through wave_uniform / readfirstlane, so they sit in scalar registers and
-// rows are 32-bit offsets from base. The arithmetic is solve_chunk's.
+// 16384 in 512. b, c and d go to chunk order through the LDS tile, wave by wave;
+// `a` then goes from HBM into the same tile by global->LDS loads, in chunk order,
+// and stays there for the sweep, so the lane holds 32 rows of b, c, d only (FP64:
+// about 256 VGPRs, two waves per SIMD: two 256-thread workgroups per CU or one
+// of 512). The tile is skewed with one pad slot per 32 rows (skew<32>, as the
+// transposes use), so lane p reads its rows at slots 33p + r. A global->LDS wave
+// instruction writes 256 contiguous LDS bytes (lane l: bytes 4l .. 4l+3 from
+// its own source): FP64, rows 32k .. 32k+31 to slots 33k ..; FP32, rows 64j ..
+// 64j+63 by two instructions with complementary lane masks, lanes 0-31 (chunk
+// 2j) to slots 66j .. and lanes 32-63 (chunk 2j+1) from base slot 66j + 1, which
+// puts row 64j + l at slot 66j + 1 + l = 33(2j+1) + (l - 32). base and N are the
+// system's first element and length (N <= 32 T), the same for every lane:
+// callers pass them through wave_uniform / readfirstlane, so they sit in
+// scalar registers and rows are 32-bit offsets from base.
 constexpr int LONG32_M = 32, LONG32_T = 256, LONG32_T_MAX = 512;
 
 // LDS of long32_solve at T lanes: the tile and the reduced solve's ring
@@ -622,14 +764,6 @@ constexpr size_t long32_lds_bytes() {
 static_assert(long32_lds_bytes<double, LONG32_T_MAX>() <= 160 * 1024, "LDS of one CU");
 
 typedef __attribute__((address_space(3))) void lds_void;
-
-// v of lane 0, which the compiler then holds in scalar registers (a value
-// every lane of the wave has).
-__device__ __forceinline__ int64_t wave_uniform(int64_t v) {
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)v >> 32));
-  return (int64_t)(((uint64_t)hi << 32) | lo);
-}
 
 // Byte address of an LDS object inside the workgroup's LDS.
 __device__ __forceinline__ uint32_t lds_address(const void *p) {
@@ -664,124 +798,102 @@ __device__ __forceinline__ void stage_wait_all() {
   asm volatile("" : : : "memory");
 }
 
-// `fetched()` runs once b is in chunk order (after a barrier that follows
-// the loads); a persistent caller decodes its next item there.
-template <typename REAL, bool INC, int T, typename OnFetched>
+// u is the array the solution is added to (INC) or stored in (u == d in place).
+// issued() runs once the loads of b, c and d are issued, loaded() once they are
+// in chunk order and a's are issued; a persistent caller decodes its next item
+// in the two.
+template <typename REAL, bool INC, int T, typename OnIssued, typename OnLoaded>
 __device__ __forceinline__ void long32_solve(int64_t base, int N, unsigned char *smem_raw,
                                              const REAL *__restrict__ a,
                                              const REAL *__restrict__ b,
                                              const REAL *__restrict__ c, const REAL *d,
-                                             REAL *u, OnFetched fetched) {
+                                             REAL *u, OnIssued issued, OnLoaded loaded) {
   constexpr int M = LONG32_M;
   static_assert(T % 64 == 0 && T <= LONG32_T_MAX, "whole waves, 32 T rows at most");
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, lane = t & 63;
   Lane L;
   L.P = T; L.W = 1; L.T = T; L.t = t; L.p = t; L.w = 0; L.pstep = 1; L.stride = 1;
   L.active = true; L.base = base; L.N = N; L.i0 = 0; L.i1 = 0;
   REAL *tile = reinterpret_cast<REAL *>(smem_raw);
   Ring ring{smem_raw + sizeof(REAL) * (size_t)T * (M + 1), (int)(3 * sizeof(REAL) * T), 0};
   const REAL *sb = b + base, *sc = c + base, *sd = d + base;
-  // b, c, d in fetch order (lane t: rows t + T*r), from rows clamped into
-  // the system so that every load is unconditional; the identity rows past N
-  // and c of row N-1 are set once the rows are in chunk order, where the
-  // lane's rows are row0 .. row0 + 31 (one row index, constant offsets,
-  // rather than 32 row indices held from the loads)
+  // b, c, d of the rows the wave's lanes hold, in fetch order (slot r: row wrow +
+  // 64 r), from rows clamped into the system so that every load is
+  // unconditional; the identity rows past N and c of row N-1 are set once the
+  // rows are in chunk order, where the lane's rows are row0 .. row0 + 31
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  const Fetch f = fetch_rows<REAL, M, true>(sd, lane);
   REAL rb[M], rc[M], rd[M];
 #pragma unroll
   for (int r = 0; r < M; ++r) {
-    const int row = t + T * r;
+    // nontemporal in FP64 (systems of 7777 rows: 5.8 TB/s against 5.6, of 16384 5.1
+    // against 4.9), plain in FP32 (5000 rows: 5.4 TB/s against 5.2)
+    const int row = wv * 64 * M + (r == 0 ? f.e0 : f.e + 64 * r);
     const int rr = row < N ? row : N - 1;
-    rb[r] = sb[rr];
-    rc[r] = sc[rr];
-    rd[r] = sd[rr];
+    rb[r] = ld<sizeof(REAL) == 8>(sb + rr);
+    rc[r] = ld<sizeof(REAL) == 8>(sc + rr);
+    rd[r] = ld<sizeof(REAL) == 8>(sd + rr);
   }
-  // transposes through the tile, hyb::to_chunk / to_fetch at P = T, M = 32:
-  // fetch-order row t + Tr sits at slot skew<32>(t + Tr) = (t + t/32) +
-  // (T + T/32)r, so each lane addresses all its slots from one base with
-  // constant offsets (no per-row address registers)
-  const int fslot = t + (t >> 5), cslot = t * (M + 1);
-  auto to_chunk = [&](REAL (&v)[M]) {
-#pragma unroll
-    for (int r = 0; r < M; ++r) tile[fslot + (T + T / M) * r] = v[r];
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < M; ++r) v[r] = tile[cslot + r];
-    __syncthreads();
-  };
-  to_chunk(rb);
-  fetched();
-  to_chunk(rc);
-  to_chunk(rd);  // ends with a barrier: the tile is free
+  issued();
+  REAL *wt = tile + (t - lane) * (M + 1);  // the wave's part of the tile
+  wave_to_chunk<M, true>(rb, wt, lane, f, 64);
+  wave_to_chunk<M, true>(rc, wt, lane, f, 64);
+  wave_to_chunk<M, true>(rd, wt, lane, f, 64);
   const int row0 = t * M;
+  {
+    // a of the wave's chunks into its part of the tile, which d's rows have left;
+    // lane l the dword l of each 256-byte window (row k*E + l*E/64, E rows a
+    // window). Row 0's a is not used and rows >= N are masked off. (The thread
+    // index passes through an empty asm: the loop's per-lane values are formed
+    // here for each item rather than hoisted out of the caller's item loop and
+    // held across it.)
+    constexpr int E = 256 / (int)sizeof(REAL);  // rows of a 256-byte window
+    int ll = lane;
+    asm volatile("" : "+v"(ll));
+    const int rl = ll * E / 64;
+    const REAL *sa = a + base;
+    const uint32_t lds = lds_address(tile);
+    for (int k = wv * (64 * M / E); k < (wv + 1) * (64 * M / E) && k * E < N; ++k) {
+      const int row = k * E + rl;
+      const bool ok = row >= 1 && row < N;
+      const uint32_t off = (uint32_t)(k * 256 + 4 * ll);
+      if constexpr (E == M) {  // FP64: the window is chunk k
+        if (ok) stage_dword(lds + k * (M + 1) * sizeof(REAL), sa, off);
+      } else {  // FP32: chunks 2k and 2k+1
+        if (ok && ll < 32) stage_dword(lds + 2 * k * (M + 1) * sizeof(REAL), sa, off);
+        if (ok && ll >= 32) stage_dword(lds + (2 * k * (M + 1) + 1) * sizeof(REAL), sa, off);
+      }
+    }
+  }
+  loaded();
+  REAL *as = tile + t * (M + 1);  // a of this lane's rows
   if (row0 + M >= N) {
 #pragma unroll
     for (int r = 0; r < M; ++r) {
       rb[r] = row0 + r < N ? rb[r] : REAL(1);
       rc[r] = row0 + r < N - 1 ? rc[r] : REAL(0);
       rd[r] = row0 + r < N ? rd[r] : REAL(0);
+      // a of the identity rows is 0: the lane clears its own slots, which no
+      // load writes
+      if (row0 + r >= N) as[r] = REAL(0);
     }
   }
-  {
-    // wave v moves the 256-byte windows k = v, v + T/64, ...; lane l the
-    // dword l of window k (row k*E + l*E/64, E rows a window). Row 0's a is
-    // not used and rows >= N are masked off. (The thread index passes
-    // through an empty asm: the loop's per-lane values are formed here for
-    // each item rather than hoisted out of the caller's item loop and held
-    // across it.)
-    constexpr int E = 256 / (int)sizeof(REAL);  // rows of a 256-byte window
-    int tt = t;
-    asm volatile("" : "+v"(tt));
-    const int lane = tt & 63;
-    const int rl = lane * E / 64;
-    const char *src = reinterpret_cast<const char *>(a + base) + 4 * lane;
-    for (int k = tt >> 6; k * E < N; k += T / 64) {
-      const int row = k * E + rl;
-      const bool ok = row >= 1 && row < N;
-      const char *s = src + k * 256;
-      if constexpr (E == M) {  // FP64: the window is chunk k
-        if (ok) __builtin_amdgcn_global_load_lds(s, (lds_void *)(tile + k * (M + 1)), 4, 0, 0);
-      } else {  // FP32: chunks 2k and 2k+1
-        if (ok && lane < 32)
-          __builtin_amdgcn_global_load_lds(s, (lds_void *)(tile + 2 * k * (M + 1)), 4, 0, 0);
-        if (ok && lane >= 32)
-          __builtin_amdgcn_global_load_lds(s, (lds_void *)(tile + 2 * k * (M + 1) + 1), 4, 0, 0);
-      }
-    }
-  }
-  REAL *al_s = tile + t * (M + 1);  // this lane's rows, chunk order
-  // a of the identity rows past N is 0: the lane clears its own slots, which
-  // no load writes
-  if (row0 + M > N) {
-#pragma unroll
-    for (int r = 0; r < M; ++r)
-      if (row0 + r >= N) al_s[r] = REAL(0);
-  }
-  // the tile is written by other waves' loads: wait for this wave's, then
-  // for every wave
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  REAL y, ym;
-  sweep_lds_a<REAL, M, 1>(L, ring, al_s, row0 == 0, rb, rc, rd, y, ym);
-  // (iv) substitution into rd; each lane reads only its own slots, which
-  // to_fetch then overwrites first
-#pragma unroll
-  for (int r = 0; r < M - 1; ++r) rd[r] = rd[r] - al_s[r] * ym - rc[r] * y;
-  rd[M - 1] = y;
-#pragma unroll
-  for (int r = 0; r < M; ++r) tile[cslot + r] = rd[r];
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < M; ++r) rd[r] = tile[fslot + (T + T / M) * r];
-  __syncthreads();
-  REAL *dst = u + base;  // u == d for a solve in place
-  // the store rows formed here from a thread index the compiler cannot
-  // match with the loads' (an empty asm), so that the loads' row indices
-  // are not held through the solve
-  int ts = t;
-  asm volatile("" : "+v"(ts));
+  stage_wait_all();
+  REAL f_d, f_a, f_g, y, ym;
+  sweep_carry<REAL, M>([&](int r) { return r == 0 && row0 == 0 ? REAL(0) : as[r]; }, rb, rc, rd,
+                       f_d, f_a, f_g);
+  reduced_solve<REAL>(L, ring, rb[M - 1], rc[M - 1], rd[M - 1], f_d, f_a, f_g, y, ym);
+  substitute_back<REAL, M>(rb, rc, rd, y, ym);
+  // the rows formed here again from a lane index the compiler cannot match with
+  // the loads' (an empty asm), so that they are not held through the solve
+  int ls = lane;
+  asm volatile("" : "+v"(ls));
+  const Fetch q = fetch_rows<REAL, M, true>(sd, ls);
+  wave_to_fetch<M, true>(rd, tile + (t - lane) * (M + 1), ls, q, 64);
+  REAL *dst = u + base;
 #pragma unroll
   for (int r = 0; r < M; ++r) {
-    const int row = ts + T * r;
+    const int row = wv * 64 * M + (r == 0 ? q.e0 : q.e + 64 * r);
     if (row < N) {
       // nontemporal stores at 256 lanes (8192 systems of 8192 rows: 0.50
       // against 0.53 ms), plain ones at 512 (16384 rows: 1.14 against 1.18)

@@ -175,9 +175,7 @@ __global__ __launch_bounds__((wide::WideBounds<REAL, M>::threads)) void adjoint_
     __syncthreads();
   }
   if (!L.active) return;
-  rd[M - 1] = y;
-#pragma unroll
-  for (int r = M - 2; r >= 0; --r) rd[r] = rd[r] - rb[r] * ym - rc[r] * rd[r + 1];
+  hyb::substitute_back<REAL, M>(rb, rc, rd, y, ym);
   auto put = [&](REAL *p, uint32_t off, REAL v) {
     hyb::st<NT>(reinterpret_cast<REAL *>(reinterpret_cast<char *>(p) + off), v);
   };

@@ -1,8 +1,7 @@
 // kernels_ragged.hip - ragged batch: S independent systems of uneven lengths
 // stored back to back (system s = rows offsets[s] .. offsets[s+1]-1 of a, b,
-// c, d), solved by persistent workgroups that take work items from a queue.
-// No counterpart in the reference, whose API needs equal lengths; per system
-// the result is the plain solve's.
+// c, d). No counterpart in the reference, whose API needs equal lengths; per
+// system the result is the plain solve's.
 //
 // Plan (four tiny kernels, all stream-ordered and capturable):
 //   reset     zero the class counters, the work counter and the error flag
@@ -11,15 +10,15 @@
 //   prefix    per class: first list slot and first work item; items are
 //             ordered longest class first (largest-first scheduling)
 //   scatter   list[slot] = s, slots reserved per workgroup and class
-// Solve: one persistent launch of T-thread workgroups, one per CU (times
-// `per_cu`), over every work item; or, split in two, systems needing more
-// than T/2 lanes by that launch and the rest by a second launch of two
-// T/2-thread workgroups per CU (one loads while the other computes). Each
-// workgroup repeatedly takes the next work item of its range from an atomic
-// counter -- W systems of one class, P lanes each, the Thomas-PCR hybrid of
-// hybrid_core.hpp -- and leaves when the counter passes the range's last
-// item, so every wave exits. Systems longer than M*T set the error flag and
-// are skipped.
+// Solve: an item is W systems of one class, P lanes each, the Thomas-PCR hybrid of
+// hybrid_core.hpp. By default each item is a 256-thread workgroup of its own
+// (rg_solve_each): the hardware keeps as many resident as registers and LDS
+// allow and starts the next as one ends. Forced or tuned shapes run it as a
+// resident grid of T-thread workgroups, `per_cu` per CU, that stride through the
+// items (rg_solve), in one launch or in two: systems needing more than T/2 lanes,
+// then the rest in T/2-thread workgroups. The mixed-precision solves take items
+// from an atomic counter. Systems longer than M*T set the error flag and are
+// skipped.
 
 #include <algorithm>
 #include <atomic>
@@ -92,13 +91,13 @@ __global__ __launch_bounds__(RG_PLAN_BLOCK) void rg_classify(const int64_t *__re
   if (t < RG_CLASSES && cnt[t] > 0) atomicAdd(&plan->counts[t], cnt[t]);
 }
 
-// Lanes of the workgroups that solve class c: Tmax for systems needing more
-// than Tshort lanes, Tshort for the rest.
-__host__ __device__ __forceinline__ int rg_threads(int c, int Tmax, int Tshort) {
-  return (1 << c) > Tshort ? Tmax : Tshort;
+// Systems of class c in a work item: one where they need more than Tshort
+// lanes, as many as fit Tshort lanes else.
+__host__ __device__ __forceinline__ int rg_systems(int c, int Tshort) {
+  return (1 << c) > Tshort ? 1 : Tshort >> c;
 }
 
-__global__ void rg_prefix(RaggedPlan *plan, int Tmax, int Tshort) {
+__global__ void rg_prefix(RaggedPlan *plan, int Tshort) {
   if (threadIdx.x != 0) return;
   int64_t sp = 0;
   for (int c = 0; c < RG_CLASSES; ++c) {
@@ -112,8 +111,8 @@ __global__ void rg_prefix(RaggedPlan *plan, int Tmax, int Tshort) {
   for (int k = 0; k < RG_CLASSES; ++k) {
     const int c = RG_CLASSES - 1 - k;
     plan->item_prefix[k] = ip;
-    const int W = rg_threads(c, Tmax, Tshort) >> c;
-    const int64_t items = W > 0 ? (plan->counts[c] + W - 1) / W : 0;
+    const int W = rg_systems(c, Tshort);
+    const int64_t items = (plan->counts[c] + W - 1) / W;
     ip += items;
     if ((1 << c) > Tshort) long_items += (int)items;
   }
@@ -169,9 +168,10 @@ __device__ __forceinline__ void rg_view_load(RgPlanView &v, const RaggedPlan *pl
   }
 }
 
-__device__ __forceinline__ RgMeta rg_meta(const RgPlanView &v, const int *__restrict__ list,
-                                          const int64_t *__restrict__ off, int item, int t,
-                                          int Tmax) {
+// Its first part: everything but the system's offset and length, with the list
+// entry (0 where the lane has no system).
+__device__ __forceinline__ RgMeta rg_entry(const RgPlanView &v, const int *__restrict__ list,
+                                           int item, int t, int Tmax, int *sys) {
   RgMeta m;
   // scheduling slot k: the last one whose first item is <= item (the
   // prefixes do not decrease, so that is the count of k >= 1 whose first
@@ -180,13 +180,30 @@ __device__ __forceinline__ RgMeta rg_meta(const RgPlanView &v, const int *__rest
 #pragma unroll
   for (int j = 1; j < RG_CLASSES; ++j) k += v.item_prefix[j] <= item ? 1 : 0;
   m.cls = RG_CLASSES - 1 - k;
-  const int P = 1 << m.cls, W = Tmax >> m.cls;
+  const int P = 1 << m.cls, W = max(1, Tmax >> m.cls);
   const int64_t first = v.sys_prefix[m.cls] + (int64_t)(item - v.item_prefix[k]) * W;
   const int64_t slot = first + t / P;
   m.active = slot < v.sys_prefix[m.cls + 1];
-  const int64_t sys = m.active ? list[slot] : 0;
-  m.base = m.active ? off[sys] : 0;
-  m.N = m.active ? (int)(off[sys + 1] - off[sys]) : 0;
+  *sys = m.active ? list[slot] : 0;
+  m.base = 0;
+  m.N = 0;
+  return m;
+}
+
+// The second part, from the list entry.
+__device__ __forceinline__ void rg_locate(RgMeta &m, const int64_t *__restrict__ off, int sys) {
+  if (m.active) {
+    m.base = off[sys];
+    m.N = (int)(off[sys + 1] - m.base);
+  }
+}
+
+__device__ __forceinline__ RgMeta rg_meta(const RgPlanView &v, const int *__restrict__ list,
+                                          const int64_t *__restrict__ off, int item, int t,
+                                          int Tmax) {
+  int sys;
+  RgMeta m = rg_entry(v, list, item, t, Tmax, &sys);
+  rg_locate(m, off, sys);
   return m;
 }
 
@@ -216,125 +233,212 @@ struct RgBounds {
   static constexpr int threads = M >= 16 ? 512 : 1024;
 };
 
-// One persistent launch over a range of items: LONG = the items whose systems
+// Threads of rg_solve_each's workgroups (per_cu 0).
+constexpr int RG_SMALL_T = 256;
+
+// One work item of rg_solve: W systems of one class, P lanes each, in T
+// threads (hyb::wave_solve). issued() runs once the loads are issued, loaded()
+// once they have arrived: the caller decodes its next item in the two.
+template <typename REAL, int M, bool INC, int T, typename OnIssued, typename OnLoaded>
+__device__ __forceinline__ void rg_item(const RgMeta &cur, unsigned char *smem_raw,
+                                        const REAL *__restrict__ a, const REAL *__restrict__ b,
+                                        const REAL *__restrict__ c, const REAL *d, REAL *u,
+                                        OnIssued issued, OnLoaded loaded) {
+  const int t = threadIdx.x;
+  const hyb::Lane L = rg_lane(cur, t, T);
+  REAL *tile = reinterpret_cast<REAL *>(smem_raw);
+  hyb::Ring ring{smem_raw + sizeof(REAL) * (size_t)T * (M + 1), (int)(3 * sizeof(REAL) * T), 0};
+  if (cur.cls >= 6)
+    hyb::wave_solve<REAL, M, INC, true>(L, tile, ring, a, b, c, d, u, issued, loaded);
+  else
+    hyb::wave_solve<REAL, M, INC, false>(L, tile, ring, a, b, c, d, u, issued, loaded);
+}
+
+// Waves per SIMD that the registers are held to: FP32 at 16 rows per lane needs
+// 134 without a bound, which would leave three waves.
+template <typename REAL, int M>
+constexpr int rg_waves() {
+  return sizeof(REAL) == 4 && M == 16 ? 4 : M == 16 ? 2 : 4;
+}
+
+// Workgroup k takes items k, k + grid, ... of its range, largest systems first.
+// `body(cur, issued, loaded)` solves one item; the next one's list entry is
+// loaded once the item's loads are issued, its offset and length once they have
+// arrived.
+template <typename Entry, typename Body>
+__device__ __forceinline__ void rg_items(int lo, int total, const int64_t *__restrict__ off,
+                                         Entry entry, Body body) {
+  int item = lo + (int)blockIdx.x, sys = 0;
+  if (item >= total) return;
+  RgMeta cur = entry(item, &sys);
+  rg_locate(cur, off, sys);
+  for (;;) {
+    const int nxt = item + (int)gridDim.x;
+    RgMeta next{};
+    body(
+        item, cur, [&] { if (nxt < total) next = entry(nxt, &sys); },
+        [&] { if (nxt < total) rg_locate(next, off, sys); });
+    if (nxt >= total) return;
+    item = nxt;
+    cur = next;
+    hyb::lds_barrier();  // the next item's LDS use starts after this one's
+  }
+}
+
+// A resident grid over a range of items: LONG = the items whose systems
 // need more than Tshort lanes (workgroups of T = Tmax threads, one per CU),
 // else the rest (T = Tshort, two workgroups per CU, so that one loads while
 // the other computes). A single launch plans with Tshort = Tmax: no item is
 // long, and the LONG = false launch at T = Tmax takes them all.
-// One work item of rg_solve: W systems of one class, P lanes each, in T
-// threads. `fetched()` runs once the loads are issued and a barrier has
-// passed (the caller decodes its next item there).
-template <typename REAL, int M, bool INC, int T, typename OnFetched>
-__device__ __forceinline__ void rg_item(const RgMeta &cur, unsigned char *smem_raw,
-                                        const REAL *__restrict__ a, const REAL *__restrict__ b,
-                                        const REAL *__restrict__ c, REAL *__restrict__ d,
-                                        REAL *__restrict__ u, OnFetched fetched) {
-  const int t = threadIdx.x;
-  const hyb::Lane L = rg_lane(cur, t, T);
-  REAL *tile = reinterpret_cast<REAL *>(smem_raw) + (size_t)L.w * L.P * (M + 1);
-  hyb::Ring ring{smem_raw + sizeof(REAL) * (size_t)T * (M + 1), (int)(3 * sizeof(REAL) * T), 0};
-  REAL ra[M], rb[M], rc[M], rd[M];
-  hyb::fetch_abcd<M, true>(L, a, b, c, d, ra, rb, rc, rd);
-  hyb::to_chunk<M, true>(L, ra, tile);  // has barriers
-  fetched();
-  hyb::to_chunk<M, true>(L, rb, tile);
-  hyb::to_chunk<M, true>(L, rc, tile);
-  hyb::to_chunk<M, true>(L, rd, tile);
-  REAL x[M];
-  hyb::solve_chunk<REAL, M, true>(L, ring, ra, rb, rc, rd, x);
-  hyb::to_fetch<M, true>(L, x, tile);
-  if (INC) hyb::store_add<M, true>(L, u, x);
-  else hyb::store<M, true>(L, d, x);
-}
-
 template <typename REAL, int M, bool INC, int T, bool LONG>
-__global__ __launch_bounds__(T) void rg_solve(
+__global__ __launch_bounds__(T, (rg_waves<REAL, M>())) void rg_solve(
     const REAL *__restrict__ a, const REAL *__restrict__ b, const REAL *__restrict__ c,
-    REAL *__restrict__ d, REAL *__restrict__ u, const int64_t *__restrict__ off,
-    const int *__restrict__ list, RaggedPlan *plan) {
-  constexpr int Tmax = T;
+    const REAL *d, REAL *u, const int64_t *__restrict__ off, const int *__restrict__ list,
+    const RaggedPlan *plan) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  __shared__ int s_next;
   __shared__ RgPlanView s_view;
-  rg_view_load(s_view, plan, threadIdx.x);
   const int t = threadIdx.x;
-  int *counter = LONG ? &plan->work : &plan->work_short;
   const int lo = LONG ? 0 : plan->long_items;
   const int total = LONG ? plan->long_items : plan->total_items;
-  if (t == 0) s_next = lo + atomicAdd(counter, 1);
+  if (lo + (int)blockIdx.x >= total) return;
+  rg_view_load(s_view, plan, t);
   __syncthreads();
-  int item = s_next;
-  RgMeta cur = item < total ? rg_meta(s_view, list, off, item, t, Tmax) : RgMeta{};
-  for (;;) {
-    __syncthreads();  // every thread has read s_next
-    if (item >= total) break;
-    // claim the following item now; its id is read after the next barrier
-    if (t == 0) s_next = lo + atomicAdd(counter, 1);
-    int nxt = total;
-    RgMeta next{};
-    rg_item<REAL, M, INC, Tmax>(cur, smem_raw, a, b, c, d, u, [&] {
-      nxt = s_next;
-      if (nxt < total) next = rg_meta(s_view, list, off, nxt, t, Tmax);
-    });
-    item = nxt;
-    cur = next;
-  }
+  rg_items(
+      lo, total, off,
+      [&](int item, int *sys) { return rg_entry(s_view, list, item, t, T, sys); },
+      [&](int, const RgMeta &cur, auto issued, auto loaded) {
+        rg_item<REAL, M, INC, T>(cur, smem_raw, a, b, c, d, u, issued, loaded);
+      });
 }
 
-// Systems needing more than 256 lanes at 16 rows per lane (4097-8192 rows):
-// hyb::long32_solve (32 rows per lane in 256 threads, `a` moved HBM->LDS in
-// chunk order). The items are single systems (plan class 9 at Tmax 512).
-constexpr int RGL_T = hyb::LONG32_T, RGL_PLAN_T = 512;
+// A system of more rows than RG_SMALL_T lanes of M hold, in one such workgroup:
+// what is left over where the shape was chosen for a max_len that the caller
+// understated. Each lane takes q blocks of RG_ROWS consecutive rows straight from
+// memory: one pass for the reduced system, keeping the sweep's state at each
+// block's start in the tile, and a second, block by block from the end, for x.
+// It reads everything twice and uncoalesced: 9765 systems of 4096 rows, FP64, 2.16 ms
+// where max_len says 2048, 0.29 where it says 4096.
+constexpr int RG_ROWS = 8;
+template <typename REAL, int M, bool INC>
+__device__ __forceinline__ void rg_item_rows(const RgMeta &cur, unsigned char *smem_raw,
+                                             const REAL *__restrict__ a,
+                                             const REAL *__restrict__ b,
+                                             const REAL *__restrict__ c, const REAL *d, REAL *u) {
+  constexpr int T = RG_SMALL_T, Q_MOST = RgBounds<REAL, M>::threads * M / (T * RG_ROWS);
+  static_assert(3 * (Q_MOST - 1) <= M + 1, "the states fit the lane's part of the tile");
+  const int t = threadIdx.x, N = __builtin_amdgcn_readfirstlane(cur.N);
+  const int q = (N + T * RG_ROWS - 1) / (T * RG_ROWS);
+  const int row0 = t * q * RG_ROWS;
+  const int64_t base = hyb::wave_uniform(cur.base);
+  const REAL *pa = a + base, *pb = b + base, *pc = c + base, *pd = d + base;
+  REAL *dst = u + base;  // u == d in place: a lane reads and writes rows of its own only
+  REAL *state = reinterpret_cast<REAL *>(smem_raw) + t * (M + 1);
+  hyb::Ring ring{smem_raw + sizeof(REAL) * (size_t)T * (M + 1), (int)(3 * sizeof(REAL) * T), 0};
+  hyb::Lane L{};
+  L.P = T; L.W = 1; L.T = T; L.t = t; L.p = t; L.pstep = 1; L.stride = 1;
+  L.active = true; L.base = base; L.N = N;
 
-// LDS of rg_solve_split: the long items' tile and ring (the rest need less).
-template <typename REAL>
-constexpr size_t rg_split_lds_bytes() {
-  return hyb::long32_lds_bytes<REAL>();
-}
-
-// The three-launch split's solve (plan at 16 rows per lane with Tmax 512 and
-// Tshort 256): one persistent launch of 256-thread workgroups over every
-// item (FP64: two per CU). The long items [0, long_items) come first in the
-// queue and take hyb::long32_solve at 32 rows per lane; the rest take rg_item at
-// 16 rows per lane. One launch, so a workgroup that runs out of long items
-// goes straight on to the short ones.
-template <typename REAL, bool INC>
-__global__ __launch_bounds__(RGL_T, 2) void rg_solve_split(
-    const REAL *__restrict__ a, const REAL *__restrict__ b, const REAL *__restrict__ c,
-    REAL *__restrict__ d, REAL *__restrict__ u, const int64_t *__restrict__ off,
-    const int *__restrict__ list, RaggedPlan *plan) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  __shared__ int s_next;
-  __shared__ RgPlanView s_view;
-  rg_view_load(s_view, plan, threadIdx.x);
-  const int t = threadIdx.x;
-  const int total = plan->total_items, nlong = plan->long_items;
-  auto decode = [&](int i) {
-    return i < nlong ? rg_meta(s_view, list, off, i, 0, RGL_PLAN_T)
-                     : rg_meta(s_view, list, off, i, t, RGL_T);
+  // one row of the sweep: al x_{s-1} + x_r + ga x_{r+1} = de
+  REAL al = -1, ga = 0, de = 0;
+  auto eliminate = [&](int row) {
+    const bool in = row < N;
+    const REAL ar = in && row > 0 ? pa[row] : REAL(0), br = in ? pb[row] : REAL(1);
+    const REAL cr = row < N - 1 ? pc[row] : REAL(0), dr = in ? pd[row] : REAL(0);
+    const REAL inv = REAL(1) / (br - ar * ga);
+    al = -ar * al * inv;
+    ga = cr * inv;
+    de = (dr - ar * de) * inv;
   };
-  if (t == 0) s_next = atomicAdd(&plan->work, 1);
-  __syncthreads();
-  int item = s_next;
-  RgMeta cur = item < total ? decode(item) : RgMeta{};
-  for (;;) {
-    __syncthreads();  // every thread has read s_next
-    if (item >= total) break;
-    if (t == 0) s_next = atomicAdd(&plan->work, 1);
-    int nxt = total;
-    RgMeta next{};
-    auto fetched = [&] {
-      nxt = s_next;
-      if (nxt < total) next = decode(nxt);
-    };
-    if (item < nlong)
-      hyb::long32_solve<REAL, INC, RGL_T>(hyb::wave_uniform(cur.base),
-                                   __builtin_amdgcn_readfirstlane(cur.N), smem_raw, a, b, c, d,
-                                   INC ? u : d, fetched);
-    else rg_item<REAL, 16, INC, RGL_T>(cur, smem_raw, a, b, c, d, u, fetched);
-    item = nxt;
-    cur = next;
+  REAL f_d = 0, f_a = 0, f_g = -1, y, ym;
+  for (int j = 0; j < q; ++j) {
+    if (j > 0) {
+      state[3 * j - 3] = al; state[3 * j - 2] = ga; state[3 * j - 1] = de;
+    }
+#pragma unroll
+    for (int r = 0; r < RG_ROWS; ++r) {
+      eliminate(row0 + RG_ROWS * j + r);
+      if (j < q - 1 || r < RG_ROWS - 1) {
+        f_d = f_d - f_g * de;
+        f_a = f_a - f_g * al;
+        f_g = -f_g * ga;
+      }
+    }
   }
+  hyb::reduced_solve<REAL, true>(L, ring, al, ga, de, f_d, f_a, f_g, y, ym);
+  REAL x = y;
+  for (int j = q - 1; j >= 0; --j) {
+    al = -1; ga = 0; de = 0;
+    if (j > 0) {
+      al = state[3 * j - 3]; ga = state[3 * j - 2]; de = state[3 * j - 1];
+    }
+    REAL ral[RG_ROWS], rga[RG_ROWS], rde[RG_ROWS];
+#pragma unroll
+    for (int r = 0; r < RG_ROWS; ++r) {
+      eliminate(row0 + RG_ROWS * j + r);
+      ral[r] = al; rga[r] = ga; rde[r] = de;
+    }
+#pragma unroll
+    for (int r = RG_ROWS - 1; r >= 0; --r) {
+      if (j < q - 1 || r < RG_ROWS - 1) x = rde[r] - ral[r] * ym - rga[r] * x;
+      rde[r] = x;
+    }
+#pragma unroll
+    for (int r = 0; r < RG_ROWS; ++r) {
+      const int row = row0 + RG_ROWS * j + r;
+      if (row < N) {
+        if (INC) dst[row] += rde[r];
+        else dst[row] = rde[r];
+      }
+    }
+  }
+}
+
+// One launch of RG_SMALL_T-thread workgroups over every item, one each, planned with
+// Tshort = RG_SMALL_T. The items [0, long_items), single systems that need more
+// lanes, come first: LONG32 (M = 16: 4097-8192 rows) takes them by
+// hyb::long32_solve, 32 rows per lane in 256 threads with `a` moved HBM->LDS in
+// chunk order; otherwise there are none but misdeclared ones (rg_item_rows). Bound by
+// HBM: with the plan's four launches (19 us), FP64, 40 M unknowns in systems of
+// 4096 rows 291 us, of 2048 (M = 8) 286; lengths of 2049-4096 at random 153 us for
+// 17.7 M unknowns, of 4097-8192 206 us for 23.6 M. What is left over the floor is
+// the last class's idle lanes (a system fills its power of two of lanes to 3/4
+// on average) and the plan. One 512- or 1024-thread workgroup per CU that took items
+// from an atomic counter: 412 and 406 us for the first two.
+template <typename REAL, int M, bool LONG32>
+constexpr size_t rg_each_lds_bytes() {
+  return LONG32 ? hyb::long32_lds_bytes<REAL>()
+                : sizeof(REAL) * (size_t)RG_SMALL_T * (M + 1) + hyb::ring_bytes<REAL>(RG_SMALL_T, 3);
+}
+
+template <typename REAL, int M, bool INC, bool LONG32>
+__global__ __launch_bounds__(RG_SMALL_T, (LONG32 ? 2 : rg_waves<REAL, M>())) void rg_solve_each(
+    const REAL *__restrict__ a, const REAL *__restrict__ b, const REAL *__restrict__ c,
+    const REAL *d, REAL *u, const int64_t *__restrict__ off, const int *__restrict__ list,
+    const RaggedPlan *plan) {
+  static_assert(!LONG32 || (M == 16 && hyb::LONG32_T == RG_SMALL_T), "long32_solve's shape");
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ RgPlanView s_view;
+  const int t = threadIdx.x;
+  const int nlong = plan->long_items, total = plan->total_items;
+  if ((int)blockIdx.x >= total) return;
+  rg_view_load(s_view, plan, t);
+  __syncthreads();
+  rg_items(
+      0, total, off,
+      [&](int i, int *sys) { return rg_entry(s_view, list, i, t, RG_SMALL_T, sys); },
+      [&](int i, const RgMeta &cur, auto issued, auto loaded) {
+        if (i >= nlong) {
+          rg_item<REAL, M, INC, RG_SMALL_T>(cur, smem_raw, a, b, c, d, u, issued, loaded);
+        } else if constexpr (LONG32) {
+          hyb::long32_solve<REAL, INC, RG_SMALL_T>(hyb::wave_uniform(cur.base),
+                                                   __builtin_amdgcn_readfirstlane(cur.N),
+                                                   smem_raw, a, b, c, d, u, issued, loaded);
+        } else {
+          issued();
+          loaded();
+          rg_item_rows<REAL, M, INC>(cur, smem_raw, a, b, c, d, u);
+        }
+      });
 }
 
 // The four planning launches: work items of at most Tmax lanes.
@@ -348,11 +452,48 @@ void launch_plan(const int64_t *off, int64_t S, int M, int Tmax, int Tshort, voi
     hipLaunchKernelGGL(rg_classify, dim3(nb), dim3(RG_PLAN_BLOCK), 0, st, off, S, M, Tmax,
                        plan);
   }
-  hipLaunchKernelGGL(rg_prefix, dim3(1), dim3(64), 0, st, plan, Tmax, Tshort);
+  hipLaunchKernelGGL(rg_prefix, dim3(1), dim3(64), 0, st, plan, Tshort);
   if (nb > 0) {
     hipLaunchKernelGGL(rg_scatter, dim3(nb), dim3(RG_PLAN_BLOCK), 0, st, off, S, M, Tmax,
                        plan, list);
   }
+}
+
+// Workgroups of a launch that gives every item one of its own: there are at most
+// S items, known only on the device, and workgroups past the last leave at once.
+// Above this many, workgroups take several.
+constexpr int64_t RG_GRID_MOST = 16384;
+
+template <typename REAL, int M, bool INC, bool LONG32>
+hipError_t launch_each(const REAL *a, const REAL *b, const REAL *c, REAL *d, REAL *u,
+                       const int64_t *off, int64_t S, void *ws, hipStream_t st) {
+  RaggedPlan *plan = static_cast<RaggedPlan *>(ws);
+  int *list = reinterpret_cast<int *>(static_cast<unsigned char *>(ws) + RAGGED_PLAN_HEADER_BYTES);
+  launch_plan(off, S, M, RgBounds<REAL, M>::threads, RG_SMALL_T, ws, st);
+  auto kern = rg_solve_each<REAL, M, INC, LONG32>;
+  static LdsGrant lds_granted;
+  constexpr size_t lds = rg_each_lds_bytes<REAL, M, LONG32>();
+  hipError_t e = ensure_lds(reinterpret_cast<const void *>(kern), lds, lds_granted);
+  if (e != hipSuccess) return e;
+  const unsigned blocks = (unsigned)std::min<int64_t>(std::max<int64_t>(S, 1), RG_GRID_MOST);
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(RG_SMALL_T), lds, st, a, b, c, d, INC ? u : d, off,
+                     list, plan);
+  return hipGetLastError();
+}
+
+// One rg_solve launch of `blocks` T-thread workgroups.
+template <typename REAL, int M, bool INC, int T, bool LONG>
+hipError_t launch_range(const REAL *a, const REAL *b, const REAL *c, REAL *d, REAL *u,
+                        const int64_t *off, const int *list, const RaggedPlan *plan,
+                        unsigned blocks, hipStream_t st) {
+  const size_t lds = sizeof(REAL) * (size_t)T * (M + 1) + hyb::ring_bytes<REAL>(T, 3);
+  auto kern = rg_solve<REAL, M, INC, T, LONG>;
+  static LdsGrant lds_granted;
+  hipError_t e = ensure_lds(reinterpret_cast<const void *>(kern), lds, lds_granted);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(T), lds, st, a, b, c, d, INC ? u : d, off, list,
+                     plan);
+  return hipGetLastError();
 }
 
 template <typename REAL, int M, bool INC>
@@ -363,56 +504,25 @@ hipError_t launch_m(const REAL *a, const REAL *b, const REAL *c, REAL *d, REAL *
   constexpr int Tshort = Tmax / 2;
   RaggedPlan *plan = static_cast<RaggedPlan *>(ws);
   int *list = reinterpret_cast<int *>(static_cast<unsigned char *>(ws) + RAGGED_PLAN_HEADER_BYTES);
+  if (launches == 3 && M != 16) return hipErrorInvalidValue;
+  if constexpr (M == 16) {  // the long systems at 32 rows per lane
+    if (launches == 3) return launch_each<REAL, M, INC, true>(a, b, c, d, u, off, S, ws, st);
+  }
+  if (per_cu == 0) return launch_each<REAL, M, INC, false>(a, b, c, d, u, off, S, ws, st);
   int cus = 256;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  const int per = std::max(1, per_cu);
+  const unsigned wgs = (unsigned)(cus * std::max(1, per_cu));
   if (launches == 1) {  // every item in one launch of Tmax-thread workgroups
     launch_plan(off, S, M, Tmax, Tmax, ws, st);
-    const size_t lds = sizeof(REAL) * (size_t)Tmax * (M + 1) + hyb::ring_bytes<REAL>(Tmax, 3);
-    auto kern = rg_solve<REAL, M, INC, Tmax, false>;
-    static LdsGrant lds_granted;
-    hipError_t e = ensure_lds(reinterpret_cast<const void *>(kern), lds, lds_granted);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(cus * per)), dim3(Tmax), lds, st, a, b, c, d, u,
-                       off, list, plan);
-    return hipGetLastError();
+    return launch_range<REAL, M, INC, Tmax, false>(a, b, c, d, u, off, list, plan, wgs, st);
   }
-  if (launches == 3 && M != 16) return hipErrorInvalidValue;
   launch_plan(off, S, M, Tmax, Tshort, ws, st);
-  if constexpr (M == 16) {
-    if (launches == 3) {  // one launch: the long systems at 32 rows per lane, then the rest
-      auto kern = rg_solve_split<REAL, INC>;
-      static LdsGrant lds_granted;
-      constexpr size_t lds = rg_split_lds_bytes<REAL>();
-      hipError_t e = ensure_lds(reinterpret_cast<const void *>(kern), lds, lds_granted);
-      if (e != hipSuccess) return e;
-      int per_sm = 0;  // resident workgroups per CU
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_sm, reinterpret_cast<const void *>(kern),
-                                                       RGL_T, lds) != hipSuccess || per_sm < 1)
-        per_sm = 1;
-      hipLaunchKernelGGL(kern, dim3((unsigned)(per_sm * cus * per)), dim3(RGL_T), lds, st, a, b,
-                         c, d, u, off, list, plan);
-      return hipGetLastError();
-    }
-  }
   if (launches == 2) {  // the long systems first (an empty range exits at once)
-    const size_t lds = sizeof(REAL) * (size_t)Tmax * (M + 1) + hyb::ring_bytes<REAL>(Tmax, 3);
-    auto kern = rg_solve<REAL, M, INC, Tmax, true>;
-    static LdsGrant lds_granted;
-    hipError_t e = ensure_lds(reinterpret_cast<const void *>(kern), lds, lds_granted);
+    const hipError_t e =
+        launch_range<REAL, M, INC, Tmax, true>(a, b, c, d, u, off, list, plan, wgs, st);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(cus * per)), dim3(Tmax), lds, st, a, b, c, d, u,
-                       off, list, plan);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  const size_t lds = sizeof(REAL) * (size_t)Tshort * (M + 1) + hyb::ring_bytes<REAL>(Tshort, 3);
-  auto kern = rg_solve<REAL, M, INC, Tshort, false>;
-  static LdsGrant lds_granted;
-  hipError_t e = ensure_lds(reinterpret_cast<const void *>(kern), lds, lds_granted);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(2 * cus * per)), dim3(Tshort), lds, st, a, b, c, d,
-                     u, off, list, plan);
-  return hipGetLastError();
+  return launch_range<REAL, M, INC, Tshort, false>(a, b, c, d, u, off, list, plan, 2 * wgs, st);
 }
 
 // FP64 systems by FP32 sweeps plus FP64 refinement (mixed_core.hpp): the
@@ -727,6 +837,8 @@ hipError_t launch_ragged_mixed(int M, const double *a, const double *b, const do
 size_t ragged_workspace_bytes(int64_t S) {
   return RAGGED_PLAN_HEADER_BYTES + sizeof(int) * (size_t)std::max<int64_t>(S, 1);
 }
+
+
 
 int ragged_max_len(int fp64, int M) {
   (void)fp64;  // the same shapes at both precisions

@@ -228,7 +228,7 @@ __global__ __launch_bounds__(T, 512 / T) void hybrid_long32_kernel(
   const uint32_t sys = hyb::xcd_remap(blockIdx.x, gridDim.x, G);
   const int64_t base = (int64_t)(sys % n0) * g.st0 + (int64_t)(sys / n0) * g.st1;
   hyb::long32_solve<REAL, INC, T>(hyb::wave_uniform(base), (int)g.N, smem_raw, a, b, c, d, u,
-                                  [] {});
+                                  [] {}, [] {});
 }
 
 template <typename REAL, bool INC, int T>

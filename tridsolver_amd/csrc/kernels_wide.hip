@@ -88,9 +88,7 @@ __global__ __launch_bounds__((WideBounds<REAL, M>::threads)) void hybrid_wide_ke
   if (!L.active) return;
   // (iv)
   if (INC) hyb::stage_wait_all();
-  rd[M - 1] = y;
-#pragma unroll
-  for (int r = M - 2; r >= 0; --r) rd[r] = rd[r] - rb[r] * ym - rc[r] * rd[r + 1];
+  hyb::substitute_back<REAL, M>(rb, rc, rd, y, ym);
   // The store offsets are recomputed here (the empty asm hides that they
   // equal the load offsets, which would otherwise be kept live in registers
   // across the whole kernel).

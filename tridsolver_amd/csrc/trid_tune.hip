@@ -624,15 +624,17 @@ void ragged_tuned_config(int dev, int64_t max_len, int *M, int *per_cu, int *lau
     *launches = (c.cfg.V >= 1 && c.cfg.V <= 3) ? c.cfg.V : 1;
     return;
   }
-  // untuned: where systems may exceed 4096 rows, 16 rows per lane -- FP64
-  // in the split launch (systems over 4096 rows at 32 rows per lane), FP32
-  // in one launch of two 512-thread workgroups per CU (the tuned choices on
-  // the 40,000-system batch of lengths up to 8192: FP64 0.45 ms against
-  // 0.53 in one launch; FP32 0.27 against 0.30 split and 0.35 at one
-  // workgroup per CU); else 8 rows per lane in one launch
-  *M = max_len > 4096 ? 16 : 8;
-  *per_cu = (max_len > 4096 && sizeof(REAL) == 4) ? 2 : 1;
-  *launches = (max_len > 4096 && sizeof(REAL) == 8) ? 3 : 1;
+  // untuned: one 256-thread workgroup per item, at as few rows per lane as hold
+  // max_len -- 8 up to 2048 rows, 16 up to 4096, else 16 with the systems over
+  // 4096 rows at 32. Plan included, against one 512- or 1024-thread workgroup per CU
+  // taking items from a queue: 40,000 systems of 8-2000 rows, FP64, 141 us against 211,
+  // 6000 of 30-1500, FP32, 23.5 against 34.6; 40,000 of 8-4000, FP64, 256 against 325;
+  // 40,000 of 8-8192, FP64, 443 against 456, FP32 252 against 268.
+  // 16 rows per lane where 8 hold the systems: 10,000 of 1025-2048, FP64, 131 us
+  // against 122.
+  *M = max_len > 2048 ? 16 : 8;
+  *per_cu = 0;
+  *launches = max_len > 4096 ? 3 : 1;
 }
 
 // Tunes the ragged kernel on the caller's offsets with scratch values.
@@ -668,7 +670,7 @@ tridStatus_t tune_ragged(int dev, const int64_t *offsets, int64_t nsys, int64_t 
   struct Cand { int M, per_cu, launches; };
   std::vector<Cand> cands;
   for (int M : {4, 8, 16})
-    for (int per_cu : {1, 2}) cands.push_back({M, per_cu, 1});
+    for (int per_cu : {0, 1, 2}) cands.push_back({M, per_cu, 1});
   if (max_len > 4096) cands.push_back({16, 1, 3});
   for (const Cand &cd : cands) {
     if (ragged_max_len(sizeof(REAL) == 8, cd.M) < max_len) continue;

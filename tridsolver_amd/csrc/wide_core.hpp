@@ -119,37 +119,10 @@ __device__ __forceinline__ void wide_sweep(const REAL *a0, uint32_t tile, int wa
   }
   if constexpr (WHOLE) hyb::stage_done(rb[0]);
   else hyb::stage_wait_all();
-  // one row at a time (scheduling barriers), the next row's a read from LDS
-  // ahead of it
-  f_d = 0; f_a = 0; f_g = -1;
-  REAL ar = as[0], al = 0;
-  if (row0 == 0) ar = REAL(0);  // a of the system's first row is not used
-#pragma unroll
-  for (int r = 0; r < M; ++r) {
-    REAL anext = 0;
-    if (r + 1 < M) anext = as[(r + 1) * W];
-    if (r == 0) {
-      const REAL inv = REAL(1) / rb[0];
-      al = ar * inv;
-      rc[0] = rc[0] * inv;
-      rd[0] = rd[0] * inv;
-      if (M >= 2) { f_d = rd[0]; f_a = al; f_g = rc[0]; }
-    } else {
-      const REAL inv = REAL(1) / (rb[r] - ar * rc[r - 1]);
-      al = -ar * al * inv;
-      // c of the system's last row is not used
-      rc[r] = (WHOLE && r == M - 1 && rows == M) ? REAL(0) : rc[r] * inv;
-      rd[r] = (rd[r] - ar * rd[r - 1]) * inv;
-      if (r < M - 1) {
-        f_d = f_d - f_g * rd[r];
-        f_a = f_a - f_g * al;
-        f_g = -f_g * rc[r];
-      }
-    }
-    rb[r] = al;
-    ar = anext;
-    __builtin_amdgcn_sched_barrier(0);
-  }
+  // (a of the system's first row is not used, nor c of its last)
+  hyb::sweep_carry<REAL, M>(
+      [&](int r) { return r == 0 && row0 == 0 ? REAL(0) : as[r * W]; }, rb, rc, rd, f_d, f_a, f_g);
+  if (WHOLE && rows == M) rc[M - 1] = REAL(0);
 }
 
 // Whether a workgroup of the shape holds the system: whole waves of W
