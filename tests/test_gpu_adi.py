@@ -277,3 +277,31 @@ def test_cli_dump_matches_oracle(tmp_path, fused, prec):
     r = adi_io.compare(ref, path, nx, ny, nz, prec)
     assert r["nan_points"] == 0
     assert r["normwise_rel"] <= (1e-12 if prec == 64 else 1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("shape", [(4, 3, 3), (8, 1, 5), (12, 2, 2), (64, 5, 9), (200, 9, 7),
+                                   (256, 7, 5), (260, 5, 6), (512, 4, 4), (516, 3, 3),
+                                   (1024, 3, 4), (1028, 3, 3), (30, 20, 18), (16, 192, 193),
+                                   (16, 193, 257), (16, 1030, 4), (8, 4, 1025), (8, 2000, 3)])
+def test_sweeps_with_several_lines_per_lane(dtype, shape):
+    """Matrix-free steps at the edges of the sweeps that take one 16-byte vector
+    of lines (y, z) or 2-4 lines (x) per lane: rows per lane, lanes per wave and
+    workgroup, lines that end a group, and lengths they leave to the general
+    sweeps; and the same steps on arrays one element off 16-byte alignment, which
+    the general sweeps take. Both against the oracle, normwise 1e-12 / 1e-5."""
+    nx, ny, nz = shape
+    n = nx * ny * nz
+    u_cpu = np.random.default_rng(n).uniform(-1, 1, n).astype(
+        np.float64 if dtype == torch.float64 else np.float32)
+    tol = 1e-12 if dtype == torch.float64 else 1e-5
+    got = []
+    for shift in (0, 1):
+        u, du = (torch.zeros(n + 4, dtype=dtype, device="cuda")[shift:shift + n]
+                 for _ in range(2))
+        u.copy_(torch.from_numpy(u_cpu))
+        adi.run_fused(0.7, u, du, 3, shape, graph=False, sync=True)
+        got.append(_np(u))
+    oracle.adi(0.7, u_cpu, nx, ny, nz, 3)
+    for g in got:
+        H.assert_norm_close(g, u_cpu, tol=tol)

@@ -122,7 +122,7 @@ tridStatus_t preproc(REAL lambda, const REAL *u, REAL *du, REAL *ax, REAL *bx, R
 // computes them from (i, j, k) with the same expressions in the same
 // precision, and reads only du (and u for the z sweep): 16 B per point
 // per sweep instead of 40 (FP64). The solve is the Thomas-PCR hybrid of
-// hybrid_core.hpp, so results equal the array-based step bit for bit.
+// hybrid_core.hpp.
 // ---------------------------------------------------------------------------
 template <typename REAL>
 struct AdiCoef {
@@ -253,100 +253,302 @@ __global__ __launch_bounds__((AdiBounds<REAL, M>::threads)) void adi_solve_kerne
   }
 }
 
-// The matrix-free x sweep with every access in chunk order (x lines of
-// N = P * 8 rows, P lanes of 8 rows, one wave per workgroup): lane p loads
-// its own rows 8p .. 8p+7 of u and of the four neighbour lines as 16-byte
-// vectors, takes the x neighbours of its first and last row from lanes p-1
-// and p+1 by ds_bpermute, solves (the PCR exchanges are wave-local too) and
-// stores its rows as vectors. No LDS tile and no transpose: the values and
-// the arithmetic are those of adi_solve_kernel's x sweep, so the results are
-// the same bit for bit. For x lines whose rows start 16-byte aligned
-// (nx * sizeof(REAL) a multiple of 16) on grids below 4 GiB, at FP32: 8 FP32
-// rows are two 16-byte vectors per lane. Measured on the 256^3 matrix-free
-// step (replay time per step): FP32 0.105 ms against 0.117-0.12 with the
-// LDS-tiled sweep; FP64, four vectors per lane (64-byte strides between
-// lanes), 0.197 ms against 0.178, so FP64 keeps the tiled sweep.
-constexpr int ADI_DX_M = 8;
+// ---- sweeps along y and z, several lines per lane ----------------------------
+// Every line away from the grid's boundary has the same coefficients, and the lines
+// on it have a right-hand side of zeros (the x sweep leaves du = 0 there), which any
+// coefficients solve to zeros. So a lane takes V neighbouring lines, one 16-byte
+// vector per row, and forms the pivots, the forward factors and the reduced
+// system's coefficients once for all of them: per point, the right-hand side's
+// four multiply-adds and 1/V of the rest (one division per row). Against a line per
+// lane (adi_solve_kernel, which was bound by that arithmetic): 200 x 168 x 147, FP32,
+// whose arrays the last-level cache holds, y 14.4 to 10.6 us, z 21.5 to 12.1; FP64
+// 20.5 to 15.8 and 29.8 to 21.4; 256^3 FP32 28.6 to 22.4 and 57.6 to 32.8, FP64 43.4 to
+// 40.3 and 65.9 to 62.1 (402 MB in the z sweep: 6.5 TB/s).
+// Lines along y: V x-neighbours of one k. Along z: the plane's lines in memory
+// order, n0 = nx * ny (the launch folds them).
+constexpr int ADI_VEC_T = 512;  // most threads of a workgroup
 
-template <typename REAL>
-__global__ __launch_bounds__(64) void adi_x_direct_kernel(Geom g, int P, int W, int G,
-                                                          AdiCoef<REAL> kc,
-                                                          REAL *__restrict__ d,
-                                                          const REAL *__restrict__ u) {
-  constexpr int M = ADI_DX_M;
-  constexpr int V = 16 / (int)sizeof(REAL);  // elements per 16-byte vector
-  typedef REAL vec __attribute__((ext_vector_type(V)));
-  __shared__ __align__(16) unsigned char ring_lds[2 * 3 * sizeof(REAL) * 64];
-  const hyb::Lane L = hyb::lane_of<true>(g, P, W, G);
-  hyb::Ring ring{ring_lds, (int)(3 * sizeof(REAL) * 64), 0};
-  const int j = (int)L.i0, k = (int)L.i1;  // the x line (j, k)
-  const bool line_inner = L.active && j > 0 && j < kc.ny - 1 && k > 0 && k < kc.nz - 1;
-  const uint32_t sy = line_inner ? (uint32_t)(kc.nx * sizeof(REAL)) : 0u;
-  const uint32_t sz = line_inner ? (uint32_t)((uint32_t)kc.nx * kc.ny * sizeof(REAL)) : 0u;
-  // lanes past the last line read line 0; their rows are identity rows
-  const uint32_t o0 = ((L.active ? (uint32_t)L.base : 0u) + (uint32_t)(L.p * M)) *
-                      (uint32_t)sizeof(REAL);
-  const char *ub = reinterpret_cast<const char *>(u);
-  auto ldv = [ub](uint32_t off) { return *reinterpret_cast<const vec *>(ub + off); };
-  REAL uc[M], ym[M], yp[M], zm[M], zp[M];
+// The solve of one chunk of V lines: x[e][r] the right-hand sides in, the solution
+// out. middle() runs once the forward sweep is done. WAVE: the lines lie in one wave
+// (no ring).
+template <typename REAL, int M, int V, bool WAVE, typename Middle>
+__device__ __forceinline__ void adi_lines(const hyb::Lane &L, hyb::Ring &ring, REAL lambda, int n,
+                                          int row0, REAL (&x)[V][M], Middle middle) {
+  // factors: al_r x_{s-1} + x_r + ga_r x_{r+1} = de_r, the chunk's first unknown
+  // x_s = f_d - f_a x_{s-1} - f_g x_{r+1} after row r (as hyb::sweep_carry)
+  const REAL ca = REAL(-0.5) * lambda, cb = REAL(1) + lambda;
+  REAL al[M], ga[M], s[2 + V], m[2 + V], q[2 + V];
+  s[0] = 0;
+  s[1] = -1;
 #pragma unroll
-  for (int q = 0; q < M / V; ++q) {
-    const uint32_t o = o0 + (uint32_t)(q * 16);
-    const vec c0 = ldv(o), c1 = ldv(o - sy), c2 = ldv(o + sy), c3 = ldv(o - sz), c4 = ldv(o + sz);
-#pragma unroll
-    for (int e = 0; e < V; ++e) {
-      uc[q * V + e] = c0[e];
-      ym[q * V + e] = c1[e];
-      yp[q * V + e] = c2[e];
-      zm[q * V + e] = c3[e];
-      zp[q * V + e] = c4[e];
-    }
-  }
-  // x neighbours: rows 8p-1 and 8p+8 live in lanes p-1 and p+1
-  REAL edge[2] = {uc[M - 1], uc[0]}, nb_lo[2], nb_hi[2];
-  hyb::exchange<3, 2>(L, ring, true, edge, L.pstep, L.p > 0, nb_lo, L.pstep, L.p + 1 < L.P,
-                      nb_hi);
-  REAL rd[M];
+  for (int e = 0; e < V; ++e) s[2 + e] = 0;
 #pragma unroll
   for (int r = 0; r < M; ++r) {
-    const int row = L.p * M + r;
-    const bool inner = line_inner && row > 0 && row < L.N - 1;
-    const REAL xm = r > 0 ? uc[r - 1] : nb_lo[0];
-    const REAL xp = r < M - 1 ? uc[r + 1] : nb_hi[1];
-    rd[r] = inner ? adi_rhs(kc.lambda, xm, xp, ym[r], yp[r], zm[r], zp[r], uc[r]) : REAL(0);
-  }
-  REAL ra[M], rb[M], rc[M];
-  adi_coefs<REAL, M, true>(L, kc, ra, rb, rc);
-  REAL x[M];
-  hyb::solve_chunk<REAL, M, true>(L, ring, ra, rb, rc, rd, x);
-  if (!L.active) return;
-  char *db = reinterpret_cast<char *>(d);
+    const int row = row0 + r;
+    const bool inner = row > 0 && row < n - 1;
+    const REAL a = inner ? ca : REAL(0), b = inner ? cb : REAL(1);
+    const REAL inv = REAL(1) / (r > 0 ? b - a * ga[r - 1] : b);
+    al[r] = r > 0 ? -a * al[r - 1] * inv : a * inv;
+    ga[r] = a * inv;
 #pragma unroll
-  for (int q = 0; q < M / V; ++q) {
+    for (int e = 0; e < V; ++e) {
+      const REAL v = row < n ? x[e][r] : REAL(0);
+      x[e][r] = (r > 0 ? v - a * x[e][r - 1] : v) * inv;
+      if (r < M - 1) s[2 + e] = s[2 + e] - s[1] * x[e][r];
+    }
+    if (r < M - 1) {
+      s[0] = s[0] - s[1] * al[r];
+      s[1] = -s[1] * ga[r];
+    }
+  }
+  middle();
+  // reduced system, as hyb::reduced_solve with V right-hand sides
+  hyb::from_above<2 + V>(L, ring, WAVE, s, q);
+  {
+    const REAL inv = REAL(1) / (REAL(1) - ga[M - 1] * q[0]);
+    s[0] = al[M - 1] * inv;
+    s[1] = -ga[M - 1] * q[1] * inv;
+#pragma unroll
+    for (int e = 0; e < V; ++e) s[2 + e] = (x[e][M - 1] - ga[M - 1] * q[2 + e]) * inv;
+  }
+  for (int h = 1; h < L.P; h <<= 1) {
+    hyb::from_both<2 + V>(L, ring, WAVE, h, s, m, q);
+    const REAL A = s[0], C = s[1];
+    const REAL inv = REAL(1) / (REAL(1) - A * m[1] - C * q[0]);
+    s[0] = -inv * A * m[0];
+    s[1] = -inv * C * q[1];
+#pragma unroll
+    for (int e = 0; e < V; ++e) s[2 + e] = inv * (s[2 + e] - A * m[2 + e] - C * q[2 + e]);
+  }
+  REAL y[V], ym[V];
+#pragma unroll
+  for (int e = 0; e < V; ++e) y[e] = s[2 + e];
+  hyb::from_below<V>(L, ring, WAVE, y, ym);
+#pragma unroll
+  for (int e = 0; e < V; ++e) x[e][M - 1] = y[e];
+#pragma unroll
+  for (int r = M - 2; r >= 0; --r) {
+#pragma unroll
+    for (int e = 0; e < V; ++e) x[e][r] = x[e][r] - al[r] * ym[e] - ga[r] * x[e][r + 1];
+  }
+}
+
+template <typename REAL, int M, bool INC>
+__global__ __launch_bounds__(ADI_VEC_T) void adi_vec_kernel(Geom g, int P, int W, int G,
+                                                            REAL lambda, REAL *__restrict__ d,
+                                                            REAL *__restrict__ u) {
+  constexpr int V = 16 / (int)sizeof(REAL);
+  typedef REAL vec __attribute__((ext_vector_type(V)));
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  hyb::Lane L{};
+  L.P = P; L.W = W; L.T = P * W;
+  L.t = threadIdx.x;
+  L.p = L.t / W;
+  L.w = L.t - L.p * W;
+  L.pstep = W;
+  hyb::Ring ring{smem_raw, (int)((2 + V) * sizeof(REAL) * L.T), 0};
+  const uint32_t groups = (uint32_t)((g.n0 + W * V - 1) / (W * V));
+  const uint32_t id = hyb::xcd_remap(blockIdx.x, gridDim.x, G);
+  const uint32_t k = id / groups, i0 = ((id - k * groups) * W + L.w) * V;
+  const int n = (int)g.N, row0 = L.p * M;
+  const bool active = i0 < (uint32_t)g.n0;
+  // 32-bit byte offsets (the launch checks the extent); rows past N and lines past
+  // n0 are read from inside the array and not stored
+  const uint32_t stride = (uint32_t)g.stride * (uint32_t)sizeof(REAL);
+  const uint32_t o = ((active ? i0 : 0u) + k * (uint32_t)g.st1) * (uint32_t)sizeof(REAL);
+  auto at = [&](REAL *base, int r) {
+    const int row = row0 + r;
+    return reinterpret_cast<vec *>(reinterpret_cast<char *>(base) + o +
+                                   (uint32_t)(row < n ? row : n - 1) * stride);
+  };
+  REAL x[V][M];
+#pragma unroll
+  for (int r = 0; r < M; ++r) {
+    const vec v = *at(d, r);
+#pragma unroll
+    for (int e = 0; e < V; ++e) x[e][r] = v[e];
+  }
+
+  // u's rows arrive during the reduced solve
+  vec uv[INC ? M : 1];
+  adi_lines<REAL, M, V, false>(L, ring, lambda, n, row0, x, [&] {
+    if (INC) {
+#pragma unroll
+      for (int r = 0; r < M; ++r) uv[r] = *at(u, r);
+    }
+  });
+  if (!active) return;
+#pragma unroll
+  for (int r = 0; r < M; ++r) {
+    if (row0 + r >= n) break;
     vec v;
 #pragma unroll
-    for (int e = 0; e < V; ++e) v[e] = x[q * V + e];
-    *reinterpret_cast<vec *>(db + o0 + (uint32_t)(q * 16)) = v;
+    for (int e = 0; e < V; ++e) v[e] = x[e][r];
+    if (INC) *at(u, r) = uv[r] + v;
+    else *at(d, r) = v;
   }
 }
 
-// The direct x sweep applies: 8 rows per lane filling the lines exactly, a
-// whole line's lanes in the wave, 16-byte aligned rows and arrays.
+// Shape of adi_vec_kernel for the sweep along sd = 1 or 2, or false where it does
+// not apply: lines in whole vectors, 16-byte aligned, arrays below 4 GiB, a line
+// within a workgroup. Eight lanes' vectors a row are a 128-byte line (four: 200 x 168 x
+// 147 FP64 66 against 68 us a step, 300^3 412 against 389; sixteen 409). 16 rows per lane
+// for the longer lines (300^3 FP64 389 against 418 us; 256^3 FP64 166 against 170, FP32
+// 82 against 81; 200 x 168 x 147 FP32 39 against 37).
 template <typename REAL>
-bool adi_x_direct_ok(const Geom &g, const HybridCfg &cfg, const REAL *d, const REAL *u,
-                     int nx) {
-  auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-  return sizeof(REAL) == 4 && cfg.M == ADI_DX_M && (int64_t)cfg.P * ADI_DX_M == g.N &&
-         cfg.W * cfg.P <= 64 && ((int64_t)nx * (int64_t)sizeof(REAL)) % 16 == 0 && al16(d) &&
-         al16(u);
+bool adi_vec_cfg(const REAL *d, const REAL *u, int nx, int ny, int nz, int sd, Geom *g,
+                 HybridCfg *cfg) {
+  constexpr int V = 16 / (int)sizeof(REAL);
+  const int64_t plane = (int64_t)nx * ny, points = plane * nz;
+  if (sd == 1) *g = Geom{ny, nx, nx, nz, 1, plane};
+  else *g = Geom{nz, plane, plane, 1, 1, 0};
+  if (g->n0 % V != 0 || points * (int64_t)sizeof(REAL) > (int64_t)0xffffffff) return false;
+  if (((reinterpret_cast<uintptr_t>(d) | reinterpret_cast<uintptr_t>(u)) & 15) != 0) return false;
+  cfg->M = g->N > (sizeof(REAL) == 8 ? 192 : 256) ? 16 : 8;
+  cfg->P = (int)std::min<int64_t>((g->N + cfg->M - 1) / cfg->M, ADI_VEC_T);
+  cfg->W = 8 * cfg->P <= ADI_VEC_T ? 8 : 4;
+  cfg->G = 8;
+  cfg->V = 0;
+  return cfg->W * cfg->P <= ADI_VEC_T && (int64_t)cfg->P * cfg->M >= g->N;
 }
 
+template <typename REAL, int M, bool INC>
+hipError_t launch_adi_vec(const Geom &g, const HybridCfg &cfg, REAL lambda, REAL *d, REAL *u,
+                          hipStream_t st) {
+  constexpr int V = 16 / (int)sizeof(REAL);
+  const int T = cfg.W * cfg.P;
+  const size_t lds = hyb::ring_bytes<REAL>(T, 2 + V);
+  const int64_t blocks = (g.n0 + cfg.W * V - 1) / (cfg.W * V) * g.n1;
+  hipLaunchKernelGGL((adi_vec_kernel<REAL, M, INC>), dim3((unsigned)blocks), dim3(T), lds, st, g,
+                     cfg.P, cfg.W, cfg.G, lambda, d, u);
+  return hipGetLastError();
+}
+
+
+// The x sweep the same way, every access in chunk order: a lane takes M rows (32
+// bytes: two vectors) of LN lines j0 .. j0 + LN - 1 of one k, P lanes of one wave a
+// line, 64 / P groups of lines a wave. The right-hand side's neighbours: along x from the
+// lanes p-1 and p+1 by ds_bpermute, along y the lines themselves and one on either
+// side, along z two more lines each. No LDS tile, no transpose, no barrier. LN = 4 in
+// FP64, 2 in FP32 (256^3 step: FP64 LN = 1, 2, 4 172, 154.5, 150 us; FP32 84.5, 80.9, 83.9).
+// Against the tiled sweep, FP64, and one line per lane, FP32: 256^3 64.0 to 46.3 and 28.1
+// to 24.1 us; 200 x 168 x 147 28.8 to 21.9 and 14.3 to 12.9.
+template <typename REAL, int M, int LN>
+__global__ __launch_bounds__(64) void adi_xvec_kernel(int nx, int ny, int nz, int P, int G,
+                                                      REAL lambda, REAL *__restrict__ d,
+                                                      const REAL *__restrict__ u) {
+  constexpr int V = 16 / (int)sizeof(REAL), Q = M / V;
+  typedef REAL vec __attribute__((ext_vector_type(V)));
+  const int W = 64 / P;
+  hyb::Lane L{};
+  L.P = P; L.W = W; L.T = 64;
+  L.t = threadIdx.x;
+  L.w = L.t / P;
+  L.p = L.t - L.w * P;
+  L.pstep = 1;
+  hyb::Ring ring{nullptr, 0, 0};  // not used: the systems are wave-local
+  const uint32_t groups = (uint32_t)((ny + W * LN - 1) / (W * LN));
+  const uint32_t id = hyb::xcd_remap(blockIdx.x, gridDim.x, G);
+  const int k = (int)(id / groups);
+  const int j0 = ((int)(id - (uint32_t)k * groups) * W + L.w) * LN;
+  const bool active = L.w < W && j0 < ny;  // (64 - W * P lanes have no line)
+  const bool k_inner = k > 0 && k < nz - 1;
+  const int row0 = L.p * M;
+
+  // vector q of line j, plane k + dk: lines and rows outside are read from inside the
+  // grid; they feed right-hand sides that are 0 below, or no stored value
+  auto ldv = [&](int j, int dk, int q) {
+    const int jj = j < 0 ? 0 : j < ny ? j : ny - 1;
+    const int row = row0 + q * V < nx ? row0 + q * V : nx - V;
+    const uint32_t e = ((uint32_t)(k + dk) * (uint32_t)ny + (uint32_t)jj) * (uint32_t)nx + (uint32_t)row;
+    return *reinterpret_cast<const vec *>(reinterpret_cast<const char *>(u) +
+                                          e * (uint32_t)sizeof(REAL));
+  };
+  const int dz = k_inner ? 1 : 0;
+  REAL c[LN + 2][M], zm[LN][M], zp[LN][M];
+#pragma unroll
+  for (int l = 0; l < LN + 2; ++l) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const vec v = ldv(j0 - 1 + l, 0, q);
+#pragma unroll
+      for (int e = 0; e < V; ++e) c[l][q * V + e] = v[e];
+    }
+  }
+#pragma unroll
+  for (int l = 0; l < LN; ++l) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const vec v = ldv(j0 + l, -dz, q), w = ldv(j0 + l, dz, q);
+#pragma unroll
+      for (int e = 0; e < V; ++e) {
+        zm[l][q * V + e] = v[e];
+        zp[l][q * V + e] = w[e];
+      }
+    }
+  }
+
+  REAL x[LN][M];
+  {
+    REAL edge[2 * LN], lo[2 * LN], hi[2 * LN];
+#pragma unroll
+    for (int l = 0; l < LN; ++l) {
+      edge[2 * l] = c[l + 1][M - 1];
+      edge[2 * l + 1] = c[l + 1][0];
+    }
+    hyb::exchange<3, 2 * LN>(L, ring, true, edge, 1, L.p > 0, lo, 1, L.p + 1 < P, hi);
+#pragma unroll
+    for (int l = 0; l < LN; ++l) {
+      const bool line_inner = k_inner && j0 + l > 0 && j0 + l < ny - 1;
+#pragma unroll
+      for (int r = 0; r < M; ++r) {
+        const bool inner = line_inner && row0 + r > 0 && row0 + r < nx - 1;
+        const REAL xm = r > 0 ? c[l + 1][r - 1] : lo[2 * l];
+        const REAL xp = r < M - 1 ? c[l + 1][r + 1] : hi[2 * l + 1];
+        x[l][r] = inner ? adi_rhs(lambda, xm, xp, c[l][r], c[l + 2][r], zm[l][r], zp[l][r],
+                                  c[l + 1][r])
+                        : REAL(0);
+      }
+    }
+  }
+  adi_lines<REAL, M, LN, true>(L, ring, lambda, nx, row0, x, [] {});
+  if (!active) return;
+#pragma unroll
+  for (int l = 0; l < LN; ++l) {
+    if (j0 + l >= ny) break;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      if (row0 + q * V >= nx) break;
+      vec v;
+#pragma unroll
+      for (int e = 0; e < V; ++e) v[e] = x[l][q * V + e];
+      const uint32_t e = ((uint32_t)k * (uint32_t)ny + (uint32_t)(j0 + l)) * (uint32_t)nx +
+                         (uint32_t)(row0 + q * V);
+      *reinterpret_cast<vec *>(reinterpret_cast<char *>(d) + e * (uint32_t)sizeof(REAL)) = v;
+    }
+  }
+}
+
+// Rows per lane of adi_xvec_kernel: 32 bytes, twice that for lines that 64 lanes
+// of 32 do not hold; 0 where it does not apply: lines of whole 16-byte vectors,
+// aligned, within a wave, arrays below 4 GiB.
 template <typename REAL>
-hipError_t launch_adi_x_direct(const Geom &g, const HybridCfg &cfg, const AdiCoef<REAL> &kc,
-                               REAL *d, const REAL *u, hipStream_t st) {
-  const int64_t blocks = (g.n0 + cfg.W - 1) / cfg.W * g.n1;
-  hipLaunchKernelGGL(adi_x_direct_kernel<REAL>, dim3((unsigned)blocks), dim3(cfg.W * cfg.P), 0,
-                     st, g, cfg.P, cfg.W, cfg.G, kc, d, u);
+int adi_xvec_rows(const REAL *d, const REAL *u, int nx, int ny, int nz) {
+  constexpr int V = 16 / (int)sizeof(REAL);
+  if (nx % V != 0 || nx > 64 * 4 * V ||
+      (uint64_t)nx * (uint64_t)ny * (uint64_t)nz * sizeof(REAL) > 0xffffffffull ||
+      ((reinterpret_cast<uintptr_t>(d) | reinterpret_cast<uintptr_t>(u)) & 15) != 0)
+    return 0;
+  return nx > 64 * 2 * V ? 4 * V : 2 * V;
+}
+
+template <typename REAL, int M, int LN>
+hipError_t launch_adi_xvec(REAL lambda, REAL *d, const REAL *u, int nx, int ny, int nz,
+                           hipStream_t st) {
+  const int P = (nx + M - 1) / M, lines = 64 / P * LN;
+  const int64_t blocks = (int64_t)((ny + lines - 1) / lines) * nz;
+  hipLaunchKernelGGL((adi_xvec_kernel<REAL, M, LN>), dim3((unsigned)blocks), dim3(64), 0, st, nx,
+                     ny, nz, P, 8, lambda, d, u);
   return hipGetLastError();
 }
 
@@ -473,6 +675,19 @@ tridStatus_t adi_sweep(int dev, REAL lambda, REAL *d, REAL *u, int nx, int ny, i
   const bool contig = sd == 0;
   hipError_t e;
   if (RHS && !contig) return TRID_STATUS_INTERNAL_ERROR;
+  if constexpr (RHS) {
+    constexpr int M = 32 / (int)sizeof(REAL), LN = sizeof(REAL) == 8 ? 4 : 2;
+    const int rows = adi_xvec_rows<REAL>(d, u, nx, ny, nz);
+    if (rows != 0) {
+      e = rows == M ? launch_adi_xvec<REAL, M, LN>(lambda, d, u, nx, ny, nz, st)
+                    : launch_adi_xvec<REAL, 2 * M, 2>(lambda, d, u, nx, ny, nz, st);
+      if (e != hipSuccess) {
+        record_hip_error(e);
+        return TRID_STATUS_EXECUTION_FAILED;
+      }
+      return TRID_STATUS_SUCCESS;
+    }
+  }
   // The right-hand side is computed in the sweep unless FP32 x lines are
   // at 16 rows per lane (they would spill) or the grid is 4 GiB or more (the
   // sweep's loads use 32-bit byte offsets): there preproc writes du and the
@@ -486,13 +701,18 @@ tridStatus_t adi_sweep(int dev, REAL lambda, REAL *d, REAL *u, int nx, int ny, i
                                     nullptr, nullptr, nullptr, nullptr, nx, ny, nz);
     if (sp != TRID_STATUS_SUCCESS) return sp;
   }
-  if (contig && rhs_here && adi_x_direct_ok<REAL>(g, cfg, d, u, nx)) {
-    e = launch_adi_x_direct<REAL>(g, cfg, kc, d, u, st);
-    if (e != hipSuccess) {
-      record_hip_error(e);
-      return TRID_STATUS_EXECUTION_FAILED;
+  if constexpr (!RHS) {
+    Geom vg;
+    HybridCfg vc;
+    if (!contig && adi_vec_cfg<REAL>(d, INC ? u : d, nx, ny, nz, sd, &vg, &vc)) {
+      e = vc.M == 16 ? launch_adi_vec<REAL, 16, INC>(vg, vc, lambda, d, u, st)
+                     : launch_adi_vec<REAL, 8, INC>(vg, vc, lambda, d, u, st);
+      if (e != hipSuccess) {
+        record_hip_error(e);
+        return TRID_STATUS_EXECUTION_FAILED;
+      }
+      return TRID_STATUS_SUCCESS;
     }
-    return TRID_STATUS_SUCCESS;
   }
 #define TRID_ADI_CASE(MM)                                                                  \
   case MM:                                                                                 \
