@@ -271,6 +271,28 @@ def test_mixed_f32_forced_strided_shapes(shape):
                 assert H.norm_rel_err(x.cpu().numpy(), xl) <= 1e-12, (sd, refine)
 
 
+@pytest.mark.parametrize("dims,sd,want", [
+    ([32, 512, 33], 2, (16, 16, 0)), ([32, 513, 33], 2, (32, 32, 3)),
+    ([33, 256, 33], 2, (16, 16, 0)), ([33, 257, 256], 2, (32, 32, 3)),
+    ([33, 257, 257], 2, (32, 32, 3)), ([33, 257, 321], 2, (32, 16, 3)),
+    ([17, 384, 520], 1, (32, 16, 3)), ([20, 450, 513], 1, (32, 32, 3)),
+    ([5, 700, 9], 1, (16, 16, 0))])
+def test_mixed_f32_default_strided_shapes(dims, sd, want):
+    """The untuned strided shapes on both sides of their rules (512 workgroups of
+    32 systems; 8 lanes per system and whole waves at 16 systems), 0 and 1
+    refinements, against the long-double oracle of the promoted system at the
+    bars of test_mixed_f32_vs_long_double_oracle."""
+    rng = np.random.default_rng(sum(dims) + sd)
+    a, b, c, d = _f32_case(rng, int(np.prod(dims)))
+    xl = oracle.batch_ld(a, b, c, d, ndim=3, solvedim=sd, dims=dims)
+    t = [dev(v) for v in (a, b, c, d)]
+    for refine, tol in ((0, 1e-5), (1, 1e-12)):
+        x = api.mixed_f32_strided_batch(*t, solvedim=sd, dims=dims, refinements=refine, sync=True)
+        algo, M, _, W, _ = api.last_config()
+        assert (algo, M) == (10, want[0]) and W <= want[1], api.last_config()
+        assert H.norm_rel_err(x.cpu().numpy(), xl) <= tol, refine
+
+
 @pytest.mark.parametrize("shape", [(16, 2, 1), (16, 4, 8), (8, 1, 8), (8, 8, 1)])
 @pytest.mark.parametrize("N", [512, 300, 700, 37])
 def test_mixed_f32_forced_contig_lds(shape, N):

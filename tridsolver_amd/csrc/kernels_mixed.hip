@@ -193,7 +193,7 @@ __global__ __launch_bounds__(MIXED_THREADS) void mixed_wide_kernel(
   __syncthreads();
 
   double X[M];
-  mixed_chunk_acc<M, MIXED_MAX_STEPS, true, false, true>(
+  mixed_chunk_acc<M, MIXED_MAX_STEPS, true, true>(
       L, ring, [&](int r) { return sa[r * W]; }, B, [&](int r) { return sc[r * W]; }, D, refine,
       X);
   if (!L.active) return;

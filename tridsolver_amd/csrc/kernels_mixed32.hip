@@ -68,7 +68,7 @@ __global__ __launch_bounds__(M32_THREADS) void mixed32_kernel(
   hyb::to_chunk<M, CONTIG>(L, Cc, ftile);
   hyb::to_chunk<M, CONTIG>(L, D, ftile);
   double X[M];
-  mixed_chunk_acc<M, MIXED_MAX_STEPS, false, ONE, true>(
+  mixed_solve<M, MIXED_MAX_STEPS, ONE, CONTIG>(
       L, ring, [&](int r) { return A[r]; }, B, [&](int r) { return Cc[r]; }, D, refine, X);
   hyb::to_fetch<M, CONTIG>(L, X, dtile);
   hyb::store<M, CONTIG, true>(L, x, X);
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(M32_THREADS) void mixed32_lds_kernel(
     // the stored registers live instead
     asm volatile("" ::: "memory");
     double X[M];
-    mixed_chunk_acc<M, STEPS, false, ONE, true>(
+    mixed_solve<M, STEPS, ONE, false>(
         L, ring, [&](int r) { return tA[r * T + t]; }, B, [&](int r) { return tC[r * T + t]; },
         D, refine, X);
     hyb::store<M, false, true>(L, x, X);
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(M32_THREADS) void mixed32_lds_kernel(
     __syncthreads();
     const float *ca = tA + L.p * (M + 1), *cc = tC + L.p * (M + 1);
     double X[M];
-    mixed_chunk_acc<M, STEPS, false, ONE, true>(
+    mixed_solve<M, STEPS, ONE, false>(
         L, ring, [&](int r) { return ca[r]; }, B, [&](int r) { return cc[r]; }, D, refine, X);
     __syncthreads();  // a and c are read to the end before x overwrites the tile
     hyb::to_fetch<M, true>(L, X, dtile);
@@ -230,7 +230,7 @@ __global__ __launch_bounds__((M32Wide<M, W>::threads)) void mixed32_wide_kernel(
   __syncthreads();
 
   double X[M];
-  mixed_chunk_acc<M, M32Wide<M, W>::steps, false, ONE, true>(
+  mixed_solve<M, (M32Wide<M, W>::steps), ONE, false>(
       L, ring, [&](int r) { return sa[r * W]; }, B, [&](int r) { return sc[r * W]; }, D, refine,
       X);
   if (!L.active) return;
@@ -429,7 +429,12 @@ bool mixed32_cfg_valid(const Geom &g, const HybridCfg &c, int refine) {
 //   0.80 ms), else 16 x-neighbours in registers. More: a and c in LDS, 8
 //   rows per lane (16 past 4096 rows), 8 x-neighbours (y 0.89, z 1.21 ms
 //   at two; the wide kernel at 16 rows per lane 0.99 / 1.28,
-//   mixed32_kernel 1.58 / 2.03).
+//   mixed32_kernel 1.58 / 2.03). Above 8 lanes per system 128-byte rows leave
+//   one workgroup per CU (LDS), 64-byte rows two: 384^3 z 358 against 371 us, y
+//   327 either way, 250 x 333 x 200 y 127 against 140, 512 x 512 x 200 y 267 against
+//   275. At most 512 workgroups of 32 systems: 16 rows per lane in registers, 16
+//   x-neighbours (64^3 z 10.5 against 13.3 us, 128^3 y 13.6 against 19.0, 64 x 64 x 400
+//   z 14.1 against 19.5; 160^3 z, 800 workgroups, 32.8 against 33.1).
 bool mixed32_default_cfg(const Geom &g, int refine, HybridCfg *cfg) {
   HybridCfg c;
   const bool contig = g.stride == 1;
@@ -450,16 +455,20 @@ bool mixed32_default_cfg(const Geom &g, int refine, HybridCfg *cfg) {
     }
     return false;
   }
-  c.V = 3;
-  c.G = 32;
+  const bool few = (g.n0 + 31) / 32 * g.n1 <= 512;
   c.M = 32;
-  c.W = 32;
   c.P = (int)((g.N + c.M - 1) / c.M);
   c.P += c.P & 1;  // whole waves: W * P a multiple of 64
-  if (mixed32_cfg_valid(g, c, refine)) { *cfg = c; return true; }
+  for (int W : {16, 32}) {
+    if (few || (W == 16 && c.P <= 8)) continue;
+    c.V = 3;
+    c.W = W;
+    c.G = W == 16 ? 8 : 32;
+    if (mixed32_cfg_valid(g, c, refine)) { *cfg = c; return true; }
+  }
   c.V = 0;
   c.G = 8;
-  for (int M : {g.N >= 256 ? 16 : 8, 8, 16}) {
+  for (int M : {few || g.N >= 256 ? 16 : 8, 8, 16}) {
     c.M = M;
     c.P = (int)((g.N + M - 1) / M);
     c.W = 16;

@@ -624,13 +624,13 @@ __global__ __launch_bounds__(T) void rg_solve_mixed32(
       }
       __syncthreads();
       const float *ca = ftile + L.p * (M + 1), *cc = tC + L.p * (M + 1);
-      mixed_chunk_acc<M, MIXED_MAX_STEPS, false, ONE, true>(
+      mixed_solve<M, MIXED_MAX_STEPS, ONE, false>(
           L, ring, [&](int r) { return ca[r]; }, B, [&](int r) { return cc[r]; }, D, refine, X);
       __syncthreads();  // a and c are read to the end before x overwrites the tile
     } else {
       hyb::to_chunk<M, true>(L, A, ftile);
       hyb::to_chunk<M, true>(L, Cc, ftile);
-      mixed_chunk_acc<M, MIXED_MAX_STEPS, false, ONE, true>(
+      mixed_solve<M, MIXED_MAX_STEPS, ONE, false>(
           L, ring, [&](int r) { return A[r]; }, B, [&](int r) { return Cc[r]; }, D, refine, X);
     }
     hyb::to_fetch<M, true>(L, X, dtile);

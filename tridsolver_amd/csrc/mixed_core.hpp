@@ -34,15 +34,11 @@ constexpr int MIXED_MAX_STEPS = 9;  // PCR steps for P <= 512
 // the system exactly (TB = float: the FP64 residual promotes them). The ring
 // needs slots of 2 doubles per thread. With STORE_INV false the pivots
 // 1/beta_i are recomputed by every right-hand-side solve instead of being
-// kept in registers (same expression, same values). ONE is for callers that
-// never ask for more than one refinement: x0 stays in FP32 registers (its
-// FP64 value is exact), and x = x0 + dx is formed in FP64 only at the end --
-// the same values as the general loop, with M fewer registers live. FAST
-// takes the FP32 reciprocals of the factorisation from the hardware's
+// kept in registers (same expression, same values). FAST takes the FP32 reciprocals of the factorisation from the hardware's
 // approximate reciprocal (v_rcp_f32, about 1 ulp) instead of a correctly
 // rounded division: the factorisation only has to be close to A's, the FP64
 // residual and the refinement make up the difference.
-template <int M, int STEPS, bool STORE_INV = true, bool ONE = false, bool FAST = false,
+template <int M, int STEPS, bool STORE_INV = true, bool FAST = false,
           typename TB, typename GetA, typename GetC>
 __device__ __forceinline__ void mixed_chunk_acc(const hyb::Lane &L, hyb::Ring &ring, GetA Aof,
                                                 const TB (&B)[M], GetC Cof, const TB (&D)[M],
@@ -157,38 +153,6 @@ __device__ __forceinline__ void mixed_chunk_acc(const hyb::Lane &L, hyb::Ring &r
     for (int r = M - 2; r >= 0; --r) v[r] = v[r] - al[r] * ym - ga[r] * v[r + 1];
   };
 
-  if constexpr (ONE) {
-    float v[M];
-#pragma unroll
-    for (int r = 0; r < M; ++r) v[r] = (float)D[r];
-    solve_rhs(v);
-    if (refine > 0) {
-      float xprev = 0, xnext = 0;  // neighbour chunks' boundary values of x0
-      {
-        float *q = ring.next<float>();
-        q[t] = v[0]; q[T + t] = v[M - 1];
-        __syncthreads();
-        if (p > 0) xprev = q[T + t - ps];
-        if (p + 1 < P) xnext = q[t + ps];
-      }
-      float w[M];
-#pragma unroll
-      for (int r = 0; r < M; ++r) {
-        const double xl = r > 0 ? v[r - 1] : xprev;
-        const double xr = r < M - 1 ? v[r + 1] : xnext;
-        const double res = (double)D[r] - ((double)B[r] * (double)v[r] + (double)Aof(r) * xl +
-                                           (double)Cof(r) * xr);
-        w[r] = (float)res;
-      }
-      solve_rhs(w);
-#pragma unroll
-      for (int r = 0; r < M; ++r) X[r] = (double)v[r] + (double)w[r];
-    } else {
-#pragma unroll
-      for (int r = 0; r < M; ++r) X[r] = (double)v[r];
-    }
-    return;
-  }
   {
     float v[M];
 #pragma unroll
@@ -223,12 +187,138 @@ __device__ __forceinline__ void mixed_chunk_acc(const hyb::Lane &L, hyb::Ring &r
 }
 
 // All four operands in registers.
+// The same for FP32 operands and at most one refinement, which keeps x0 in FP32
+// registers (its FP64 value is exact) and forms x = x0 + dx in FP64 only at the
+// end. Factorisation and the first solve are one sweep in row order, so that it can
+// follow loads in flight (hyb::sweep_carry's form: the chunk's first unknown is carried
+// along), and share the PCR's exchanges; the second solve reads al, ga and the PCR's
+// coefficients back and forms the pivots again. WAVE: contiguous systems, which may
+// lie in one wave. Ring slots of 3 floats per thread.
+template <int M, int STEPS, bool WAVE, typename GetA, typename GetC>
+__device__ __forceinline__ void mixed_one(const hyb::Lane &L, hyb::Ring &ring, GetA Aof,
+                                          const float (&B)[M], GetC Cof, const float (&D)[M],
+                                          int refine, double (&X)[M]) {
+  const bool wave = WAVE && hyb::wave_local(L);
+  float ga[M], al[M], v[M];
+  float f[3] = {0.0f, -1.0f, 0.0f};  // the first unknown: f_a, f_g, f_d
+  float an = Aof(0), cn = Cof(0);    // the next row's a and c, read ahead of it
+#pragma unroll
+  for (int r = 0; r < M; ++r) {
+    const float ar = an, cr = cn;
+    if (r + 1 < M) {
+      an = Aof(r + 1);
+      cn = Cof(r + 1);
+    }
+    const float inv = __builtin_amdgcn_rcpf(r == 0 ? B[0] : B[r] - ar * ga[r - 1]);
+    al[r] = r == 0 ? ar * inv : -ar * al[r - 1] * inv;
+    ga[r] = cr * inv;
+    v[r] = r == 0 ? D[0] * inv : (D[r] - ar * v[r - 1]) * inv;
+    if (r < M - 1) {
+      f[2] = f[2] - f[1] * v[r];
+      f[0] = f[0] - f[1] * al[r];
+      f[1] = -f[1] * ga[r];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  const float al_e = al[M - 1], ga_e = ga[M - 1];
+  float nx[3];
+  hyb::from_above<3>(L, ring, wave, f, nx);
+  const float invB = __builtin_amdgcn_rcpf(1.0f - ga_e * nx[0]);
+  // PCR: A, C, D; a step's A, C and reciprocal are kept for the second solve
+  float q[3] = {al_e * invB, -ga_e * nx[1] * invB, (v[M - 1] - ga_e * nx[2]) * invB};
+  float sA[STEPS], sC[STEPS], sR[STEPS];
+#pragma unroll
+  for (int s = 0; s < STEPS; ++s) {
+    sA[s] = q[0]; sC[s] = q[1]; sR[s] = 1.0f;
+    if ((1 << s) < L.P) {
+      float m[3], n[3];
+      hyb::from_both<3>(L, ring, wave, 1 << s, q, m, n);
+      sR[s] = __builtin_amdgcn_rcpf(1.0f - sA[s] * m[1] - sC[s] * n[0]);
+      q[0] = -sR[s] * sA[s] * m[0];
+      q[1] = -sR[s] * sC[s] * n[1];
+      q[2] = sR[s] * (q[2] - sA[s] * m[2] - sC[s] * n[2]);
+    }
+  }
+  auto substitute = [&](float (&w)[M], float y) {
+    const float yv[1] = {y};
+    float ym[1];
+    hyb::from_below<1>(L, ring, wave, yv, ym);
+    w[M - 1] = y;
+#pragma unroll
+    for (int r = M - 2; r >= 0; --r) w[r] = w[r] - al[r] * ym[0] - ga[r] * w[r + 1];
+  };
+  substitute(v, q[2]);
+  if (refine <= 0) {
+#pragma unroll
+    for (int r = 0; r < M; ++r) X[r] = (double)v[r];
+    return;
+  }
+  float xprev = 0, xnext = 0;  // neighbour chunks' boundary values of x0
+  {
+    const float e[2] = {v[0], v[M - 1]};
+    float lo[2], hi[2];
+    hyb::from_both<2>(L, ring, wave, 1, e, lo, hi);
+    xprev = lo[1];
+    xnext = hi[0];
+  }
+  float w[M], f_d = 0.0f, f_g = -1.0f;
+  an = Aof(0);
+  cn = Cof(0);
+#pragma unroll
+  for (int r = 0; r < M; ++r) {
+    const float ar = an, cr = cn;
+    if (r + 1 < M) {
+      an = Aof(r + 1);
+      cn = Cof(r + 1);
+    }
+    const double xl = r > 0 ? v[r - 1] : xprev;
+    const double xr = r < M - 1 ? v[r + 1] : xnext;
+    const double res =
+        (double)D[r] - ((double)B[r] * (double)v[r] + (double)ar * xl + (double)cr * xr);
+    const float inv = __builtin_amdgcn_rcpf(r == 0 ? B[0] : B[r] - ar * ga[r - 1]);
+    w[r] = r == 0 ? (float)res * inv : ((float)res - ar * w[r - 1]) * inv;
+    if (r < M - 1) {
+      f_d = f_d - f_g * w[r];
+      f_g = -f_g * ga[r];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  float y;
+  {
+    const float fv[1] = {f_d};
+    float nd[1];
+    hyb::from_above<1>(L, ring, wave, fv, nd);
+    y = (w[M - 1] - ga_e * nd[0]) * invB;
+  }
+#pragma unroll
+  for (int s = 0; s < STEPS; ++s) {
+    if ((1 << s) < L.P) {
+      const float yv[1] = {y};
+      float m[1], n[1];
+      hyb::from_both<1>(L, ring, wave, 1 << s, yv, m, n);
+      y = sR[s] * (y - sA[s] * m[0] - sC[s] * n[0]);
+    }
+  }
+  substitute(w, y);
+#pragma unroll
+  for (int r = 0; r < M; ++r) X[r] = (double)v[r] + (double)w[r];
+}
+
+// FP32 operands: at most one refinement (ONE), or any number.
+template <int M, int STEPS, bool ONE, bool WAVE, typename GetA, typename GetC>
+__device__ __forceinline__ void mixed_solve(const hyb::Lane &L, hyb::Ring &ring, GetA Aof,
+                                            const float (&B)[M], GetC Cof, const float (&D)[M],
+                                            int refine, double (&X)[M]) {
+  if constexpr (ONE) mixed_one<M, STEPS, WAVE>(L, ring, Aof, B, Cof, D, refine, X);
+  else mixed_chunk_acc<M, STEPS, false, true>(L, ring, Aof, B, Cof, D, refine, X);
+}
+
 template <int M>
 __device__ __forceinline__ void mixed_chunk(const hyb::Lane &L, hyb::Ring &ring,
                                             const double (&A)[M], const double (&B)[M],
                                             const double (&Cc)[M], const double (&D)[M],
                                             int refine, double (&X)[M]) {
-  mixed_chunk_acc<M, MIXED_MAX_STEPS, true, false, true>(
+  mixed_chunk_acc<M, MIXED_MAX_STEPS, true, true>(
       L, ring, [&](int r) { return A[r]; }, B, [&](int r) { return Cc[r]; }, D, refine, X);
 }
 
@@ -282,7 +372,7 @@ __device__ __forceinline__ void mixed_contig_lds(const hyb::Lane &L, hyb::Ring &
   __syncthreads();
   const double *ca = tA + L.p * (M + 1), *cc = tC + L.p * (M + 1);
   double X[M];
-  mixed_chunk_acc<M, STEPS, true, false, true>(
+  mixed_chunk_acc<M, STEPS, true, true>(
       L, ring, [&](int r) { return ca[r]; }, B, [&](int r) { return cc[r]; }, D, refine, X);
   hyb::to_fetch<M, true>(L, X, tA);
   // the store base is recomputed behind an empty asm, so that the load
