@@ -59,6 +59,20 @@ def test_long_vs_oracle(dims, sd, inc, dtype):
     assert cfg[0] == _expected_algo(dims[sd], sd, dtype == np.float64), cfg
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("dims,sd", [([32, 4352, 2], 1), ([33, 4353, 2], 1), ([2, 4097], 1),
+                                     ([15, 4607, 3], 1), ([64, 4224], 1), ([7, 9, 4225], 2),
+                                     ([16, 16, 4480], 2), ([31, 2, 4479], 2)])
+def test_long_strided_segment_edges(dims, sd, dtype):
+    """Strided systems of whole segments (256 rows FP64, 128 FP32), one row more
+    or less, whose last segment holds one row; groups of systems cut short;
+    rows that are and are not 128-byte aligned (nontemporal and plain loads).
+    Plain and Inc, against the oracle (run_case's tolerances)."""
+    for inc in (False, True):
+        cfg = run_case(dims, sd, dtype, inc, (0, 0, 0), seed=sum(dims) + 3)
+        assert cfg[0] == LONG, cfg
+
+
 @pytest.mark.parametrize("sd", [0, 1, 2])
 def test_long_padded(sd):
     """Halo-padded arrays, pointers offset by one halo layer: the padding is
