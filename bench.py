@@ -557,7 +557,7 @@ def bench_ragged(torch, api, tune):
         gbs = (bpp * total + 8 * (len(off))) / (gms * 1e-3) / 1e9
         out[key]["graph"] = {"ms_per_replay": round(gms, 4),
                              "gpts_s": round(total / gms / 1e6, 2), "alg_GBs": round(gbs, 1),
-                             "what": "planning kernels + persistent solve captured once in a "
+                             "what": "planning kernels + solve captured once in a "
                                      "hipGraph, replayed back to back"}
         del a, b, c, d
     # FP32 sweeps + FP64 refinement on the same 40,000 FP64 systems, at 1 and
