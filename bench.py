@@ -509,7 +509,7 @@ def bench_adjoint(torch, api, tune, n=256):
 
 
 def ragged_graph_ms(torch, api, a, b, c, d, toff, reps=20):
-    """Mean time per replay of the ragged solve (plan + persistent launch)
+    """Mean time per replay of the ragged solve (plan + solve launch)
     captured once in a hipGraph on a side stream whose workspace is reserved
     beforehand; events on that stream around `reps` back-to-back replays."""
     s = torch.cuda.Stream()

@@ -247,15 +247,21 @@ def test_solve_to_equals_solve_in_place(dims, sd, force, dtype):
     ([61, 300, 520], 1, 256),    # misaligned rows (plain access), partial last group
     ([64, 512, 300], 2, 256), ([256, 8, 512], 2, 128),
     ([16, 512, 2], 1, 128), ([16, 513, 2], 1, 128), ([40, 1023, 1], 1, 128),
-    ([17, 2, 1024], 2, 128), ([7, 1000, 1], 1, 128)])
+    ([17, 2, 1024], 2, 128), ([7, 1000, 1], 1, 128), ([300, 513, 14], 1, 128),
+    ([300, 14, 1024], 2, 128), ([64, 513, 64], 1, 128)])
 def test_default_strided_shapes(dims, sd, seg, inc, dtype):
     """The default strided shapes at the edges of their ranges: 256-byte rows
     for systems up to 512 rows in many workgroups, 128-byte rows else, up to 1024
     rows; waves whose rows all lie inside their systems beside waves with rows
     past N or systems past n0. FP32 may take 128-byte rows where FP64 takes
-    256."""
+    256, and runs systems over 512 rows in at most 256 groups of 16 by the plain
+    kernel."""
     cfg = run_case(dims, sd, dtype, inc, (0, 0, 0), seed=sum(dims))
     esize = np.dtype(dtype).itemsize
+    groups = -(-dims[0] // 16) * (int(np.prod(dims)) // dims[0] // dims[sd])
+    if dtype == np.float32 and dims[sd] > 512 and groups <= 256:
+        assert cfg[:2] == (3, 16), cfg
+        return
     assert cfg[0] == 8
     assert cfg[3] * esize in ((seg,) if dtype == np.float64 else (128, 256))
 

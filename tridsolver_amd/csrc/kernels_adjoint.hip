@@ -378,7 +378,7 @@ bool adjoint_default_cfg(const Geom &g, HybridCfg *cfg) {
   // as the forward solve where they fit the adjoint's register budget, else
   // the next valid one.
   HybridCfg c;
-  if (g.stride != 1 && hybrid_default_cfg<REAL>(g, &c) && adjoint_wide<REAL>(g, c)) {
+  if (hybrid_wide_default_cfg<REAL>(g, &c) && adjoint_wide<REAL>(g, c)) {
     if (sizeof(REAL) == 4 && g.N <= 512 && wide::wide_many_groups<REAL>(g)) {
       // nine streams of 128-byte rows want more bytes per row than the
       // solve's five: 256-byte rows at every length (256^3 FP32 y / z 108 /

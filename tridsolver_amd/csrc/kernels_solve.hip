@@ -356,44 +356,52 @@ bool hybrid_plain_cfg(const Geom &g, HybridCfg *cfg) {
 }
 
 template <typename REAL>
+bool hybrid_wide_default_cfg(const Geom &g, HybridCfg *cfg) {
+  if (g.stride == 1) return false;
+  // Strided systems: the wide variant (kernels_wide.hip). The lines below
+  // lie where both sides were measured, in three sets of arrays used in
+  // turn (so that no call finds its data in a cache), on 40 grids from
+  // 33 x 80 x 50 to 512^3:
+  //  - rows of 256 bytes where such a workgroup holds the system (N <= 512)
+  //    and there are enough of them (wide_many_groups): fewer row segments
+  //    and fewer misaligned edges per byte (FP64 777 x 300 x 250 y 504 against
+  //    532 us, 256^3 z 127 against 155). 128-byte rows otherwise.
+  //  - FP64 at 16 rows per lane (512^3 z 0.94 against 0.95 ms at 32, 251 x
+  //    300 x 300 y 213 against 222 us). FP32 at 32 rows per lane on 256-byte
+  //    rows of 257-512 (512^3 y 0.466 against 0.484 ms for 16 on 128-byte
+  //    rows, given 1024 such workgroups: 200 x 300 x 150 y, 600, 56 against 48
+  //    us) and above 512, else at 16 on 128-byte rows (203 x 170 x 300 y 52
+  //    against 55 us).
+  //  - workgroups dealt to the XCDs in 8 ranges (G), so that neighbouring
+  //    segments, which share lines where rows are misaligned, pass through
+  //    one L2 (777 x 300 x 250 z 494 against 544 us at G = 1); in plain order
+  //    where rows lie a power of two of at least 64 KiB apart (512^3 z 0.94
+  //    against 1.04 ms at G = 8, 256^3 z 127 against 140 us).
+  HybridCfg c;
+  const bool fp64 = sizeof(REAL) == 8;
+  const int64_t row_bytes = g.stride * (int64_t)sizeof(REAL);
+  const bool wide = g.N <= 512 && (fp64 ? wide::wide_many_groups<REAL>(g)
+                                        : g.N > 256 && wide::wide_many_groups<REAL>(g, 1024));
+  c.M = fp64 || (!wide && g.N <= 512) ? 16 : 32;
+  c.W = (wide ? 256 : 128) / (int)sizeof(REAL);
+  const int per_wave = std::max(1, 64 / c.W);
+  c.P = (int)((g.N + c.M - 1) / c.M);
+  c.P = (c.P + per_wave - 1) / per_wave * per_wave;
+  c.G = row_bytes >= (64 << 10) && (row_bytes & (row_bytes - 1)) == 0 ? 1 : 8;
+  c.V = 3;
+  if (!hybrid_cfg_valid<REAL>(g, c)) return false;
+  *cfg = c;
+  return true;
+}
+
+template <typename REAL>
 bool hybrid_default_cfg(const Geom &g, HybridCfg *cfg) {
-  if (g.stride != 1) {
-    // Strided systems: the wide variant (kernels_wide.hip). The lines below
-    // lie where both sides were measured, in three sets of arrays used in
-    // turn (so that no call finds its data in a cache), on 40 grids from
-    // 33 x 80 x 50 to 512^3:
-    //  - rows of 256 bytes where such a workgroup holds the system (N <= 512)
-    //    and there are enough of them (wide_many_groups): fewer row segments
-    //    and fewer misaligned edges per byte (FP64 777 x 300 x 250 y 504 against
-    //    532 us, 256^3 z 127 against 155). 128-byte rows otherwise.
-    //  - FP64 at 16 rows per lane (512^3 z 0.94 against 0.95 ms at 32, 251 x
-    //    300 x 300 y 213 against 222 us). FP32 at 32 rows per lane on 256-byte
-    //    rows of 257-512 (512^3 y 0.466 against 0.484 ms for 16 on 128-byte
-    //    rows, given 1024 such workgroups: 200 x 300 x 150 y, 600, 56 against 48
-    //    us) and above 512, else at 16 on 128-byte rows (203 x 170 x 300 y 52
-    //    against 55 us).
-    //  - workgroups dealt to the XCDs in 8 ranges (G), so that neighbouring
-    //    segments, which share lines where rows are misaligned, pass through
-    //    one L2 (777 x 300 x 250 z 494 against 544 us at G = 1); in plain order
-    //    where rows lie a power of two of at least 64 KiB apart (512^3 z 0.94
-    //    against 1.04 ms at G = 8, 256^3 z 127 against 140 us).
-    HybridCfg c;
-    const bool fp64 = sizeof(REAL) == 8;
-    const int64_t row_bytes = g.stride * (int64_t)sizeof(REAL);
-    const bool wide = g.N <= 512 && (fp64 ? wide::wide_many_groups<REAL>(g)
-                                          : g.N > 256 && wide::wide_many_groups<REAL>(g, 1024));
-    c.M = fp64 || (!wide && g.N <= 512) ? 16 : 32;
-    c.W = (wide ? 256 : 128) / (int)sizeof(REAL);
-    const int per_wave = std::max(1, 64 / c.W);
-    c.P = (int)((g.N + c.M - 1) / c.M);
-    c.P = (c.P + per_wave - 1) / per_wave * per_wave;
-    c.G = row_bytes >= (64 << 10) && (row_bytes & (row_bytes - 1)) == 0 ? 1 : 8;
-    c.V = 3;
-    if (hybrid_cfg_valid<REAL>(g, c)) {
-      *cfg = c;
-      return true;
-    }
-  }
+  // FP32 systems of more than 512 rows so few that workgroups of 16 take one round
+  // (one per CU) run the plain kernel at 16 rows per lane there: 32 x 600 x 128 y 12.3 us
+  // against 15.1 with the wide one's 32, 64 x 64 x 800 z 19.8 against 23.6, 32 x 1000 x 20 y
+  // 15.5 against 17.7. In two rounds it loses: 32 x 600 x 136 y 21.6 against 15.1.
+  const bool few = sizeof(REAL) == 4 && g.N > 512 && (g.n0 + 15) / 16 * g.n1 <= 256;
+  if (!few && hybrid_wide_default_cfg<REAL>(g, cfg)) return true;
   // Contiguous systems of 4097-8192 rows: one per 256-thread workgroup at 32
   // rows per lane (variant 4), FP64 throughout (4500 / 6000 / 8192 rows: 3.8
   // / 4.3 / 4.7 TB/s against 3.2 / 3.7 / 4.0 with 512 lanes of 16 rows), FP32
@@ -466,6 +474,7 @@ hipError_t launch_hybrid(const Geom &g, const HybridCfg &cfg, const REAL *a,
       const REAL *, const REAL *, const REAL *, REAL *, REAL *, hipStream_t);    \
   template bool hybrid_cfg_valid<REAL>(const Geom &, const HybridCfg &);         \
   template bool hybrid_default_cfg<REAL>(const Geom &, HybridCfg *);               \
+  template bool hybrid_wide_default_cfg<REAL>(const Geom &, HybridCfg *);          \
   template bool hybrid_plain_cfg<REAL>(const Geom &, HybridCfg *);
 
 TRID_INST(float)

@@ -260,6 +260,9 @@ const HybridCfg &forced_config();
 // are too long for one workgroup.
 template <typename REAL>
 bool hybrid_default_cfg(const Geom &g, HybridCfg *cfg);
+// The wide variant's part of it (strided systems), also the strided adjoint's shape.
+template <typename REAL>
+bool hybrid_wide_default_cfg(const Geom &g, HybridCfg *cfg);
 // The default among plain-kernel shapes only (V = 0).
 template <typename REAL>
 bool hybrid_plain_cfg(const Geom &g, HybridCfg *cfg);

@@ -26,7 +26,7 @@ template <typename REAL>
 bool adjoint_tuned_config(int dev, const Geom &g, bool grads, HybridCfg *cfg);
 
 // Rows per lane M, workgroups per CU and solve launches (1, or 2 with the
-// short systems apart) of the ragged persistent kernel for systems up to
+// short systems apart) of the ragged kernel for systems up to
 // max_len long.
 template <typename REAL>
 void ragged_tuned_config(int dev, int64_t max_len, int *M, int *per_cu, int *launches);
