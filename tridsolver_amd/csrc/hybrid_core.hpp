@@ -770,7 +770,13 @@ __device__ __forceinline__ uint32_t lds_address(const void *p) {
   return (uint32_t)(uintptr_t)(lds_void *)p;
 }
 
-// One global->LDS wave instruction: lane l's dword at base + off goes to LDS
+// Global->LDS loads of one wave (staging). The wave's LDS reads count in lgkmcnt
+// and the staging's LDS writes in vmcnt, which nothing orders: a load that returns
+// early would replace what an earlier read of the same slots has yet to take.
+// So staging starts with a wait for the wave's LDS reads. Slots that other
+// waves read need a workgroup barrier before it.
+//
+// dword() is one wave instruction: lane l's dword at base + off goes to LDS
 // byte lds + 4 l (lds wave-uniform). Written in asm because the compiler waits
 // for every outstanding load (vmcnt(0)) before a register load issued behind
 // the builtin is used; it does not see this one. It has no register
@@ -778,12 +784,15 @@ __device__ __forceinline__ uint32_t lds_address(const void *p) {
 // register load that it issues after the staging: loads whose address passed
 // through loads_after_stage() come behind it, and stage_done(v) waits until v,
 // one of them, has arrived.
-__device__ __forceinline__ void stage_dword(uint32_t lds, const void *base, uint32_t off) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
-               :
-               : "s"(lds), "v"(off), "s"(base)
-               : "m0", "memory");
-}
+struct Stage {
+  __device__ __forceinline__ Stage() { asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory"); }
+  __device__ __forceinline__ void dword(uint32_t lds, const void *base, uint32_t off) const {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                 :
+                 : "s"(lds), "v"(off), "s"(base)
+                 : "m0", "memory");
+  }
+};
 __device__ __forceinline__ uint32_t loads_after_stage(uint32_t off) {
   asm volatile("" : "+v"(off) : : "memory");
   return off;
@@ -853,15 +862,16 @@ __device__ __forceinline__ void long32_solve(int64_t base, int N, unsigned char 
     const int rl = ll * E / 64;
     const REAL *sa = a + base;
     const uint32_t lds = lds_address(tile);
+    const Stage stage;
     for (int k = wv * (64 * M / E); k < (wv + 1) * (64 * M / E) && k * E < N; ++k) {
       const int row = k * E + rl;
       const bool ok = row >= 1 && row < N;
       const uint32_t off = (uint32_t)(k * 256 + 4 * ll);
       if constexpr (E == M) {  // FP64: the window is chunk k
-        if (ok) stage_dword(lds + k * (M + 1) * sizeof(REAL), sa, off);
+        if (ok) stage.dword(lds + k * (M + 1) * sizeof(REAL), sa, off);
       } else {  // FP32: chunks 2k and 2k+1
-        if (ok && ll < 32) stage_dword(lds + 2 * k * (M + 1) * sizeof(REAL), sa, off);
-        if (ok && ll >= 32) stage_dword(lds + (2 * k * (M + 1) + 1) * sizeof(REAL), sa, off);
+        if (ok && ll < 32) stage.dword(lds + 2 * k * (M + 1) * sizeof(REAL), sa, off);
+        if (ok && ll >= 32) stage.dword(lds + (2 * k * (M + 1) + 1) * sizeof(REAL), sa, off);
       }
     }
   }

@@ -52,6 +52,7 @@ template <typename REAL, int M, int SEG, int CH, bool WHOLE, int SHIFT = 0>
 __device__ __forceinline__ void wide_stage(const REAL *src, uint32_t tile, int row0, int lane,
                                            uint32_t row_bytes, int N, int64_t nsys) {
   constexpr int K = 256 / SEG;
+  const hyb::Stage stage;
   const int sub = (lane * 4) / SEG;
   const uint32_t byte = (uint32_t)(lane * 4) % SEG;
   if constexpr (WHOLE) {
@@ -62,7 +63,7 @@ __device__ __forceinline__ void wide_stage(const REAL *src, uint32_t tile, int r
       for (int q = 0; q < CH; ++q) {
         uint32_t off = o + (uint32_t)(q * M + r) * row_bytes;
         if (SHIFT) off -= r == 0 && q == 0 && row0 + sub == 0 ? 0u : row_bytes;
-        hyb::stage_dword(tile + q * wide_chunk_bytes(M, SEG) + r * SEG, src, off);
+        stage.dword(tile + q * wide_chunk_bytes(M, SEG) + r * SEG, src, off);
       }
   } else {
     if ((int)byte / (int)sizeof(REAL) >= nsys) return;
@@ -70,8 +71,8 @@ __device__ __forceinline__ void wide_stage(const REAL *src, uint32_t tile, int r
       for (int q = 0; q < CH; ++q) {
         const int row = row0 + q * M + r + sub;
         if (row < N)
-          hyb::stage_dword(tile + q * wide_chunk_bytes(M, SEG) + r * SEG, src,
-                           (uint32_t)(SHIFT && row > 0 ? row - 1 : row) * row_bytes + byte);
+          stage.dword(tile + q * wide_chunk_bytes(M, SEG) + r * SEG, src,
+                      (uint32_t)(SHIFT && row > 0 ? row - 1 : row) * row_bytes + byte);
       }
   }
 }
