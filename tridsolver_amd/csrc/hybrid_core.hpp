@@ -779,18 +779,19 @@ __device__ __forceinline__ uint32_t lds_address(const void *p) {
 // dword() is one wave instruction: lane l's dword at base + off goes to LDS
 // byte lds + 4 l (lds wave-uniform). Written in asm because the compiler waits
 // for every outstanding load (vmcnt(0)) before a register load issued behind
-// the builtin is used; it does not see this one. It has no register
-// output. Loads complete in order, so the caller waits for it through a
+// the builtin is used; it does not see this one. The LDS address is an input in
+// m0, which the compiler sets (s_nop: the wait that m0 needs between its write and
+// the load). The load has no register output. Loads complete in order, so the caller waits for it through a
 // register load that it issues after the staging: loads whose address passed
 // through loads_after_stage() come behind it, and stage_done(v) waits until v,
 // one of them, has arrived.
 struct Stage {
   __device__ __forceinline__ Stage() { asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory"); }
   __device__ __forceinline__ void dword(uint32_t lds, const void *base, uint32_t off) const {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+    asm volatile("s_nop 0\n\tglobal_load_lds_dword %1, %2"
                  :
-                 : "s"(lds), "v"(off), "s"(base)
-                 : "m0", "memory");
+                 : "{m0}"(lds), "v"(off), "s"(base)
+                 : "memory");
   }
 };
 __device__ __forceinline__ uint32_t loads_after_stage(uint32_t off) {
