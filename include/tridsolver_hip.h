@@ -269,13 +269,16 @@ EXTERN_C tridStatus_t tridDmtsvRaggedBatchNoAlloc(const TridParams *ctx, const d
                                                   const double *b, const double *c, double *d,
                                                   const int64_t *offsets, int64_t nsys,
                                                   int64_t max_len);
-/* Forces the ragged kernel's rows per lane (4, 8 or 16), workgroups per CU
- * and solve launches (1; 2: systems needing more than half a workgroup's
- * lanes, then the rest in half-size workgroups, two per CU; 3, at M = 16
- * only: one launch of 256-thread workgroups taking the systems over 4096 rows
- * at 32 rows per lane, then the rest) for this thread's calls; M = 0 restores
- * the tuned choice. The mixed ragged solve takes the same settings (its M = 4
- * and 8 always run in one launch; 3 is refused). */
+/* Forces the ragged kernel's rows per lane (4, 8 or 16), workgroups per CU of
+ * its resident grid (1 to 8; 0: no resident grid, one 256-thread workgroup per
+ * work item) and solve launches (1; 2, not with per_cu 0: systems needing more
+ * than half a workgroup's lanes, then the rest in half-size workgroups, two per
+ * CU; 3, at M = 16 only: a workgroup per item in one launch, whatever per_cu
+ * says, with the systems over 4096 rows at 32 rows per lane) for this thread's
+ * calls; M = 0 restores the tuned choice. M, per_cu = G and launches = W as
+ * tridHipLastConfig reports them force that call's shape. The mixed ragged
+ * solves take the same settings (M = 4 and 8 always run in one launch there;
+ * per_cu 0 and 3 launches are refused). */
 EXTERN_C tridStatus_t tridHipForceRaggedConfig(int M, int per_cu, int launches);
 
 /* ---- measurement ---------------------------------------------------------

@@ -70,12 +70,12 @@ tridStatus_t ragged_mixed(const TridParams *ctx, const double *a, const double *
     return s;
   HybridCfg rec;
   // M = 4 and 8 always run in one launch; the mixed solve has no
-  // three-launch split. Unforced, batches with systems over 4096 rows take
+  // three-launch split and no workgroup per item. Unforced, batches with systems over 4096 rows take
   // two launches (those systems in 512-thread workgroups, then the rest in
   // 256-thread ones, two per CU): 0.56 against 0.58 ms on 40,000 systems of
   // 8-8192 rows.
   const int launches = M != 16 ? 1 : forced ? tl_ragged_launches : (max_len > 4096 ? 2 : 1);
-  if (launches == 3) return TRID_STATUS_INVALID_VALUE;
+  if (launches == 3 || tl_ragged_per_cu == 0) return TRID_STATUS_INVALID_VALUE;
   rec.M = M; rec.P = 0; rec.W = launches; rec.G = tl_ragged_per_cu;
   record_config(9, &rec);
   s = finish(ctx, st, launch_ragged_mixed(M, a, b, c, d, offsets, nsys, tl_ragged_per_cu,
@@ -152,7 +152,7 @@ tridStatus_t ragged_mixed32(const TridParams *ctx, const float *a, const float *
   // launches: forced (1 or 2), else two where systems may exceed 4096 rows
   // (as the FP64-stored mixed solve)
   const int launches = tl_ragged_m ? tl_ragged_launches : (max_len > 4096 ? 2 : 1);
-  if (launches != 1 && launches != 2) return TRID_STATUS_INVALID_VALUE;
+  if ((launches != 1 && launches != 2) || tl_ragged_per_cu == 0) return TRID_STATUS_INVALID_VALUE;
   HybridCfg rec;
   rec.M = 16; rec.P = 0; rec.W = launches; rec.G = tl_ragged_per_cu;
   record_config(11, &rec);
@@ -326,8 +326,9 @@ EXTERN_C tridStatus_t tridHipForceRaggedConfig(int M, int per_cu, int launches) 
     tl_ragged_launches = 1;
     return TRID_STATUS_SUCCESS;
   }
-  if ((M != 4 && M != 8 && M != 16) || per_cu < 1 || per_cu > 8 || launches < 1 ||
-      launches > 3)
+  // per_cu 0, a workgroup per item, is one launch
+  if ((M != 4 && M != 8 && M != 16) || per_cu < 0 || per_cu > 8 || launches < 1 ||
+      launches > 3 || (per_cu == 0 && launches == 2))
     return TRID_STATUS_INVALID_VALUE;
   tl_ragged_m = M;
   tl_ragged_per_cu = per_cu;
