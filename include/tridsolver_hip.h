@@ -205,9 +205,12 @@ EXTERN_C tridStatus_t tridSmtsvStridedBatchAdjoint(const TridParams *ctx, const 
  * offsets[s] .. offsets[s+1]-1 of a, b, c, d (offsets: nsys+1 int64 values in
  * device memory, non-decreasing; nsys <= 2^31 - 1). Within a system the data
  * contract of tridsolver.h holds (a[first] and c[last] unused). max_len is an
- * upper bound of every length, known to the caller (at most 8192); a longer
- * system found on the device is skipped and, for a synchronous call, reported
- * as TRID_STATUS_INVALID_VALUE (an asynchronous call cannot report it). Four
+ * upper bound of every length, known to the caller (at most 8192), by which the
+ * kernel's shape is chosen. A longer system found on the device is solved all
+ * the same, but takes about 1.7 times as long, up to 8192 rows (4096 at 4 rows
+ * per lane, forced or tuned); beyond that it is skipped and, for a synchronous
+ * call, reported as TRID_STATUS_INVALID_VALUE (an asynchronous call cannot
+ * report it). Four
  * small planning kernels, then one solve launch over every system
  * (tridHipForceRaggedConfig can split it in two); capturable.
  * Needs tridHipRaggedWorkspaceBytes(nsys) of the stream's workspace (reserve

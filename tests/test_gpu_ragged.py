@@ -76,3 +76,32 @@ def test_forced_shapes_refused():
             api.ragged_batch_mixed(dev(a), dev(b), dev(c), dev(d), dev(off), max_len=300, sync=True)
         with pytest.raises(_lib.TridError):
             api.ragged_batch_mixed_f32(*f, dev(off), max_len=300, sync=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_understated_max_len_is_not_slow(dtype):
+    """Systems of twice the rows that max_len says are solved on the shape chosen for
+    it; they read their arrays a second time, so three times the declared call's time
+    is the bound (a solve of each lane's rows straight from memory took seven)."""
+    n, count = 4096, 4000
+    g = torch.Generator(device="cuda").manual_seed(5)
+    a, c, d = (torch.rand(n * count, dtype=dtype, device="cuda", generator=g) - 0.5
+               for _ in range(3))
+    b = 2 + a.abs() + c.abs()
+    off = torch.arange(0, (n + 1) * count, n, device="cuda")[:count + 1].contiguous()
+    best, x = {}, {}
+    for said in (n // 2, n):
+        times = []
+        for _ in range(8):
+            x[said] = d.clone()
+            ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            ev[0].record()
+            api.ragged_batch(a, b, c, x[said], off, max_len=said)
+            ev[1].record()
+            torch.cuda.synchronize()
+            times.append(ev[0].elapsed_time(ev[1]))
+        best[said] = min(times)
+    print("understated %.3f ms, declared %.3f ms" % (best[n // 2], best[n]))
+    tol = 1e-12 if dtype == torch.float64 else 1e-5
+    assert (x[n] - x[n // 2]).abs().max().item() <= tol * x[n].abs().max().item()
+    assert best[n // 2] <= 3 * best[n]

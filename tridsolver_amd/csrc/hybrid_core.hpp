@@ -660,20 +660,21 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" : : : "memory");
 }
 
-// One workgroup's contiguous systems of P lanes each (P a power of two, M rows
-// per lane): loads, transposes inside the waves, solve, transposed store. L.base,
-// L.N and L.active are the lane's system; tile: 64 * (M + 1) elements per wave.
-// FULL: P >= 64, so that every lane of a wave has the same system (scalar base
-// address). Loads are unconditional, from rows clamped into the system; the
-// identity rows past N, and a of the first and c of the last row, are set once
-// the rows are in chunk order. issued() runs once the loads are issued,
-// loaded() once they have been transposed.
-template <typename REAL, int M, bool INC, bool FULL, typename OnIssued, typename OnLoaded>
-__device__ __forceinline__ void wave_solve(const Lane &L, REAL *tile, Ring &ring,
-                                           const REAL *__restrict__ a,
-                                           const REAL *__restrict__ b,
-                                           const REAL *__restrict__ c, const REAL *d, REAL *u,
-                                           OnIssued issued, OnLoaded loaded) {
+// The rows of one workgroup's contiguous systems of P lanes each (P a power of two,
+// M rows per lane), in chunk order. L.base, L.N and L.active are the lane's system;
+// tile: 64 * (M + 1) elements per wave. FULL: P >= 64, so that every lane of a wave
+// has the same system (scalar base address). Loads are unconditional, from rows
+// clamped into the system; the identity rows past N, c of the last row and, where
+// first says that the system starts here, a of the first, are set once the rows are
+// in chunk order. issued() runs once the loads are issued, loaded() once they have
+// been transposed.
+template <typename REAL, int M, bool FULL, typename OnIssued, typename OnLoaded>
+__device__ __forceinline__ void wave_rows(const Lane &L, REAL *tile, bool first,
+                                          const REAL *__restrict__ a,
+                                          const REAL *__restrict__ b,
+                                          const REAL *__restrict__ c, const REAL *d, REAL (&ra)[M],
+                                          REAL (&rb)[M], REAL (&rc)[M], REAL (&rd)[M],
+                                          OnIssued issued, OnLoaded loaded) {
   const int P64 = FULL ? 64 : L.P, lane = L.t & 63;
   const int lp = lane & (P64 - 1);
   REAL *wt = tile + (L.t - lp) * (M + 1);  // the waves' tiles follow each other
@@ -681,7 +682,6 @@ __device__ __forceinline__ void wave_solve(const Lane &L, REAL *tile, Ring &ring
   const int N = (int)L.N;
   const int64_t base = FULL ? wave_uniform(L.base) : L.base;
   const Fetch f = fetch_rows<REAL, M, FULL>(d + base, lp);
-  REAL ra[M], rb[M], rc[M], rd[M];
   if (L.active) {
     const REAL *pa = a + base, *pb = b + base, *pc = c + base, *pd = d + base;
     auto rows_of = [&](const REAL *p, REAL (&v)[M]) {
@@ -704,7 +704,7 @@ __device__ __forceinline__ void wave_solve(const Lane &L, REAL *tile, Ring &ring
   wave_to_chunk<M, FULL>(rd, wt, lp, f, P64);
   loaded();
   const int row0 = L.p * M, rows = L.active ? N - row0 : 0;
-  if (row0 == 0) ra[0] = REAL(0);
+  if (first && row0 == 0) ra[0] = REAL(0);
   if (rows <= M) {
 #pragma unroll
     for (int r = 0; r < M; ++r) {
@@ -714,27 +714,48 @@ __device__ __forceinline__ void wave_solve(const Lane &L, REAL *tile, Ring &ring
       rd[r] = r < rows ? rd[r] : REAL(0);
     }
   }
-  REAL f_d, f_a, f_g, y, ym;
-  sweep_carry<REAL, M>([&](int r) { return ra[r]; }, rb, rc, rd, f_d, f_a, f_g);
-  reduced_solve<REAL, true>(L, ring, rb[M - 1], rc[M - 1], rd[M - 1], f_d, f_a, f_g, y, ym);
-  substitute_back<REAL, M>(rb, rc, rd, y, ym);
-  // (the tile slots and rows from here on are formed again, not held through
-  // the solve: empty asm)
-  int lq = lp;
+}
+
+// The lane's rows v in chunk order to u (INC: added), through the tile, as wave_rows
+// took them. The tile slots and rows are formed again, not held through the solve
+// (empty asm).
+template <typename REAL, int M, bool INC, bool FULL>
+__device__ __forceinline__ void wave_put(const Lane &L, REAL *tile, const REAL *d, REAL *u,
+                                         REAL (&v)[M]) {
+  const int P64 = FULL ? 64 : L.P;
+  const int64_t base = FULL ? wave_uniform(L.base) : L.base;
+  int lq = (L.t & 63) & (P64 - 1);
   asm volatile("" : "+v"(lq));
   const Fetch q = fetch_rows<REAL, M, FULL>(d + base, lq);
-  wave_to_fetch<M, FULL>(rd, tile + (L.t - lq) * (M + 1), lq, q, P64);
+  wave_to_fetch<M, FULL>(v, tile + (L.t - lq) * (M + 1), lq, q, P64);
   if (L.active) {
     REAL *dst = u + base;  // u == d for a solve in place
+    const int N = (int)L.N;
 #pragma unroll
     for (int r = 0; r < M; ++r) {
       const int row = (L.p - lq) * M + (r == 0 ? q.e0 : q.e + P64 * r);
       if (row < N) {
-        if (INC) dst[row] += rd[r];
-        else st<FULL>(&dst[row], rd[r]);
+        if (INC) dst[row] += v[r];
+        else st<FULL>(&dst[row], v[r]);
       }
     }
   }
+}
+
+// One workgroup's contiguous systems: loads, transposes inside the waves, solve,
+// transposed store (wave_rows, wave_put).
+template <typename REAL, int M, bool INC, bool FULL, typename OnIssued, typename OnLoaded>
+__device__ __forceinline__ void wave_solve(const Lane &L, REAL *tile, Ring &ring,
+                                           const REAL *__restrict__ a,
+                                           const REAL *__restrict__ b,
+                                           const REAL *__restrict__ c, const REAL *d, REAL *u,
+                                           OnIssued issued, OnLoaded loaded) {
+  REAL ra[M], rb[M], rc[M], rd[M], f_d, f_a, f_g, y, ym;
+  wave_rows<REAL, M, FULL>(L, tile, true, a, b, c, d, ra, rb, rc, rd, issued, loaded);
+  sweep_carry<REAL, M>([&](int r) { return ra[r]; }, rb, rc, rd, f_d, f_a, f_g);
+  reduced_solve<REAL, true>(L, ring, rb[M - 1], rc[M - 1], rd[M - 1], f_d, f_a, f_g, y, ym);
+  substitute_back<REAL, M>(rb, rc, rd, y, ym);
+  wave_put<REAL, M, INC, FULL>(L, tile, d, u, rd);
 }
 
 // ---- one long system in one workgroup, 32 rows per lane -----------------

@@ -311,85 +311,148 @@ __global__ __launch_bounds__(T, (rg_waves<REAL, M>())) void rg_solve(
       });
 }
 
+// Segments of RG_SMALL_T * M rows in the longest system that a shape's plan lists.
+template <typename REAL, int M>
+constexpr int rg_segments() {
+  return RgBounds<REAL, M>::threads / RG_SMALL_T;
+}
+// LDS elements of rg_item_segments behind the tile: the equations of all segments
+// but the last, and the first-row forms of the waves' first chunks.
+template <typename REAL, int M>
+constexpr int rg_segment_reals() {
+  return 3 * RG_SMALL_T * (rg_segments<REAL, M>() - 1) + 3 * (RG_SMALL_T / 64) * rg_segments<REAL, M>();
+}
+
 // A system of more rows than RG_SMALL_T lanes of M hold, in one such workgroup:
 // what is left over where the shape was chosen for a max_len that the caller
-// understated. Each lane takes q blocks of RG_ROWS consecutive rows straight from
-// memory: one pass for the reduced system, keeping the sweep's state at each
-// block's start in the tile, and a second, block by block from the end, for x.
-// It reads everything twice and uncoalesced: 9765 systems of 4096 rows, FP64, 2.16 ms
-// where max_len says 2048, 0.29 where it says 4096.
-constexpr int RG_ROWS = 8;
+// understated. Its segments of T * M rows are swept one after the other (lane t of
+// segment j has chunk j * T + t), the reduced system of all their chunks is solved
+// by PCR in LDS, and the segments are read and swept again for x. Bound by the two
+// readings: 9765 systems of 4096 rows, FP64, 0.50 ms where max_len says 2048, 0.29
+// where it says 4096 (2.16 with every lane's rows read straight from memory, 0.41 in
+// one 1024-thread workgroup per CU, which every other batch paid for).
 template <typename REAL, int M, bool INC>
-__device__ __forceinline__ void rg_item_rows(const RgMeta &cur, unsigned char *smem_raw,
-                                             const REAL *__restrict__ a,
-                                             const REAL *__restrict__ b,
-                                             const REAL *__restrict__ c, const REAL *d, REAL *u) {
-  constexpr int T = RG_SMALL_T, Q_MOST = RgBounds<REAL, M>::threads * M / (T * RG_ROWS);
-  static_assert(3 * (Q_MOST - 1) <= M + 1, "the states fit the lane's part of the tile");
-  const int t = threadIdx.x, N = __builtin_amdgcn_readfirstlane(cur.N);
-  const int q = (N + T * RG_ROWS - 1) / (T * RG_ROWS);
-  const int row0 = t * q * RG_ROWS;
+__device__ __forceinline__ void rg_item_segments(const RgMeta &cur, unsigned char *smem_raw,
+                                                 const REAL *__restrict__ a,
+                                                 const REAL *__restrict__ b,
+                                                 const REAL *__restrict__ c, const REAL *d,
+                                                 REAL *u) {
+  constexpr int T = RG_SMALL_T, ROWS = T * M, Q = rg_segments<REAL, M>();
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));  // (what is formed from it is not held across the items)
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int N = __builtin_amdgcn_readfirstlane(cur.N), nseg = (N + ROWS - 1) / ROWS;
   const int64_t base = hyb::wave_uniform(cur.base);
-  const REAL *pa = a + base, *pb = b + base, *pc = c + base, *pd = d + base;
-  REAL *dst = u + base;  // u == d in place: a lane reads and writes rows of its own only
-  REAL *state = reinterpret_cast<REAL *>(smem_raw) + t * (M + 1);
-  hyb::Ring ring{smem_raw + sizeof(REAL) * (size_t)T * (M + 1), (int)(3 * sizeof(REAL) * T), 0};
+  REAL *tile = reinterpret_cast<REAL *>(smem_raw), *eqs = tile + T * (M + 1);
+  REAL *edge = eqs + 3 * T * (Q - 1);
+  // the equations [A, C, D][T] of segment j; the last one's in the tile
+  auto block = [&](int j) { return j == nseg - 1 ? tile : eqs + 3 * T * j; };
   hyb::Lane L{};
-  L.P = T; L.W = 1; L.T = T; L.t = t; L.p = t; L.pstep = 1; L.stride = 1;
-  L.active = true; L.base = base; L.N = N;
+  L.P = T; L.W = 1; L.T = T; L.t = t; L.p = t; L.pstep = 1; L.stride = 1; L.active = true;
 
-  // one row of the sweep: al x_{s-1} + x_r + ga x_{r+1} = de
-  REAL al = -1, ga = 0, de = 0;
-  auto eliminate = [&](int row) {
-    const bool in = row < N;
-    const REAL ar = in && row > 0 ? pa[row] : REAL(0), br = in ? pb[row] : REAL(1);
-    const REAL cr = row < N - 1 ? pc[row] : REAL(0), dr = in ? pd[row] : REAL(0);
-    const REAL inv = REAL(1) / (br - ar * ga);
-    al = -ar * al * inv;
-    ga = cr * inv;
-    de = (dr - ar * de) * inv;
+  REAL rb[M], rc[M], rd[M], e[3];
+  auto sweep = [&](int j, REAL (&f)[3]) {
+    REAL ra[M];
+    L.t = t;
+    asm volatile("" : "+v"(L.t));  // (nor are the loads' addresses across the segments)
+    L.p = L.t;
+    L.base = base + (int64_t)j * ROWS;
+    L.N = N - j * ROWS;
+    hyb::wave_rows<REAL, M, true>(L, tile, j == 0, a, b, c, d, ra, rb, rc, rd, [] {}, [] {});
+    hyb::sweep_carry<REAL, M>([&](int r) { return ra[r]; }, rb, rc, rd, f[0], f[1], f[2]);
   };
-  REAL f_d = 0, f_a = 0, f_g = -1, y, ym;
-  for (int j = 0; j < q; ++j) {
-    if (j > 0) {
-      state[3 * j - 3] = al; state[3 * j - 2] = ga; state[3 * j - 1] = de;
-    }
+  // a chunk's equation from its last row (al, ga, de) and the next chunk's first row
+  // (f_d, f_a, f_g), as in hyb::reduced_solve
+  auto close = [&](REAL nd, REAL na, REAL ng) {
+    const REAL inv = REAL(1) / (REAL(1) - e[1] * na);
+    e[2] = (e[2] - e[1] * nd) * inv;
+    e[0] = e[0] * inv;
+    e[1] = -e[1] * ng * inv;
+  };
+  auto put = [&](int j) {
 #pragma unroll
-    for (int r = 0; r < RG_ROWS; ++r) {
-      eliminate(row0 + RG_ROWS * j + r);
-      if (j < q - 1 || r < RG_ROWS - 1) {
-        f_d = f_d - f_g * de;
-        f_a = f_a - f_g * al;
-        f_g = -f_g * ga;
-      }
+    for (int k = 0; k < 3; ++k) block(j)[k * T + t] = e[k];
+  };
+  for (int j = 0; j < nseg; ++j) {
+    REAL f[3], nx[3];
+    sweep(j, f);
+    e[0] = rb[M - 1]; e[1] = rc[M - 1]; e[2] = rd[M - 1];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      if ((t & 63) == 0) edge[3 * (j * (T / 64) + wv) + k] = f[k];
+      nx[k] = hyb::wave_read(f[k], (t & 63) + 1);
+    }
+    if ((t & 63) != 63) close(nx[0], nx[1], nx[2]);
+    if (j < nseg - 1) put(j);
+  }
+  hyb::lds_barrier();  // the edges are there, the tile is free
+  put(nseg - 1);
+  if ((t & 63) == 63) {
+    for (int j = 0; j < nseg; ++j) {
+      const int w = j * (T / 64) + wv + 1;  // the next wave's first chunk
+      const bool last = w == nseg * (T / 64);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) e[k] = block(j)[k * T + t];
+      close(last ? REAL(0) : edge[3 * w], last ? REAL(0) : edge[3 * w + 1],
+            last ? REAL(0) : edge[3 * w + 2]);
+      put(j);
     }
   }
-  hyb::reduced_solve<REAL, true>(L, ring, al, ga, de, f_d, f_a, f_g, y, ym);
-  REAL x = y;
-  for (int j = q - 1; j >= 0; --j) {
-    al = -1; ga = 0; de = 0;
-    if (j > 0) {
-      al = state[3 * j - 3]; ga = state[3 * j - 2]; de = state[3 * j - 1];
-    }
-    REAL ral[RG_ROWS], rga[RG_ROWS], rde[RG_ROWS];
+  hyb::lds_barrier();
+  for (int h = 1; h < nseg * T; h <<= 1) {
+    REAL v[Q][3];
 #pragma unroll
-    for (int r = 0; r < RG_ROWS; ++r) {
-      eliminate(row0 + RG_ROWS * j + r);
-      ral[r] = al; rga[r] = ga; rde[r] = de;
-    }
+    for (int j = 0; j < Q; ++j) {
+      if (j >= nseg) break;
+      const int lo = j * T + t - h, hi = j * T + t + h;
+      const REAL *own = block(j) + t, *below = block(lo >= 0 ? lo / T : 0) + lo % T;
+      const REAL *above = block(hi < nseg * T ? hi / T : 0) + hi % T;
+      REAL m[3] = {}, q[3] = {};
 #pragma unroll
-    for (int r = RG_ROWS - 1; r >= 0; --r) {
-      if (j < q - 1 || r < RG_ROWS - 1) x = rde[r] - ral[r] * ym - rga[r] * x;
-      rde[r] = x;
-    }
-#pragma unroll
-    for (int r = 0; r < RG_ROWS; ++r) {
-      const int row = row0 + RG_ROWS * j + r;
-      if (row < N) {
-        if (INC) dst[row] += rde[r];
-        else dst[row] = rde[r];
+      for (int k = 0; k < 3; ++k) {
+        if (lo >= 0) m[k] = below[k * T];
+        if (hi < nseg * T) q[k] = above[k * T];
       }
+      const REAL A = own[0], C = own[T], D = own[2 * T];
+      const REAL inv = REAL(1) / (REAL(1) - A * m[1] - C * q[0]);
+      v[j][0] = -inv * A * m[0];
+      v[j][1] = -inv * C * q[1];
+      v[j][2] = inv * (D - A * m[2] - C * q[2]);
     }
+    hyb::lds_barrier();
+#pragma unroll
+    for (int j = 0; j < Q; ++j) {
+      if (j >= nseg) break;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) block(j)[k * T + t] = v[j][k];
+    }
+    hyb::lds_barrier();
+  }
+  // x of the lane's chunks' last rows and of those before them, out of the tile's way
+  static_assert(2 * Q * T <= std::max(6 * T, rg_segment_reals<REAL, M>()), "LDS behind the tile");
+  {
+    REAL y[Q][2] = {};
+#pragma unroll
+    for (int j = 0; j < Q; ++j) {
+      if (j >= nseg) break;
+      const int k = j * T + t - 1;
+      y[j][0] = block(j)[2 * T + t];
+      if (k >= 0) y[j][1] = block(k / T)[2 * T + k % T];
+    }
+    hyb::lds_barrier();
+#pragma unroll
+    for (int j = 0; j < Q; ++j) {
+      if (j >= nseg) break;
+      eqs[2 * T * j + t] = y[j][0];
+      eqs[2 * T * j + T + t] = y[j][1];
+    }
+  }
+  for (int j = 0; j < nseg; ++j) {
+    REAL f[3];
+    sweep(j, f);
+    const REAL y = eqs[2 * T * j + t], ym = eqs[2 * T * j + T + t];
+    hyb::substitute_back<REAL, M>(rb, rc, rd, y, ym);
+    hyb::wave_put<REAL, M, INC, true>(L, tile, d, u, rd);
   }
 }
 
@@ -397,7 +460,7 @@ __device__ __forceinline__ void rg_item_rows(const RgMeta &cur, unsigned char *s
 // Tshort = RG_SMALL_T. The items [0, long_items), single systems that need more
 // lanes, come first: LONG32 (M = 16: 4097-8192 rows) takes them by
 // hyb::long32_solve, 32 rows per lane in 256 threads with `a` moved HBM->LDS in
-// chunk order; otherwise there are none but misdeclared ones (rg_item_rows). Bound by
+// chunk order; otherwise there are none but misdeclared ones (rg_item_segments). Bound by
 // HBM: with the plan's four launches (19 us), FP64, 40 M unknowns in systems of
 // 4096 rows 291 us, of 2048 (M = 8) 286; lengths of 2049-4096 at random 153 us for
 // 17.7 M unknowns, of 4097-8192 206 us for 23.6 M. What is left over the floor is
@@ -406,8 +469,10 @@ __device__ __forceinline__ void rg_item_rows(const RgMeta &cur, unsigned char *s
 // from an atomic counter: 412 and 406 us for the first two.
 template <typename REAL, int M, bool LONG32>
 constexpr size_t rg_each_lds_bytes() {
-  return LONG32 ? hyb::long32_lds_bytes<REAL>()
-                : sizeof(REAL) * (size_t)RG_SMALL_T * (M + 1) + hyb::ring_bytes<REAL>(RG_SMALL_T, 3);
+  if (LONG32) return hyb::long32_lds_bytes<REAL>();
+  // the tile, and the ring or what rg_item_segments keeps
+  return sizeof(REAL) * (size_t)RG_SMALL_T * (M + 1) +
+         std::max(hyb::ring_bytes<REAL>(RG_SMALL_T, 3), sizeof(REAL) * (size_t)rg_segment_reals<REAL, M>());
 }
 
 template <typename REAL, int M, bool INC, bool LONG32>
@@ -434,9 +499,9 @@ __global__ __launch_bounds__(RG_SMALL_T, (LONG32 ? 2 : rg_waves<REAL, M>())) voi
                                                    __builtin_amdgcn_readfirstlane(cur.N),
                                                    smem_raw, a, b, c, d, u, issued, loaded);
         } else {
+          rg_item_segments<REAL, M, INC>(cur, smem_raw, a, b, c, d, u);
           issued();
           loaded();
-          rg_item_rows<REAL, M, INC>(cur, smem_raw, a, b, c, d, u);
         }
       });
 }
