@@ -305,3 +305,38 @@ def test_sweeps_with_several_lines_per_lane(dtype, shape):
     oracle.adi(0.7, u_cpu, nx, ny, nz, 3)
     for g in got:
         H.assert_norm_close(g, u_cpu, tol=tol)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_sweeps_tune_no_shape_they_do_not_use(dtype, tmp_path):
+    """In tune-on-first-use mode a step whose sweeps take several lines per lane tunes
+    nothing; the general sweeps (rows that are no whole vectors) tune theirs."""
+    from tridsolver_amd import _lib
+    L = _lib.lib()
+
+    def tuned(shape, array):
+        assert L.tridHipAutotuneClear() == 0
+        u = adi.initial_u(*shape, dtype, "random", seed=3)
+        if array:
+            adi.step(1.0, u, adi.Workspace(*shape, dtype), sync=True)
+        else:
+            adi.run_fused(1.0, u, torch.empty_like(u), 1, shape, graph=False, sync=True)
+        path = tmp_path / "tuned.txt"
+        assert L.tridHipAutotuneSave(str(path).encode()) == 0
+        return [ln for ln in path.read_text().splitlines() if not ln.startswith("#")]
+
+    assert L.tridHipSetAutotuneMode(1) == 0
+    try:
+        for array in (False, True):
+            assert tuned((64, 20, 18), array) == []
+            assert len(tuned((33, 21, 19), array)) == 2  # y and z
+    finally:
+        L.tridHipSetAutotuneMode(0)
+        L.tridHipAutotuneClear()
+
+
+def test_grid_of_too_many_planes_is_refused():
+    """2^27 planes of two points: more work-items than a HIP grid holds."""
+    from tridsolver_amd import _lib
+    u, du = (torch.empty(2 << 27, dtype=torch.float64, device="cuda") for _ in range(2))
+    assert _lib.lib().tridAdiStepFusedD(1.0, u.data_ptr(), du.data_ptr(), 2, 1, 1 << 27) == 3

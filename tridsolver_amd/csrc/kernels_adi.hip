@@ -409,7 +409,10 @@ bool adi_vec_cfg(const REAL *d, const REAL *u, int nx, int ny, int nz, int sd, G
   cfg->W = 8 * cfg->P <= ADI_VEC_T ? 8 : 4;
   cfg->G = 8;
   cfg->V = 0;
-  return cfg->W * cfg->P <= ADI_VEC_T && (int64_t)cfg->P * cfg->M >= g->N;
+  // (HIP grids hold 2^32 work-items)
+  const int64_t blocks = (g->n0 + cfg->W * V - 1) / (cfg->W * V) * g->n1;
+  return cfg->W * cfg->P <= ADI_VEC_T && (int64_t)cfg->P * cfg->M >= g->N &&
+         blocks <= (int64_t)UINT32_MAX / (cfg->W * cfg->P);
 }
 
 template <typename REAL, int M, bool INC>
@@ -529,9 +532,20 @@ __global__ __launch_bounds__(64) void adi_xvec_kernel(int nx, int ny, int nz, in
   }
 }
 
+// Lines per lane, and workgroups (one wave each), at M rows per lane.
+template <typename REAL>
+constexpr int adi_xvec_lines(int M) {
+  return sizeof(REAL) == 8 && M == 4 ? 4 : 2;
+}
+template <typename REAL>
+int64_t adi_xvec_blocks(int M, int nx, int ny, int nz) {
+  const int lines = 64 / ((nx + M - 1) / M) * adi_xvec_lines<REAL>(M);
+  return (int64_t)((ny + lines - 1) / lines) * nz;
+}
+
 // Rows per lane of adi_xvec_kernel: 32 bytes, twice that for lines that 64 lanes
 // of 32 do not hold; 0 where it does not apply: lines of whole 16-byte vectors,
-// aligned, within a wave, arrays below 4 GiB.
+// aligned, within a wave, arrays below 4 GiB, 2^32 work-items (HIP's grids).
 template <typename REAL>
 int adi_xvec_rows(const REAL *d, const REAL *u, int nx, int ny, int nz) {
   constexpr int V = 16 / (int)sizeof(REAL);
@@ -539,14 +553,16 @@ int adi_xvec_rows(const REAL *d, const REAL *u, int nx, int ny, int nz) {
       (uint64_t)nx * (uint64_t)ny * (uint64_t)nz * sizeof(REAL) > 0xffffffffull ||
       ((reinterpret_cast<uintptr_t>(d) | reinterpret_cast<uintptr_t>(u)) & 15) != 0)
     return 0;
-  return nx > 64 * 2 * V ? 4 * V : 2 * V;
+  const int M = nx > 64 * 2 * V ? 4 * V : 2 * V;
+  return adi_xvec_blocks<REAL>(M, nx, ny, nz) <= (int64_t)UINT32_MAX / 64 ? M : 0;
 }
 
 template <typename REAL, int M, int LN>
 hipError_t launch_adi_xvec(REAL lambda, REAL *d, const REAL *u, int nx, int ny, int nz,
                            hipStream_t st) {
-  const int P = (nx + M - 1) / M, lines = 64 / P * LN;
-  const int64_t blocks = (int64_t)((ny + lines - 1) / lines) * nz;
+  static_assert(LN == adi_xvec_lines<REAL>(M), "the grid is the one that was checked");
+  const int P = (nx + M - 1) / M;
+  const int64_t blocks = adi_xvec_blocks<REAL>(M, nx, ny, nz);
   hipLaunchKernelGGL((adi_xvec_kernel<REAL, M, LN>), dim3((unsigned)blocks), dim3(64), 0, st, nx,
                      ny, nz, P, 8, lambda, d, u);
   return hipGetLastError();
@@ -668,19 +684,31 @@ tridStatus_t adi_sweep(int dev, REAL lambda, REAL *d, REAL *u, int nx, int ny, i
   bool empty = false;
   tridStatus_t s = make_geom(3, sd, dims, dims, &g, &empty);
   if (s != TRID_STATUS_SUCCESS || empty) return s;
-  HybridCfg cfg;
-  if (!adi_sweep_cfg<REAL, INC>(dev, g, sd, &cfg)) return TRID_STATUS_INVALID_VALUE;
   AdiCoef<REAL> kc{lambda, nx, ny, nz, sd};
   hipStream_t st = current_stream();
   const bool contig = sd == 0;
   hipError_t e;
   if (RHS && !contig) return TRID_STATUS_INTERNAL_ERROR;
+  // the kernels with several lines per lane choose their own shape; only the general
+  // sweep behind them asks for a tuned one
   if constexpr (RHS) {
-    constexpr int M = 32 / (int)sizeof(REAL), LN = sizeof(REAL) == 8 ? 4 : 2;
+    constexpr int M = 32 / (int)sizeof(REAL), LN = adi_xvec_lines<REAL>(M);
     const int rows = adi_xvec_rows<REAL>(d, u, nx, ny, nz);
     if (rows != 0) {
       e = rows == M ? launch_adi_xvec<REAL, M, LN>(lambda, d, u, nx, ny, nz, st)
-                    : launch_adi_xvec<REAL, 2 * M, 2>(lambda, d, u, nx, ny, nz, st);
+                    : launch_adi_xvec<REAL, 2 * M, adi_xvec_lines<REAL>(2 * M)>(lambda, d, u, nx, ny, nz, st);
+      if (e != hipSuccess) {
+        record_hip_error(e);
+        return TRID_STATUS_EXECUTION_FAILED;
+      }
+      return TRID_STATUS_SUCCESS;
+    }
+  } else {
+    Geom vg;
+    HybridCfg vc;
+    if (!contig && adi_vec_cfg<REAL>(d, INC ? u : d, nx, ny, nz, sd, &vg, &vc)) {
+      e = vc.M == 16 ? launch_adi_vec<REAL, 16, INC>(vg, vc, lambda, d, u, st)
+                     : launch_adi_vec<REAL, 8, INC>(vg, vc, lambda, d, u, st);
       if (e != hipSuccess) {
         record_hip_error(e);
         return TRID_STATUS_EXECUTION_FAILED;
@@ -688,6 +716,8 @@ tridStatus_t adi_sweep(int dev, REAL lambda, REAL *d, REAL *u, int nx, int ny, i
       return TRID_STATUS_SUCCESS;
     }
   }
+  HybridCfg cfg;
+  if (!adi_sweep_cfg<REAL, INC>(dev, g, sd, &cfg)) return TRID_STATUS_INVALID_VALUE;
   // The right-hand side is computed in the sweep unless FP32 x lines are
   // at 16 rows per lane (they would spill) or the grid is 4 GiB or more (the
   // sweep's loads use 32-bit byte offsets): there preproc writes du and the
@@ -700,19 +730,6 @@ tridStatus_t adi_sweep(int dev, REAL lambda, REAL *d, REAL *u, int nx, int ny, i
     tridStatus_t sp = preproc<REAL>(lambda, u, d, nullptr, nullptr, nullptr, nullptr, nullptr,
                                     nullptr, nullptr, nullptr, nullptr, nx, ny, nz);
     if (sp != TRID_STATUS_SUCCESS) return sp;
-  }
-  if constexpr (!RHS) {
-    Geom vg;
-    HybridCfg vc;
-    if (!contig && adi_vec_cfg<REAL>(d, INC ? u : d, nx, ny, nz, sd, &vg, &vc)) {
-      e = vc.M == 16 ? launch_adi_vec<REAL, 16, INC>(vg, vc, lambda, d, u, st)
-                     : launch_adi_vec<REAL, 8, INC>(vg, vc, lambda, d, u, st);
-      if (e != hipSuccess) {
-        record_hip_error(e);
-        return TRID_STATUS_EXECUTION_FAILED;
-      }
-      return TRID_STATUS_SUCCESS;
-    }
   }
 #define TRID_ADI_CASE(MM)                                                                  \
   case MM:                                                                                 \
@@ -863,6 +880,11 @@ bool array_step_matrix_free(const TridParams *ctx, const REAL *u, const REAL *du
     HybridCfg cfg;
     bool empty = false;
     if (make_geom(3, sd, dims, dims, &g, &empty) != TRID_STATUS_SUCCESS || empty) return false;
+    // (as adi_sweep chooses)
+    Geom vg;
+    if (sd == 0 ? adi_xvec_rows<REAL>(du, u, nx, ny, nz) != 0
+                : adi_vec_cfg<REAL>(du, sd == 2 ? u : du, nx, ny, nz, sd, &vg, &cfg))
+      continue;
     const bool ok = sd == 2 ? adi_sweep_cfg<REAL, true>(dev, g, sd, &cfg)
                             : adi_sweep_cfg<REAL, false>(dev, g, sd, &cfg);
     if (!ok) return false;
