@@ -340,3 +340,65 @@ def test_grid_of_too_many_planes_is_refused():
     from tridsolver_amd import _lib
     u, du = (torch.empty(2 << 27, dtype=torch.float64, device="cuda") for _ in range(2))
     assert _lib.lib().tridAdiStepFusedD(1.0, u.data_ptr(), du.data_ptr(), 2, 1, 1 << 27) == 3
+
+
+# --- steps that keep preproc and the array solves -----------------------------
+# A step whose solves the caller chooses, or with a line that no workgroup holds, is
+# captured and replayed; default steps are matrix-free launches with and without
+# a graph, and agree with these to rounding.
+
+def _replayed_and_launched(dtype, shape, iters, seed):
+    """u after `iters` steps, work of its own, and `iters` more, replayed and launched;
+    and the same by the matrix-free call on the same field."""
+    u0 = adi.initial_u(*shape, dtype, "random", seed=seed)
+    got = []
+    for graph in (True, False):
+        u, ws = u0.clone(), adi.Workspace(*shape, dtype)
+        for _ in range(3):
+            adi.run(0.8, u, ws, iters, graph=graph, sync=True)
+            u.mul_(0.75)
+            torch.cuda.synchronize()
+        got.append((u, ws.du.clone()))
+    return u0, got
+
+
+def _assert_adi_oracle(u0, u, shape, iters, dtype):
+    want = _np(u0).copy()
+    for _ in range(3):
+        oracle.adi(0.8, want, *shape, iters)
+        want *= want.dtype.type(0.75)
+    H.assert_norm_close(_np(u), want, tol=1e-12 if dtype == torch.float64 else 1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("shape,cfg", [((40, 36, 32), (4, 10, 8)), ((64, 33, 47), (8, 8, 8)),
+                                       ((30, 100, 21), (16, 7, 4))])
+def test_replayed_hybrid_steps_equal_launched(dtype, shape, cfg):
+    """A forced hybrid shape (M, P, W) that holds all three directions: the captured
+    and replayed steps equal the launched ones bit for bit, and the matrix-free steps
+    and the oracle to rounding."""
+    from tridsolver_amd import api
+    with api.forced_hybrid(*cfg):
+        u0, ((ug, dg), (ul, dl)) = _replayed_and_launched(dtype, shape, 3, 31)
+        assert api.last_config() == (3, *cfg, 8)  # the z solve's
+    assert torch.equal(ug, ul) and torch.equal(dg, dl)
+    _assert_adi_oracle(u0, ug, shape, 3, dtype)
+    uf, ws = u0.clone(), adi.Workspace(*shape, dtype)
+    for _ in range(3):
+        adi.run(0.8, uf, ws, 3, graph=False, sync=True)
+        uf.mul_(0.75)
+    tol = 1e-12 if dtype == torch.float64 else 1e-5
+    assert not torch.equal(uf, ug)  # another path indeed
+    H.assert_norm_close(_np(uf), _np(ug), tol=tol)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_replayed_steps_with_a_long_line(dtype):
+    """A z line longer than a workgroup holds: its solve needs a workspace, which the
+    captured run reserves for the capture stream."""
+    from tridsolver_amd import api
+    shape = (7, 3, 8200)
+    u0, ((ug, dg), (ul, dl)) = _replayed_and_launched(dtype, shape, 2, 32)
+    assert api.last_config()[0] == 12
+    assert torch.equal(ug, ul) and torch.equal(dg, dl)
+    _assert_adi_oracle(u0, ug, shape, 2, dtype)
