@@ -240,6 +240,33 @@ def test_solve_to_equals_solve_in_place(dims, sd, force, dtype):
     assert bool((x == 7.0).all())
 
 
+@pytest.mark.parametrize("dims,sd,dtype,seg", [
+    # one 128-byte segment per line: 256-byte groups would be half empty
+    ([16, 500, 400], 1, np.float64, 128), ([11, 64, 384], 1, np.float64, 128),
+    ([16, 400, 256], 2, np.float64, 128), ([32, 300, 1024], 1, np.float32, 128),
+    ([16, 32, 400], 1, np.float64, 256),  # short systems: half the lanes at 128 bytes
+    # three: the same; two: whole 256-byte segments
+    ([40, 200, 192], 1, np.float64, 128), ([96, 300, 520], 1, np.float32, 128),
+    ([32, 200, 384], 1, np.float64, 256), ([64, 300, 1030], 1, np.float32, 256),
+    # five and more: by the systems' length, until the empty half is small
+    ([80, 320, 128], 1, np.float64, 256), ([80, 321, 128], 1, np.float64, 128),
+    ([144, 384, 342], 1, np.float32, 128), ([144, 385, 342], 1, np.float32, 256),
+    ([400, 400, 31], 1, np.float64, 256), ([368, 400, 33], 1, np.float64, 128),
+    ([288, 300, 206], 1, np.float32, 256)])
+def test_rows_of_lines_that_end_in_half_a_segment(dims, sd, dtype, seg):
+    """Strided batches whose lines are an odd number of 128-byte segments: the row
+    width of the default shape, and the results of the smaller ones."""
+    n = int(np.prod(dims))
+    if n <= 4000000:
+        cfg = run_case(dims, sd, dtype, False, (0, 0, 0), seed=sum(dims))
+    else:
+        t = torch.float64 if dtype == np.float64 else torch.float32
+        a, c, d = (torch.rand(n, dtype=t, device="cuda") - 0.5 for _ in range(3))
+        api.trid_strided_batch(a, 2 + a.abs() + c.abs(), c, d, solvedim=sd, dims=dims, sync=True)
+        cfg = api.last_config()
+    assert cfg[0] == 8 and cfg[3] * np.dtype(dtype).itemsize == seg, cfg
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("inc", [False, True])
 @pytest.mark.parametrize("dims,sd,seg", [
