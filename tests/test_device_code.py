@@ -139,3 +139,19 @@ def test_staging_compiles_without_warnings(tmp_path):
                        capture_output=True, text=True)
     assert r.returncode == 0 and "warning:" not in r.stderr, r.stderr[:2000]
     assert "-Werror" in B.CFLAGS
+
+
+def test_registers_of_the_largest_fp32_workgroups(tmp_path):
+    """The strided FP32 kernel at 16 rows of 128 bytes runs up to 1024 threads; two such
+    workgroups share a CU only at 64 VGPRs or fewer."""
+    lib = shutil.copy(_lib.LIBPATH, tmp_path)
+    subprocess.run([OBJDUMP, "--offloading", os.path.basename(lib)], cwd=tmp_path, check=True,
+                   capture_output=True)
+    found = {}
+    for obj in glob.glob(str(tmp_path / "*gfx950")):
+        notes = subprocess.run([os.path.join(os.path.dirname(OBJDUMP), "llvm-readelf"), "--notes",
+                                obj], check=True, capture_output=True, text=True).stdout
+        for name, vgprs in re.findall(r"\.symbol: +(\S+)\.kd.*?\.vgpr_count: +(\d+)", notes, re.S):
+            if "hybrid_wide_kernelIfLi16ELi128E" in name:
+                found[name] = int(vgprs)
+    assert len(found) == 4 and max(found.values()) <= 64, found

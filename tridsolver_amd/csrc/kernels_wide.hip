@@ -44,8 +44,17 @@ namespace {
 
 using namespace wide;
 
+// Waves per SIMD that the registers are held to: at FP32, 16 rows of 128 bytes, two of
+// the largest workgroups (1024 threads) share a CU at 64 VGPRs, which the compiler
+// exceeds by two without the bound (32 x 500 x 2048 y 101 against 120 us).
+template <typename REAL, int M, int SEG>
+constexpr int wide_waves() {
+  return sizeof(REAL) == 4 && M == 16 && SEG == 128 ? 8 : 1;
+}
+
 template <typename REAL, int M, int SEG, bool INC, bool NT>
-__global__ __launch_bounds__((WideBounds<REAL, M>::threads)) void hybrid_wide_kernel(
+__global__ __launch_bounds__((WideBounds<REAL, M>::threads), (wide_waves<REAL, M, SEG>()))
+void hybrid_wide_kernel(
     Geom g, int P, int G, int slots, const REAL *__restrict__ a, const REAL *__restrict__ b,
     const REAL *__restrict__ c, const REAL *d, REAL *u) {
   constexpr int W = WideShape<REAL, SEG>::W;
@@ -85,21 +94,23 @@ __global__ __launch_bounds__((WideBounds<REAL, M>::threads)) void hybrid_wide_ke
   // (iii)
   REAL y, ym;
   hyb::reduced_solve<REAL>(L, ring, rb[M - 1], rc[M - 1], rd[M - 1], f_d, f_a, f_g, y, ym);
-  if (!L.active) return;
-  // (iv)
+  // (iv). The lane's rows and offsets are formed here again from a thread index that
+  // the compiler cannot match with the first (empty asm), so that none of them is held
+  // in registers across the whole kernel.
+  int ts = L.t;
+  asm volatile("" : "+v"(ts));
+  const int p = ts / W, w = ts % W;
+  if (w >= nsys) return;
   if (INC) hyb::stage_wait_all();
   hyb::substitute_back<REAL, M>(rb, rc, rd, y, ym);
-  // The store offsets are recomputed here (the empty asm hides that they
-  // equal the load offsets, which would otherwise be kept live in registers
-  // across the whole kernel).
-  uint32_t obs = ob;
-  asm volatile("" : "+v"(obs));
+  const uint32_t obs = (uint32_t)(base0 + w + (int64_t)p * M * L.stride) * (uint32_t)sizeof(REAL);
+  const REAL *us = reinterpret_cast<REAL *>(smem_raw + p * PITCH) + w;
   char *dst = reinterpret_cast<char *>(u);  // u == d for a solve in place
 #pragma unroll
   for (int r = 0; r < M; ++r) {
-    if (r < rows) {
+    if (p * M + r < N) {
       REAL *q = reinterpret_cast<REAL *>(dst + obs + (uint32_t)r * os);
-      if (INC) hyb::st<NT>(q, as[r * W] + rd[r]);
+      if (INC) hyb::st<NT>(q, us[r * W] + rd[r]);
       else hyb::st<NT>(q, rd[r]);
     }
   }
