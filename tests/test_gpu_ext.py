@@ -1050,3 +1050,22 @@ def test_ragged_mixed_rejects():
         api.ragged_batch_mixed(dev(a.astype(np.float32)), dev(b.astype(np.float32)),
                                dev(c.astype(np.float32)), dev(d.astype(np.float32)), dev(off),
                                max_len=4096)
+
+
+def _adjoint_config(dims, sd, dtype, grads):
+    """The shape an untuned adjoint of the batch takes, on random operands."""
+    n = int(np.prod(dims))
+    t = torch.float64 if dtype == np.float64 else torch.float32
+    a, c, x, w = (torch.rand(n, dtype=t, device="cuda") - 0.5 for _ in range(4))
+    g = dict(grad_a=True, grad_b=True, grad_c=True) if grads else {}
+    api.adjoint_strided_batch(a, 2 + a.abs() + c.abs(), c, x if grads else None, w, solvedim=sd,
+                              dims=dims, sync=True, **g)
+    return api.last_config()
+
+
+@pytest.mark.parametrize("dims,seg", [([32, 128, 400], 128), ([96, 200, 200], 128),
+                                      ([64, 128, 400], 256), ([288, 128, 100], 256)])
+def test_adjoint_rows_of_lines_that_end_in_half_a_segment(dims, seg):
+    """The FP32 adjoint's 256-byte rows: not where they leave half of a group empty."""
+    cfg = _adjoint_config(dims, 1, np.float32, True)
+    assert cfg[0] == 4 and cfg[3] * 4 == seg, cfg

@@ -379,7 +379,8 @@ bool adjoint_default_cfg(const Geom &g, HybridCfg *cfg) {
   // the next valid one.
   HybridCfg c;
   if (hybrid_wide_default_cfg<REAL>(g, &c) && adjoint_wide<REAL>(g, c)) {
-    if (sizeof(REAL) == 4 && g.N <= 512 && wide::wide_many_groups<REAL>(g)) {
+    if (sizeof(REAL) == 4 && g.N <= 512 && wide::wide_many_groups<REAL>(g) &&
+        wide::wide_whole_segments<REAL>(g)) {
       // nine streams of 128-byte rows want more bytes per row than the
       // solve's five: 256-byte rows at every length (256^3 FP32 y / z 108 /
       // 113 against 114 / 127 us, 203 x 170 x 300 z 117 against 128)

@@ -365,15 +365,8 @@ bool hybrid_wide_default_cfg(const Geom &g, HybridCfg *cfg) {
   //  - rows of 256 bytes where such a workgroup holds the system (N <= 512)
   //    and there are enough of them (wide_many_groups): fewer row segments
   //    and fewer misaligned edges per byte (FP64 777 x 300 x 250 y 504 against
-  //    532 us, 256^3 z 127 against 155). 128-byte rows otherwise, and where lines
-  //    are an odd number of 128-byte segments, so that the last 256-byte group of a
-  //    line is half empty, and that counts: lines of one or three, and of up to 23 with
-  //    systems whose 256-byte group fills a CU (FP64, 256 against 128 bytes: 16 x 500
-  //    x 1100 y 93 against 61 us, 48 x 400 x 550 y 92 against 72, 104 x 500 x 275 y 153 against
-  //    128; 130 x 100 x 280 z the other way, 37 against 46; FP32: 32 x 300 x 1100 y 62 against
-  //    42, 224 x 300 x 275 y 79 against 69, 288 x 500 x 220 y 110 against 122). FP64
-  //    systems of up to 32 rows leave half the lanes of a 128-byte group idle
-  //    as well (16 x 32 x 1100 y 8.3 against 8.8): 256.
+  //    532 us, 256^3 z 127 against 155). 128-byte rows otherwise, and where
+  //    256-byte ones would leave too many systems out (wide_whole_segments).
   //  - FP64 at 16 rows per lane (512^3 z 0.94 against 0.95 ms at 32, 251 x
   //    300 x 300 y 213 against 222 us). FP32 at 32 rows per lane on 256-byte
   //    rows of 257-512 (512^3 y 0.466 against 0.484 ms for 16 on 128-byte
@@ -388,11 +381,7 @@ bool hybrid_wide_default_cfg(const Geom &g, HybridCfg *cfg) {
   HybridCfg c;
   const bool fp64 = sizeof(REAL) == 8;
   const int64_t row_bytes = g.stride * (int64_t)sizeof(REAL);
-  const int64_t segs = (g.n0 * (int64_t)sizeof(REAL) + 127) / 128;
-  const bool whole = segs % 2 == 0 ||
-                     (fp64 ? g.N <= 32 || segs >= 25 || (segs >= 5 && g.N <= 320)
-                           : segs >= 9 || (segs >= 5 && g.N > 384));
-  const bool wide = g.N <= 512 && whole &&
+  const bool wide = g.N <= 512 && wide::wide_whole_segments<REAL>(g) &&
                     (fp64 ? wide::wide_many_groups<REAL>(g)
                           : g.N > 256 && wide::wide_many_groups<REAL>(g, 1024));
   c.M = fp64 || (!wide && g.N <= 512) ? 16 : 32;

@@ -153,6 +153,22 @@ bool wide_many_groups(const Geom &g, int64_t least = 384) {
   return (g.n0 * (int64_t)sizeof(REAL) + 255) / 256 * g.n1 >= least;
 }
 
+// Whether 256-byte rows suit the lines: not where a line is an odd number of 128-byte
+// segments, so that its last 256-byte group is half empty, and that counts: lines of
+// one or three, and of up to 23 with systems whose 256-byte group fills a CU (256
+// against 128 bytes, FP64: 16 x 500 x 1100 y 93 against 61 us, 48 x 400 x 550 y 92 against 72,
+// 104 x 500 x 275 y 153 against 128; 130 x 100 x 280 z the other way, 37 against 46; FP32:
+// 32 x 300 x 1100 y 62 against 42, 224 x 300 x 275 y 79 against 69, 288 x 500 x 220 y 110
+// against 122). FP64 systems of up to 32 rows leave half the lanes of a 128-byte group
+// idle as well (16 x 32 x 1100 y 8.3 against 8.8).
+template <typename REAL>
+bool wide_whole_segments(const Geom &g) {
+  const int64_t segs = (g.n0 * (int64_t)sizeof(REAL) + 127) / 128;
+  if (segs % 2 == 0) return true;
+  if (sizeof(REAL) == 8) return g.N <= 32 || segs >= 25 || (segs >= 5 && g.N <= 320);
+  return segs >= 9 || (segs >= 5 && g.N > 384);
+}
+
 // Whether every row of the batch starts on a 128-byte line, with `low` the
 // arrays' addresses or-ed together. Kernels take nontemporal access then, and
 // plain access where rows are misaligned: a workgroup's segments share lines
