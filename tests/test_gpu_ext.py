@@ -1069,3 +1069,16 @@ def test_adjoint_rows_of_lines_that_end_in_half_a_segment(dims, seg):
     """The FP32 adjoint's 256-byte rows: not where they leave half of a group empty."""
     cfg = _adjoint_config(dims, 1, np.float32, True)
     assert cfg[0] == 4 and cfg[3] * 4 == seg, cfg
+
+
+@pytest.mark.parametrize("dims,dtype,grads,plain", [
+    ([16, 16, 384], np.float64, True, True), ([16, 40, 384], np.float64, False, True),
+    ([16, 40, 513], np.float64, False, False), ([22, 31, 110], np.float64, True, True),
+    ([16, 600, 96], np.float64, True, True), ([16, 600, 97], np.float64, True, False),
+    ([32, 46, 500], np.float32, True, True), ([32, 900, 40], np.float32, True, False)])
+def test_adjoint_of_few_systems(dims, dtype, grads, plain):
+    """Few strided systems take the kernel without staging, at its fewer rows per lane
+    or narrower rows; more take the wide one (16 or 32 rows, 128 bytes or more)."""
+    cfg = _adjoint_config(dims, 1, dtype, grads)
+    wide = cfg[1] in (16, 32) and cfg[3] * np.dtype(dtype).itemsize >= 128
+    assert cfg[0] == 4 and wide != plain, cfg

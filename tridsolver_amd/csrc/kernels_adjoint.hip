@@ -372,13 +372,38 @@ bool adjoint_cfg_valid(const Geom &g, const HybridCfg &c) {
   return lds <= 160 * 1024;
 }
 
+// The most 128-byte rows of strided systems that adjoint_kernel solves: with few
+// groups the chip is idle either way and what counts is one workgroup's time, which
+// the wide kernel's staged tile, whole waves and serial outputs lengthen; it pays once
+// workgroups follow each other on a CU. More so where the system fills its waves
+// (N a multiple of 64 rows in FP64, 32 in FP32, at 16 rows per lane), less so on
+// short systems. adjoint_kernel against the wide one, us, on lines of one group: FP64,
+// all gradients, 16 rows, 512 groups 5.0 / 9.5; 96 rows, 512 groups 10.1 / 12.0, 1024
+// 20.8 / 19.3; 64 rows, 256 groups 6.6 / 7.3, 512 10.6 / 7.8; 400 rows, 256 groups 21.3 /
+// 23.2, 512 56 / 49; 1000 rows, 64 groups 22.3 / 28.2, 128 39.6 / 34.7; lambda alone, 64 rows
+// 5.8 / 5.0 at 256 groups, 1000 rows 23.2 / 24.4 at 128, 32.3 / 24.5 at 192. FP32, all
+// gradients, 40 rows, 512 groups 7.9 / 8.5, 768 11.6 / 9.1; 800 rows, 32 groups 20.2 / 22.7,
+// 64 32.8 / 27.8.
 template <typename REAL>
-bool adjoint_default_cfg(const Geom &g, HybridCfg *cfg) {
-  // Strided systems: the forward solve's wide shape. Otherwise the same shapes
-  // as the forward solve where they fit the adjoint's register budget, else
-  // the next valid one.
+static int64_t adjoint_plain_most(int64_t N, bool grads) {
+  const bool fp64 = sizeof(REAL) == 8, whole = N % (fp64 ? 64 : 32) == 0;
+  if (N <= 16) return fp64 ? INT64_MAX : 16384 / N;
+  if (N > 512) return fp64 ? (grads ? 96 : 128) : grads ? 32 : 64;
+  if (N > 256) return fp64 ? (whole ? 0 : 256) : grads ? 96 : 128;
+  if (whole) return !grads ? 0 : N <= 96 ? 256 : N <= 192 ? 192 : fp64 ? 0 : 128;
+  if (!grads) return fp64 && N < 64 ? 512 : 256;
+  return N < 64 && fp64 ? 1024 : fp64 || N < 96 ? 512 : 384;
+}
+
+template <typename REAL>
+bool adjoint_default_cfg(const Geom &g, bool grads, HybridCfg *cfg) {
+  // Strided systems: the forward solve's wide shape, unless they are few
+  // (adjoint_plain_most). Otherwise the same shapes as the forward solve where
+  // they fit the adjoint's register budget, else the next valid one.
   HybridCfg c;
-  if (hybrid_wide_default_cfg<REAL>(g, &c) && adjoint_wide<REAL>(g, c)) {
+  const int64_t rows = (g.n0 * g.n1 * (int64_t)sizeof(REAL) + 127) / 128;
+  if (g.stride != 1 && rows > adjoint_plain_most<REAL>(g.N, grads) &&
+      hybrid_wide_default_cfg<REAL>(g, &c) && adjoint_wide<REAL>(g, c)) {
     if (sizeof(REAL) == 4 && g.N <= 512 && wide::wide_many_groups<REAL>(g) &&
         wide::wide_whole_segments<REAL>(g)) {
       // nine streams of 128-byte rows want more bytes per row than the
@@ -459,8 +484,8 @@ hipError_t launch_adjoint(const Geom &g, const HybridCfg &cfg, const REAL *a, co
 
 template bool adjoint_cfg_valid<float>(const Geom &, const HybridCfg &);
 template bool adjoint_cfg_valid<double>(const Geom &, const HybridCfg &);
-template bool adjoint_default_cfg<float>(const Geom &, HybridCfg *);
-template bool adjoint_default_cfg<double>(const Geom &, HybridCfg *);
+template bool adjoint_default_cfg<float>(const Geom &, bool, HybridCfg *);
+template bool adjoint_default_cfg<double>(const Geom &, bool, HybridCfg *);
 template hipError_t launch_adjoint<float>(const Geom &, const HybridCfg &, const float *,
                                           const float *, const float *, const float *,
                                           const float *, float *, float *, float *, float *,

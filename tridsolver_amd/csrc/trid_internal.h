@@ -147,7 +147,7 @@ hipError_t launch_mixed32_promote(const Geom &g, const float *a, const float *b,
 template <typename REAL>
 bool adjoint_cfg_valid(const Geom &g, const HybridCfg &c);
 template <typename REAL>
-bool adjoint_default_cfg(const Geom &g, HybridCfg *cfg);
+bool adjoint_default_cfg(const Geom &g, bool grads, HybridCfg *cfg);
 template <typename REAL>
 hipError_t launch_adjoint(const Geom &g, const HybridCfg &cfg, const REAL *a, const REAL *b,
                           const REAL *c, const REAL *x, const REAL *w, REAL *lam, REAL *ga,

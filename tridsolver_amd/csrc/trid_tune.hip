@@ -513,7 +513,7 @@ tridStatus_t tune_adjoint(int dev, const Geom &g, bool grads, Choice *best) {
     // no adjoint kernel shape holds these systems: the call takes the
     // transposed batched solve, nothing to tune (algo 14, no time)
     HybridCfg any;
-    if (!adjoint_default_cfg<REAL>(g, &any)) {
+    if (!adjoint_default_cfg<REAL>(g, grads, &any)) {
       best->algo = 14;
       best->ms = 0.0f;
       return TRID_STATUS_SUCCESS;
@@ -610,7 +610,7 @@ bool adjoint_tuned_config(int dev, const Geom &g, bool grads, HybridCfg *cfg) {
     *cfg = c.cfg;
     return true;
   }
-  return adjoint_default_cfg<REAL>(g, cfg);
+  return adjoint_default_cfg<REAL>(g, grads, cfg);
 }
 
 template <typename REAL>
