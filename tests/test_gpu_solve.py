@@ -240,6 +240,17 @@ def test_solve_to_equals_solve_in_place(dims, sd, force, dtype):
     assert bool((x == 7.0).all())
 
 
+@pytest.mark.parametrize("N,systems,dtype,M", [
+    (40, 2048, np.float64, 1), (40, 8192, np.float64, 4), (128, 64, np.float64, 2),
+    (129, 64, np.float64, 8), (8, 16384, np.float64, 1), (7, 16384, np.float64, 2),
+    (100, 2000, np.float32, 2), (100, 2001, np.float32, 4), (64, 1024, np.float32, 1)])
+@pytest.mark.parametrize("inc", [False, True])
+def test_small_contiguous_batches(N, systems, dtype, M, inc):
+    """Contiguous batches too small to fill the chip take the fewest rows per lane."""
+    cfg = run_case([N, systems], 0, dtype, inc, (0, 0, 0), seed=N + systems)
+    assert cfg[:2] == (3, M), cfg
+
+
 @pytest.mark.parametrize("dims,sd,dtype,seg", [
     # one 128-byte segment per line: 256-byte groups would be half empty
     ([16, 500, 400], 1, np.float64, 128), ([11, 64, 384], 1, np.float64, 128),

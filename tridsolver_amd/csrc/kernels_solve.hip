@@ -301,6 +301,22 @@ bool hybrid_cfg_valid(const Geom &g, const HybridCfg &cfg) {
   return lds <= 160 * 1024;
 }
 
+// Contiguous systems at the fewest rows per lane that keep a system in one wave (16
+// beyond), in workgroups of about 256 threads.
+template <typename REAL>
+bool hybrid_fewest_rows_cfg(const Geom &g, HybridCfg *cfg) {
+  for (int M : {1, 2, 4, 8, 16}) {
+    const int64_t P = (g.N + M - 1) / M;
+    if (P > 64 && M < 16) continue;
+    HybridCfg c;
+    c.M = M;
+    c.P = (int)P;
+    c.W = (int)std::max<int64_t>(1, 256 / P);
+    if (hybrid_cfg_valid<REAL>(g, c)) { *cfg = c; return true; }
+  }
+  return false;
+}
+
 template <typename REAL>
 bool hybrid_plain_cfg(const Geom &g, HybridCfg *cfg) {
   const bool contig = g.stride == 1;
@@ -423,6 +439,13 @@ bool hybrid_default_cfg(const Geom &g, HybridCfg *cfg) {
       return true;
     }
   }
+  // Contiguous batches too small to fill the chip: fewer rows per lane, whose shorter
+  // chains count there (us at the fewest rows / at hybrid_plain_cfg's: FP64 40 x 2048
+  // 5.9 / 7.4, 4096 6.7 / 7.7, 8192 8.7 / 8.5; 128 x 1024 6.4 / 6.7, 2048 7.5 / 6.9; 8 x 16384
+  // 4.4 / 5.5; FP32 12 x 8192 4.7 / 5.3, 100 x 2048 5.7 / 6.2, 64 x 4096 5.6 / 4.6).
+  if (g.stride == 1 && g.N >= 8 && g.N <= 128 && g.N * g.nsys() <= 200000 &&
+      hybrid_fewest_rows_cfg<REAL>(g, cfg))
+    return true;
   return hybrid_plain_cfg<REAL>(g, cfg);
 }
 
@@ -477,6 +500,7 @@ hipError_t launch_hybrid(const Geom &g, const HybridCfg &cfg, const REAL *a,
   template bool hybrid_cfg_valid<REAL>(const Geom &, const HybridCfg &);         \
   template bool hybrid_default_cfg<REAL>(const Geom &, HybridCfg *);               \
   template bool hybrid_wide_default_cfg<REAL>(const Geom &, HybridCfg *);          \
+  template bool hybrid_fewest_rows_cfg<REAL>(const Geom &, HybridCfg *);           \
   template bool hybrid_plain_cfg<REAL>(const Geom &, HybridCfg *);
 
 TRID_INST(float)

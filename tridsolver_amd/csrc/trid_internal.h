@@ -263,6 +263,9 @@ bool hybrid_default_cfg(const Geom &g, HybridCfg *cfg);
 // The wide variant's part of it (strided systems), also the strided adjoint's shape.
 template <typename REAL>
 bool hybrid_wide_default_cfg(const Geom &g, HybridCfg *cfg);
+// Contiguous systems at the fewest rows per lane that keep a system in one wave.
+template <typename REAL>
+bool hybrid_fewest_rows_cfg(const Geom &g, HybridCfg *cfg);
 // The default among plain-kernel shapes only (V = 0).
 template <typename REAL>
 bool hybrid_plain_cfg(const Geom &g, HybridCfg *cfg);
