@@ -1071,6 +1071,24 @@ def test_adjoint_rows_of_lines_that_end_in_half_a_segment(dims, seg):
     assert cfg[0] == 4 and cfg[3] * 4 == seg, cfg
 
 
+@pytest.mark.parametrize("N,systems,dtype,grads,M", [
+    (16, 70000, np.float32, True, 1), (12, 65536, np.float32, True, 1),
+    (12, 16384, np.float32, True, 4), (80, 32768, np.float32, True, 2),
+    (80, 8192, np.float32, True, 4), (64, 1024, np.float32, True, 1),
+    (64, 8192, np.float32, True, 4), (8, 512, np.float32, False, 1),
+    (16, 512, np.float32, False, 4), (16, 65536, np.float64, True, 1),
+    (16, 16384, np.float64, True, 2), (16, 65536, np.float64, False, 2)])
+def test_adjoint_of_short_contiguous_systems(N, systems, dtype, grads, M):
+    """Rows per lane of short contiguous systems, on both sides of the rule's lines."""
+    cfg = _adjoint_config([N, systems], 0, dtype, grads)
+    assert cfg[:2] == (4, M), cfg
+
+
+def test_adjoint_of_a_few_longer_contiguous_systems():
+    assert _adjoint_config([1000, 256], 0, np.float64, True) == (4, 8, 125, 1, 1)
+    assert _adjoint_config([1000, 257], 0, np.float64, True)[3] == 2
+
+
 @pytest.mark.parametrize("dims,dtype,grads,plain", [
     ([16, 16, 384], np.float64, True, True), ([16, 40, 384], np.float64, False, True),
     ([16, 40, 513], np.float64, False, False), ([22, 31, 110], np.float64, True, True),

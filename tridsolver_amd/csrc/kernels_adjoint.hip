@@ -395,6 +395,22 @@ static int64_t adjoint_plain_most(int64_t N, bool grads) {
   return N < 64 && fp64 ? 1024 : fp64 || N < 96 ? 512 : 384;
 }
 
+// Whether contiguous systems take the fewest rows per lane that keep a system in one
+// wave (hybrid_fewest_rows_cfg). At more rows a wave's accesses spread over more lines
+// each, which nine streams feel on short systems: us at the fewest rows / at the
+// solve's shape, all gradients, FP32: 8 x 262144 21 / 41, 16 x 65536 13 / 17, 24 x 65536 21 /
+// 25, 24 x 16384 7.9 / 7.4, 100 x 65536 58 / 64, 100 x 8192 10.7 / 9.2, 64 x 2048 5.5 / 5.9, 64 x
+// 4096 6.6 / 6.1; FP64: 16 x 65536 17.9 / 19.7, 16 x 16384 7.9 / 6.8. lambda alone, FP32, 8 x
+// 16384 4.1 / 4.6.
+template <typename REAL>
+static bool adjoint_fewest_rows(const Geom &g, bool grads) {
+  const int64_t N = g.N, n = N * g.nsys();
+  if (sizeof(REAL) == 8) return grads && N <= 24 && n >= 750000;
+  if (!grads) return N == 8;
+  if ((N & (N - 1)) == 0 || N < 4) return N <= 32 || (N <= 128 && n <= 200000);
+  return N <= 24 ? n >= 750000 : N <= 100 && n >= 2500000;
+}
+
 template <typename REAL>
 bool adjoint_default_cfg(const Geom &g, bool grads, HybridCfg *cfg) {
   // Strided systems: the forward solve's wide shape, unless they are few
@@ -416,6 +432,11 @@ bool adjoint_default_cfg(const Geom &g, bool grads, HybridCfg *cfg) {
     *cfg = c;
     return true;
   }
+  if (g.stride == 1 && adjoint_fewest_rows<REAL>(g, grads) &&
+      hybrid_fewest_rows_cfg<REAL>(g, &c) && adjoint_cfg_valid<REAL>(g, c)) {
+    *cfg = c;
+    return true;
+  }
   if (g.stride == 1 && sizeof(REAL) == 8 && g.N > 32 && g.N <= 256) {
     // fewer rows per lane than the solve takes at these lengths: with nine
     // streams the loads in flight matter more than the PCR (all gradients, 100
@@ -428,6 +449,8 @@ bool adjoint_default_cfg(const Geom &g, bool grads, HybridCfg *cfg) {
     if (adjoint_cfg_valid<REAL>(g, c)) { *cfg = c; return true; }
   }
   if (hybrid_plain_cfg<REAL>(g, &c)) {
+    // (a workgroup each for a few longer systems: 1000 rows x 64 FP64 8.5 against 9.9 us)
+    if (g.stride == 1 && sizeof(REAL) == 8 && g.N > 512 && g.nsys() <= 256) c.W = 1;
     for (int k = 0; k < 4 && !adjoint_cfg_valid<REAL>(g, c); ++k) {
       if (g.stride == 1 && c.W > 1) c.W /= 2;
       else if (c.M < 16) { c.M *= 2; c.P = (int)((g.N + c.M - 1) / c.M); }
