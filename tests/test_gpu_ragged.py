@@ -78,30 +78,55 @@ def test_forced_shapes_refused():
             api.ragged_batch_mixed_f32(*f, dev(off), max_len=300, sync=True)
 
 
+def _best_ms(call):
+    """The shortest of eight timed calls."""
+    times = []
+    for _ in range(8):
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        ev[0].record()
+        call()
+        ev[1].record()
+        torch.cuda.synchronize()
+        times.append(ev[0].elapsed_time(ev[1]))
+    return min(times)
+
+
+def _operands(n, dtype):
+    g = torch.Generator(device="cuda").manual_seed(5)
+    a, c, d = (torch.rand(n, dtype=dtype, device="cuda", generator=g) - 0.5 for _ in range(3))
+    return a, 2 + a.abs() + c.abs(), c, d
+
+
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 def test_understated_max_len_is_not_slow(dtype):
     """Systems of twice the rows that max_len says are solved on the shape chosen for
     it; they read their arrays a second time, so three times the declared call's time
     is the bound (a solve of each lane's rows straight from memory took seven)."""
     n, count = 4096, 4000
-    g = torch.Generator(device="cuda").manual_seed(5)
-    a, c, d = (torch.rand(n * count, dtype=dtype, device="cuda", generator=g) - 0.5
-               for _ in range(3))
-    b = 2 + a.abs() + c.abs()
+    a, b, c, d = _operands(n * count, dtype)
     off = torch.arange(0, (n + 1) * count, n, device="cuda")[:count + 1].contiguous()
     best, x = {}, {}
     for said in (n // 2, n):
-        times = []
-        for _ in range(8):
-            x[said] = d.clone()
-            ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
-            ev[0].record()
-            api.ragged_batch(a, b, c, x[said], off, max_len=said)
-            ev[1].record()
-            torch.cuda.synchronize()
-            times.append(ev[0].elapsed_time(ev[1]))
-        best[said] = min(times)
+        x[said] = d.clone()
+        api.ragged_batch(a, b, c, x[said], off, max_len=said)
+        y = d.clone()
+        best[said] = _best_ms(lambda: api.ragged_batch(a, b, c, y, off, max_len=said))
     print("understated %.3f ms, declared %.3f ms" % (best[n // 2], best[n]))
     tol = 1e-12 if dtype == torch.float64 else 1e-5
     assert (x[n] - x[n // 2]).abs().max().item() <= tol * x[n].abs().max().item()
     assert best[n // 2] <= 3 * best[n]
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_adding_to_u_costs_its_traffic(dtype):
+    """The Inc form reads u besides: 6 / 5 of the plain solve's bytes, so 1.4 times its
+    time is the bound (with every row's addition waiting for its own load it took 1.5)."""
+    rng = np.random.default_rng(8)
+    lens = np.exp(rng.uniform(np.log(237), np.log(6000), 16000)).astype(np.int64)
+    off = dev(np.concatenate([[0], np.cumsum(lens)]))
+    a, b, c, d = _operands(int(lens.sum()), dtype)
+    u = torch.zeros_like(d)
+    inc = _best_ms(lambda: api.ragged_batch(a, b, c, d, off, max_len=6000, u=u))
+    plain = _best_ms(lambda: api.ragged_batch(a, b, c, d, off, max_len=6000))
+    print("Inc %.3f ms, plain %.3f ms" % (inc, plain))
+    assert inc <= 1.4 * plain

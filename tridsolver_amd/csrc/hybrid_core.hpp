@@ -727,15 +727,27 @@ __device__ __forceinline__ void wave_put(const Lane &L, REAL *tile, const REAL *
   int lq = (L.t & 63) & (P64 - 1);
   asm volatile("" : "+v"(lq));
   const Fetch q = fetch_rows<REAL, M, FULL>(d + base, lq);
-  wave_to_fetch<M, FULL>(v, tile + (L.t - lq) * (M + 1), lq, q, P64);
-  if (L.active) {
-    REAL *dst = u + base;  // u == d for a solve in place
-    const int N = (int)L.N;
+  REAL *dst = u + base;  // u == d for a solve in place
+  const int N = (int)L.N, w0 = (L.p - lq) * M;
+  // Inc: u's rows all at once, from rows clamped into the system, ahead of the
+  // transpose. Row by row, each addition waits for its own load: 16,000 systems of
+  // 237-6000 rows 426 against 325 us in FP64, 238 against 171 in FP32.
+  REAL uv[INC ? M : 1];
+  if (INC && L.active) {
 #pragma unroll
     for (int r = 0; r < M; ++r) {
-      const int row = (L.p - lq) * M + (r == 0 ? q.e0 : q.e + P64 * r);
+      const int row = w0 + (r == 0 ? q.e0 : q.e + P64 * r);
+      uv[r] = dst[row < N ? row : N - 1];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  wave_to_fetch<M, FULL>(v, tile + (L.t - lq) * (M + 1), lq, q, P64);
+  if (L.active) {
+#pragma unroll
+    for (int r = 0; r < M; ++r) {
+      const int row = w0 + (r == 0 ? q.e0 : q.e + P64 * r);
       if (row < N) {
-        if (INC) dst[row] += v[r];
+        if (INC) dst[row] = uv[r] + v[r];
         else st<FULL>(&dst[row], v[r]);
       }
     }
@@ -921,15 +933,29 @@ __device__ __forceinline__ void long32_solve(int64_t base, int N, unsigned char 
   int ls = lane;
   asm volatile("" : "+v"(ls));
   const Fetch q = fetch_rows<REAL, M, true>(sd, ls);
-  wave_to_fetch<M, true>(rd, tile + (t - lane) * (M + 1), ls, q, 64);
   REAL *dst = u + base;
+  // Inc: u's rows half of them at once, as in wave_put (FP64 holds no more beside x)
+  constexpr int H = INC ? M / 2 : 1;
+  REAL uv[H];
+  auto row_of = [&](int r) { return wv * 64 * M + (r == 0 ? q.e0 : q.e + 64 * r); };
+  auto fetch_u = [&](int r0) {
+#pragma unroll
+    for (int r = 0; r < H; ++r) {
+      const int row = row_of(r0 + r);
+      uv[r] = dst[row < N ? row : N - 1];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (INC) fetch_u(0);
+  wave_to_fetch<M, true>(rd, tile + (t - lane) * (M + 1), ls, q, 64);
 #pragma unroll
   for (int r = 0; r < M; ++r) {
-    const int row = wv * 64 * M + (r == 0 ? q.e0 : q.e + 64 * r);
+    if (INC && r == H) fetch_u(H);
+    const int row = row_of(r);
     if (row < N) {
       // nontemporal stores at 256 lanes (8192 systems of 8192 rows: 0.50
       // against 0.53 ms), plain ones at 512 (16384 rows: 1.14 against 1.18)
-      if (INC) dst[row] += rd[r];
+      if (INC) dst[row] = uv[r % H] + rd[r];
       else st<(T == LONG32_T)>(&dst[row], rd[r]);
     }
   }
