@@ -293,6 +293,27 @@ def test_mixed_f32_default_strided_shapes(dims, sd, want):
         assert H.norm_rel_err(x.cpu().numpy(), xl) <= tol, refine
 
 
+@pytest.mark.parametrize("dims,sd,want", [
+    # one round of workgroups of 16 systems, and one workgroup more
+    ([32, 512, 128], 1, (16, 0)), ([32, 512, 129], 1, (32, 3)),
+    ([17, 257, 128], 1, (16, 0)), ([17, 257, 129], 1, (32, 3)),
+    ([15, 256, 512], 1, (16, 0)), ([15, 256, 513], 1, (32, 3)),
+    ([15, 160, 768], 1, (16, 0)), ([15, 160, 769], 1, (32, 3)),
+    ([16, 128, 1024], 1, (16, 0)), ([16, 128, 1025], 1, (32, 3))])
+def test_mixed_f32_strided_rounds(dims, sd, want):
+    """The kernel in registers only while all its workgroups run at once (two waves per
+    SIMD), with 0 and 1 refinements, at the bars of test_mixed_f32_vs_long_double_oracle."""
+    rng = np.random.default_rng(sum(dims) + sd)
+    a, b, c, d = _f32_case(rng, int(np.prod(dims)))
+    xl = oracle.batch_ld(a, b, c, d, ndim=3, solvedim=sd, dims=dims)
+    t = [dev(v) for v in (a, b, c, d)]
+    for refine, tol in ((0, 1e-5), (1, 1e-12)):
+        x = api.mixed_f32_strided_batch(*t, solvedim=sd, dims=dims, refinements=refine, sync=True)
+        algo, M, _, W, _ = api.last_config()
+        assert (algo, M) == (10, want[0]), (api.last_config(), refine)
+        assert H.norm_rel_err(x.cpu().numpy(), xl) <= tol, refine
+
+
 @pytest.mark.parametrize("shape", [(16, 2, 1), (16, 4, 8), (8, 1, 8), (8, 8, 1)])
 @pytest.mark.parametrize("N", [512, 300, 700, 37])
 def test_mixed_f32_forced_contig_lds(shape, N):

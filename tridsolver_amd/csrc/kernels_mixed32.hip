@@ -432,9 +432,12 @@ bool mixed32_cfg_valid(const Geom &g, const HybridCfg &c, int refine) {
 //   mixed32_kernel 1.58 / 2.03). Above 8 lanes per system 128-byte rows leave
 //   one workgroup per CU (LDS), 64-byte rows two: 384^3 z 358 against 371 us, y
 //   327 either way, 250 x 333 x 200 y 127 against 140, 512 x 512 x 200 y 267 against
-//   275. At most 512 workgroups of 32 systems: 16 rows per lane in registers, 16
-//   x-neighbours (64^3 z 10.5 against 13.3 us, 128^3 y 13.6 against 19.0, 64 x 64 x 400
-//   z 14.1 against 19.5; 160^3 z, 800 workgroups, 32.8 against 33.1).
+//   275. Up to as many workgroups of 16 systems as the CUs hold at two waves per
+//   SIMD (four per CU at most): 16 rows per lane in registers, 16 x-neighbours (64^3 z
+//   10.5 against 13.3 us, 128^3 y 13.6 against 19.0, 31 x 512 x 128 y 14.9 against 17.6,
+//   31 x 256 x 256 y 13.0 against 15.9, 31 x 128 x 512 y 13.5 against 16.0). In a second
+//   round they lose: 31 x 512 x 192 y 25.5 against 16.8, 31 x 256 x 300 y 19.7 against
+//   16.9, 160^3 z 32.8 against 33.1.
 bool mixed32_default_cfg(const Geom &g, int refine, HybridCfg *cfg) {
   HybridCfg c;
   const bool contig = g.stride == 1;
@@ -455,7 +458,8 @@ bool mixed32_default_cfg(const Geom &g, int refine, HybridCfg *cfg) {
     }
     return false;
   }
-  const bool few = (g.n0 + 31) / 32 * g.n1 <= 512;
+  const int64_t per_cu = std::min<int64_t>(4, 32 / std::max<int64_t>(1, (g.N + 15) / 16));
+  const bool few = (g.n0 + 15) / 16 * g.n1 <= 256 * per_cu;
   c.M = 32;
   c.P = (int)((g.N + c.M - 1) / c.M);
   c.P += c.P & 1;  // whole waves: W * P a multiple of 64
