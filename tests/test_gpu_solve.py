@@ -278,6 +278,19 @@ def test_rows_of_lines_that_end_in_half_a_segment(dims, sd, dtype, seg):
     assert cfg[0] == 8 and cfg[3] * np.dtype(dtype).itemsize == seg, cfg
 
 
+@pytest.mark.parametrize("inc", [False, True])
+@pytest.mark.parametrize("dims,sd,wide", [
+    ([16, 513, 300], 1, False), ([9, 1024, 257], 1, False), ([48, 700, 100], 1, False),
+    ([33, 1024, 86], 1, False),
+    ([17, 513, 300], 1, True), ([49, 700, 86], 1, True), ([80, 700, 52], 1, True),
+    ([16, 512, 257], 1, True)])
+def test_long_fp32_systems_on_narrow_lines(dims, sd, wide, inc):
+    """FP32 systems of 513-1024 rows: lines of one or three 16-system groups run the plain
+    kernel, others the wide one, whose last group they would leave half empty."""
+    cfg = run_case(dims, sd, np.float32, inc, (0, 0, 0), seed=sum(dims))
+    assert cfg[0] == (8 if wide else 3), cfg
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("inc", [False, True])
 @pytest.mark.parametrize("dims,sd,seg", [

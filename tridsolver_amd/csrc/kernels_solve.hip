@@ -418,8 +418,14 @@ bool hybrid_default_cfg(const Geom &g, HybridCfg *cfg) {
   // (one per CU) run the plain kernel at 16 rows per lane there: 32 x 600 x 128 y 12.3 us
   // against 15.1 with the wide one's 32, 64 x 64 x 800 z 19.8 against 23.6, 32 x 1000 x 20 y
   // 15.5 against 17.7. In two rounds it loses: 32 x 600 x 136 y 21.6 against 15.1.
-  const bool few = sizeof(REAL) == 4 && g.N > 512 && (g.n0 + 15) / 16 * g.n1 <= 256;
-  if (!few && hybrid_wide_default_cfg<REAL>(g, cfg)) return true;
+  // Lines of one or three such 16-system groups take it too: half of the last
+  // 32-system group would be empty (16 x 816 x 736 y 46.6 us against 51.6, 16 x 600 x 1800
+  // 89.5 against 115.5, 48 x 1000 x 400 92.7 against 119.8, the incremental solve 120
+  // against 143; lines of five the other way, 80 x 816 x 220 81.1 against 79.2).
+  const int64_t lines16 = (g.n0 + 15) / 16;
+  const bool plain = sizeof(REAL) == 4 && g.N > 512 &&
+                     (lines16 * g.n1 <= 256 || lines16 == 1 || lines16 == 3);
+  if (!plain && hybrid_wide_default_cfg<REAL>(g, cfg)) return true;
   // Contiguous systems of 4097-8192 rows: one per 256-thread workgroup at 32
   // rows per lane (variant 4), FP64 throughout (4500 / 6000 / 8192 rows: 3.8
   // / 4.3 / 4.7 TB/s against 3.2 / 3.7 / 4.0 with 512 lanes of 16 rows), FP32
