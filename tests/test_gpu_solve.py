@@ -279,6 +279,26 @@ def test_rows_of_lines_that_end_in_half_a_segment(dims, sd, dtype, seg):
 
 
 @pytest.mark.parametrize("inc", [False, True])
+@pytest.mark.parametrize("N,pad,G", [(16384, 0, 8), (16257, 127, 8), (16256, 128, 1),
+                                     (16380, 5, 1)])
+def test_workgroup_order_of_rows_64_kib_apart(N, pad, G, inc):
+    """Contiguous FP32 systems that fill rows 64 KiB apart: workgroups in eight ranges."""
+    rng = np.random.default_rng(N)
+    dims, pads = [N, 9], [N + pad, 9]
+    a, b, c, d = H.diag_dominant(rng, pads[0] * 9, np.float32)
+    u = rng.uniform(-1, 1, d.size).astype(np.float32) if inc else None
+    gd, gu = gpu_solve(a, b, c, d, u, solvedim=0, dims=dims, pads=pads)
+    cfg = api.last_config()
+    assert cfg[0] == 3 and cfg[4] == G, cfg
+    got, was = (gu - u, u) if inc else (gd, d)
+    for s in range(9):
+        i = slice(s * pads[0], s * pads[0] + N)
+        x = d[i].copy()
+        oracle.batch(a[i], b[i], c[i], x, None, ndim=1, solvedim=0, dims=[N], inc=False)
+        H.assert_norm_close(got[i], x, np.float32)
+
+
+@pytest.mark.parametrize("inc", [False, True])
 @pytest.mark.parametrize("dims,sd,wide", [
     ([16, 513, 300], 1, False), ([9, 1024, 257], 1, False), ([48, 700, 100], 1, False),
     ([33, 1024, 86], 1, False),

@@ -333,7 +333,9 @@ bool hybrid_plain_cfg(const Geom &g, HybridCfg *cfg) {
     // power of two and fill most of one wave: there one wave, whose PCR needs
     // no barrier (100 / 400 rows: 70 / 81 against 76 / 85 us). Plain workgroup
     // order: neighbouring systems share no lines, and all XCDs reading one
-    // region ran 4-8 % faster than eight regions at every length.
+    // region ran 4-8 % faster than eight regions at every length. Only FP32 systems
+    // that fill rows 64 KiB apart run faster in eight (1000 of 16384 rows 92.0 against
+    // 96.4 us; of 16000 rows 94.4 against 92.5, on rows 96 KiB apart 92.5 against 91.6).
     const int64_t n4 = sizeof(REAL) == 8 ? 112 : 256;
     const int first = g.N <= 4 ? 1
                       : sizeof(REAL) == 8 && g.N <= 32 ? 2
@@ -347,7 +349,7 @@ bool hybrid_plain_cfg(const Geom &g, HybridCfg *cfg) {
       c.P = (int)P;
       c.W = (int)std::max<int64_t>(1, 256 / P);
       if ((P & (P - 1)) != 0 && P <= 64 && 64 / P * P >= 48) c.W = (int)(64 / P);
-      c.G = 1;
+      c.G = sizeof(REAL) == 4 && g.st0 % 16384 == 0 && g.N > 16256 ? 8 : 1;
       if (hybrid_cfg_valid<REAL>(g, c)) { *cfg = c; return true; }
     }
     return false;
