@@ -240,9 +240,60 @@ def test_solve_to_equals_solve_in_place(dims, sd, force, dtype):
     assert bool((x == 7.0).all())
 
 
+@pytest.mark.parametrize("N,pad,systems,dtype,M,W", [
+    # FP32: vectors where every row holds whole ones, else 2 rows per lane up to 64
+    (8, 0, 40000, np.float32, 4, 128), (8, 4, 40000, np.float32, 4, 128),
+    (8, 2, 40000, np.float32, 2, 64), (7, 0, 40000, np.float32, 2, 64),
+    (12, 0, 40000, np.float32, 4, 21), (12, 2, 40000, np.float32, 2, 42),
+    (64, 1, 4000, np.float32, 2, 8), (65, 1, 4000, np.float32, 4, 3),
+    (200, 0, 2000, np.float32, 4, 5), (200, 2, 2000, np.float32, 4, 1),
+    (4, 3, 90000, np.float32, 1, 64), (3, 1, 90000, np.float32, 1, 85),
+    # FP64: rows apart, odd pitches
+    (8, 0, 40000, np.float64, 2, 64), (8, 1, 40000, np.float64, 1, 32),
+    (9, 1, 40000, np.float64, 2, 51), (5, 0, 60000, np.float64, 2, 85),
+    (5, 2, 60000, np.float64, 1, 51), (6, 0, 60000, np.float64, 2, 21),
+    (176, 0, 2000, np.float64, 8, 11), (176, 1, 2000, np.float64, 4, 5),
+    (190, 1, 2000, np.float64, 4, 1), (192, 1, 2000, np.float64, 8, 2),
+    (100, 0, 3200, np.float64, 2, 5), (100, 0, 3201, np.float64, 4, 2),
+    (64, 0, 3126, np.float64, 4, 16), (64, 2, 5000, np.float64, 1, 4),
+    (64, 2, 5001, np.float64, 4, 16)])
+@pytest.mark.parametrize("inc", [False, True])
+def test_contiguous_systems_apart(N, pad, systems, dtype, M, W, inc):
+    """Rows per lane and systems per workgroup of short contiguous systems by the layout of
+    their rows, and the results on a sample of the systems."""
+    rng = np.random.default_rng(N + systems)
+    dims, pads = [N, systems], [N + pad, systems]
+    a, b, c, d = H.diag_dominant(rng, pads[0] * systems, dtype)
+    u = rng.uniform(-1, 1, d.size).astype(dtype) if inc else None
+    gd, gu = gpu_solve(a, b, c, d, u, solvedim=0, dims=dims, pads=pads)
+    cfg = api.last_config()
+    assert cfg[0] == 3 and (cfg[1], cfg[3]) == (M, W), cfg
+    got, was = (gu, u) if inc else (gd, d)
+    for s in list(range(0, systems, 997)) + [systems - 1]:
+        i = slice(s * pads[0], s * pads[0] + N)
+        x = d[i].copy()
+        oracle.batch(a[i], b[i], c[i], x, None, ndim=1, solvedim=0, dims=[N], inc=False)
+        H.assert_norm_close(got[i] - was[i] if inc else got[i], x, dtype)
+        assert np.array_equal(got[i.stop:i.stop + pad], was[i.stop:i.stop + pad]), s
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_contiguous_lines_shorter_than_a_workgroup(dtype):
+    """No lanes beyond the systems of a line, where lines of systems lie apart."""
+    dims, pads = [16, 12, 1200], [16, 14, 1200]
+    n = int(np.prod(pads))
+    rng = np.random.default_rng(3)
+    a, b, c, d = H.diag_dominant(rng, n, dtype)
+    gd, _ = gpu_solve(a, b, c, d, solvedim=0, dims=dims, pads=pads)
+    assert api.last_config()[0] == 3 and api.last_config()[3] == 12, api.last_config()
+    od = d.copy()
+    oracle.batch(a, b, c, od, None, ndim=3, solvedim=0, dims=dims, pads=pads, inc=False)
+    H.assert_norm_close(gd, od, dtype)
+
+
 @pytest.mark.parametrize("N,systems,dtype,M", [
     (40, 2048, np.float64, 1), (40, 8192, np.float64, 4), (128, 64, np.float64, 2),
-    (129, 64, np.float64, 8), (8, 16384, np.float64, 1), (7, 16384, np.float64, 2),
+    (130, 64, np.float64, 8), (8, 16384, np.float64, 1), (7, 16384, np.float64, 2),
     (100, 2000, np.float32, 2), (100, 2001, np.float32, 4), (64, 1024, np.float32, 1)])
 @pytest.mark.parametrize("inc", [False, True])
 def test_small_contiguous_batches(N, systems, dtype, M, inc):

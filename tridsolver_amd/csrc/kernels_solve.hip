@@ -329,18 +329,28 @@ bool hybrid_plain_cfg(const Geom &g, HybridCfg *cfg) {
     // rows below against 99 / 87 / 132 / 133 / 909 / 232 / 153 at the fewest rows
     // that keep a system in one wave (1, 2, 2, 4, 8, 16, 16 with G = 8). FP32 stays
     // at 4 rows (one vector) up to 256: 200 rows 49 against 54 us at 8.
+    // Vector access needs whole vectors in every row; without it 2 rows there, up to
+    // 64 (4000000 elements of 8 / 16 / 32 rows, 2 apart: 22.6 / 21.4 / 21.2 us against 41.7
+    // / 35.0 / 31.5 at 4 and 30.1 / 31.6 / 34.2 at 1). FP64 rows apart from each other:
+    // 1 up to 8 rows (5 rows, 2 apart: 46.5 against 52.3 us; abutting 39 against 35.5),
+    // and 4 up to 190 on odd pitches (128 / 176 rows 31.8 / 31.9 against 35.5 / 35.9).
     // Workgroups of about 256 threads, except where the systems' lanes are no
     // power of two and fill most of one wave: there one wave, whose PCR needs
-    // no barrier (100 / 400 rows: 70 / 81 against 76 / 85 us). Plain workgroup
+    // no barrier (100 / 400 rows: 70 / 81 against 76 / 85 us), but not systems of a few
+    // lanes that rows past N or misaligned rows split (11 rows FP64 43.7 against 45.6
+    // us, 12 rows FP32, 2 apart, 24.3 / 25.7) nor one of 48-51 lanes of vectors (200 rows
+    // FP32 62.6 against 66.2). Plain workgroup
     // order: neighbouring systems share no lines, and all XCDs reading one
     // region ran 4-8 % faster than eight regions at every length. Only FP32 systems
     // that fill rows 64 KiB apart run faster in eight (1000 of 16384 rows 92.0 against
     // 96.4 us; of 16000 rows 94.4 against 92.5, on rows 96 KiB apart 92.5 against 91.6).
-    const int64_t n4 = sizeof(REAL) == 8 ? 112 : 256;
-    const int first = g.N <= 4 ? 1
-                      : sizeof(REAL) == 8 && g.N <= 32 ? 2
-                      : g.N <= n4 ? 4
-                      : g.N <= 2048 ? 8 : 16;
+    const bool fp64 = sizeof(REAL) == 8;
+    const bool vec = !fp64 && g.N % 4 == 0 && g.st0 % 4 == 0 && g.st1 % 4 == 0;
+    const bool apart = g.st0 != g.N;
+    const bool one = g.N <= 4 || (fp64 && g.N <= 8 && apart);
+    const int64_t n2 = fp64 ? 32 : vec ? 4 : 64;
+    const int64_t n4 = !fp64 ? 256 : g.st0 % 2 != 0 ? 190 : 112;
+    const int first = one ? 1 : g.N <= n2 ? 2 : g.N <= n4 ? 4 : g.N <= 2048 ? 8 : 16;
     for (int M : Ms) {
       if (M < first) continue;
       const int64_t P = (g.N + M - 1) / M;
@@ -348,7 +358,11 @@ bool hybrid_plain_cfg(const Geom &g, HybridCfg *cfg) {
       c.M = M;
       c.P = (int)P;
       c.W = (int)std::max<int64_t>(1, 256 / P);
-      if ((P & (P - 1)) != 0 && P <= 64 && 64 / P * P >= 48) c.W = (int)(64 / P);
+      const bool split = ((P < 5 || one) && apart && !vec) || g.N % M != 0 || !(fp64 || vec);
+      if ((P & (P - 1)) != 0 && P <= 64 && 64 / P * P >= (vec && P > 32 ? 52 : 48) &&
+          (P >= 8 || !split))
+        c.W = (int)(64 / P);
+      c.W = (int)std::min<int64_t>(c.W, g.n0);  // no lanes beyond a line's systems
       c.G = sizeof(REAL) == 4 && g.st0 % 16384 == 0 && g.N > 16256 ? 8 : 1;
       if (hybrid_cfg_valid<REAL>(g, c)) { *cfg = c; return true; }
     }
@@ -450,8 +464,12 @@ bool hybrid_default_cfg(const Geom &g, HybridCfg *cfg) {
   // Contiguous batches too small to fill the chip: fewer rows per lane, whose shorter
   // chains count there (us at the fewest rows / at hybrid_plain_cfg's: FP64 40 x 2048
   // 5.9 / 7.4, 4096 6.7 / 7.7, 8192 8.7 / 8.5; 128 x 1024 6.4 / 6.7, 2048 7.5 / 6.9; 8 x 16384
-  // 4.4 / 5.5; FP32 12 x 8192 4.7 / 5.3, 100 x 2048 5.7 / 6.2, 64 x 4096 5.6 / 4.6).
-  if (g.stride == 1 && g.N >= 8 && g.N <= 128 && g.N * g.nsys() <= 200000 &&
+  // 4.4 / 5.5; FP32 12 x 8192 4.7 / 5.3, 100 x 2048 5.7 / 6.2, 64 x 4096 5.6 / 4.6; 80 x 3100 and
+  // 100 x 2500 FP64 7.9 / 8.3 and 7.6 / 8.6, at 100 x 4000 the same).
+  const bool pow2 = (g.N & (g.N - 1)) == 0;
+  const int64_t small =
+      sizeof(REAL) == 8 && g.N > 32 && (!pow2 || g.st0 != g.N) ? 320000 : 200000;
+  if (g.stride == 1 && g.N >= 8 && g.N <= 128 && g.N * g.nsys() <= small &&
       hybrid_fewest_rows_cfg<REAL>(g, cfg))
     return true;
   return hybrid_plain_cfg<REAL>(g, cfg);
