@@ -1114,10 +1114,82 @@ def test_adjoint_of_a_few_longer_contiguous_systems():
     ([16, 16, 384], np.float64, True, True), ([16, 40, 384], np.float64, False, True),
     ([16, 40, 513], np.float64, False, False), ([22, 31, 110], np.float64, True, True),
     ([16, 600, 96], np.float64, True, True), ([16, 600, 97], np.float64, True, False),
-    ([32, 46, 500], np.float32, True, True), ([32, 900, 40], np.float32, True, False)])
+    ([32, 46, 500], np.float32, True, True), ([32, 900, 49], np.float32, True, False),
+    ([32, 900, 48], np.float32, True, True)])
 def test_adjoint_of_few_systems(dims, dtype, grads, plain):
     """Few strided systems take the kernel without staging, at its fewer rows per lane
     or narrower rows; more take the wide one (16 or 32 rows, 128 bytes or more)."""
     cfg = _adjoint_config(dims, 1, dtype, grads)
     wide = cfg[1] in (16, 32) and cfg[3] * np.dtype(dtype).itemsize >= 128
     assert cfg[0] == 4 and wide != plain, cfg
+
+
+@pytest.mark.parametrize("dims,dtype,grads,plain", [
+    # lines of at most half a 128-byte segment
+    ([8, 1000, 512], np.float64, False, True), ([9, 600, 129], np.float64, False, False),
+    ([16, 300, 1024], np.float32, True, True), ([17, 300, 129], np.float32, True, False),
+    # whole waves: aligned and misaligned lines
+    ([16, 128, 40], np.float64, False, False), ([33, 128, 80], np.float64, False, True),
+    ([33, 128, 101], np.float64, True, False), ([16, 128, 512], np.float64, True, True),
+    # one long misaligned line
+    ([28001, 256], np.float64, True, True), ([28000, 256], np.float64, True, False),
+    ([28001, 256], np.float64, False, False)])
+def test_adjoint_kernel_by_the_shape_of_the_lines(dims, dtype, grads, plain):
+    """The wide kernel runs 16 rows per lane on 128 bytes or more (32 in FP32)."""
+    cfg = _adjoint_config(dims, 1, dtype, grads)
+    wide = cfg[1] in (16, 32) and cfg[3] * np.dtype(dtype).itemsize >= 128
+    assert cfg[0] == 4 and wide != plain, cfg
+
+
+@pytest.mark.parametrize("dims,W,G", [
+    ([64, 256, 80], 32, 8), ([64, 256, 79], 16, 8), ([48, 256, 200], 16, 8),
+    ([64, 192, 300], 32, 1), ([66, 192, 300], 32, 8), ([64, 513, 80], 16, 8)])
+def test_adjoint_rows_and_order(dims, W, G):
+    """FP64 adjoint on strided systems: 256-byte rows from 160 workgroups, plain order for
+    short systems on aligned lines, and the results at the bar above."""
+    assert _adjoint_config(dims, 1, np.float64, True)[3:] == (W, G)
+    rng = np.random.default_rng(sum(dims))
+    n = int(np.prod(dims))
+    a, b, c, x = H.diag_dominant(rng, n, np.float64)
+    w = rng.standard_normal(n)
+    ref = oracle.adjoint(a, b, c, x, w, ndim=3, solvedim=1, dims=dims)
+    out = api.adjoint_strided_batch(*(dev(v) for v in (a, b, c, x, w)), solvedim=1, dims=dims,
+                                    grad_a=True, grad_b=True, grad_c=True, sync=True)
+    for got, want in zip(out, ref):
+        assert H.norm_rel_err(got.cpu().numpy(), want) <= 1e-12
+
+
+@pytest.mark.parametrize("N,pad,systems,dtype,M", [
+    (8, 0, 90000, np.float64, 2), (8, 2, 90000, np.float64, 1), (12, 2, 33333, np.float64, 1),
+    (12, 2, 29999, np.float64, 2), (40, 1, 70000, np.float64, 1), (40, 1, 60000, np.float64, 2),
+    (12, 0, 16499, np.float32, 4), (12, 2, 16500, np.float32, 1), (64, 1, 40000, np.float32, 1),
+    (64, 1, 30000, np.float32, 2), (64, 4, 40000, np.float32, 4)])
+def test_adjoint_of_contiguous_systems_apart(N, pad, systems, dtype, M):
+    """Rows per lane of short contiguous systems on rows apart from each other, against the
+    oracle on a sample of the systems."""
+    rng = np.random.default_rng(N + systems)
+    n = (N + pad) * systems
+    a, b, c, x = H.diag_dominant(rng, n, dtype)
+    w = rng.standard_normal(n).astype(dtype)
+    out = api.adjoint_strided_batch(*(dev(v) for v in (a, b, c, x, w)), solvedim=0,
+                                    dims=[N, systems], pads=[N + pad, systems], grad_a=True,
+                                    grad_b=True, grad_c=True, sync=True)
+    assert api.last_config()[:2] == (4, M), api.last_config()
+    out = [t.cpu().numpy() for t in out]
+    for s in list(range(0, systems, 4999)) + [systems - 1]:
+        i = slice(s * (N + pad), s * (N + pad) + N)
+        ref = oracle.adjoint(*(v[i].astype(np.float64) for v in (a, b, c, x, w)), ndim=1,
+                             solvedim=0, dims=[N])
+        for got, want in zip(out, ref):
+            assert H.norm_rel_err(got[i], want) <= (1e-12 if dtype == np.float64 else 1e-5), s
+
+
+def test_adjoint_of_contiguous_planes_apart():
+    """Gaps between planes count as gaps between rows do."""
+    for dims, pads, M in (([16, 40, 1000], [16, 42, 1000], 1), ([16, 40, 1000], None, 2)):
+        n = int(np.prod(pads or dims))
+        a, c, x, w = (torch.rand(n, dtype=torch.float64, device="cuda") - 0.5 for _ in range(4))
+        api.adjoint_strided_batch(a, 2 + a.abs() + c.abs(), c, x, w, solvedim=0, dims=dims,
+                                  pads=pads or dims, grad_a=True, grad_b=True, grad_c=True,
+                                  sync=True)
+        assert api.last_config()[:2] == (4, M), (api.last_config(), pads)

@@ -384,15 +384,34 @@ bool adjoint_cfg_valid(const Geom &g, const HybridCfg &c) {
 // 5.8 / 5.0 at 256 groups, 1000 rows 23.2 / 24.4 at 128, 32.3 / 24.5 at 192. FP32, all
 // gradients, 40 rows, 512 groups 7.9 / 8.5, 768 11.6 / 9.1; 800 rows, 32 groups 20.2 / 22.7,
 // 64 32.8 / 27.8.
+// By the lines' shape too: on lines of at most half a segment the wide kernel leaves half
+// its systems out (half: 8 x 1000 x 512 FP64 y, lambda alone, 38 against 50; 16 x 512 x 512
+// FP32 20.5 against 23.0), and whole waves count for less where rows are misaligned
+// (33 x 128 x 62 FP64 y, lambda alone, 5.9 against 6.9, on aligned lines 5.8 against 5.1).
+// One long misaligned line of FP64 systems of up to 256 rows stays with adjoint_kernel,
+// all gradients (32763 x 256 z 151 against 165, 601 x 404 x 136 z 580 against 597; 16379 x
+// 300 z 94 against 92, 199 x 123 x 200 z, 1530 groups, 102 against 91).
 template <typename REAL>
-static int64_t adjoint_plain_most(int64_t N, bool grads) {
+static int64_t adjoint_plain_most(const Geom &g, bool grads) {
+  const int64_t N = g.N;
   const bool fp64 = sizeof(REAL) == 8, whole = N % (fp64 ? 64 : 32) == 0;
+  const bool half = g.n0 * (int64_t)sizeof(REAL) <= 64;
+  const bool aligned = !half && wide::wide_rows_aligned<REAL>(g, 0);
   if (N <= 16) return fp64 ? INT64_MAX : 16384 / N;
-  if (N > 512) return fp64 ? (grads ? 96 : 128) : grads ? 32 : 64;
-  if (N > 256) return fp64 ? (whole ? 0 : 256) : grads ? 96 : 128;
-  if (whole) return !grads ? 0 : N <= 96 ? 256 : N <= 192 ? 192 : fp64 ? 0 : 128;
-  if (!grads) return fp64 && N < 64 ? 512 : 256;
-  return N < 64 && fp64 ? 1024 : fp64 || N < 96 ? 512 : 384;
+  if (half && (fp64 ? N > 512 : N > 256 && N <= 512)) return INT64_MAX;
+  if (fp64 && grads && !aligned && g.n1 == 1 && N <= 256 && g.n0 > 28000) return INT64_MAX;
+  if (N > 512) return fp64 ? (grads ? 96 : 128) : grads ? 48 : 64;
+  if (N > 256) return !fp64 ? 128 : !whole ? 256 : half ? 160 : 0;
+  if (!whole) {
+    if (!grads) return N < 64 ? 512 : aligned ? 256 : 300;
+    return fp64 && N < 64 ? 1024 : fp64 || N <= 192 ? 512 : 384;
+  }
+  if (!grads)
+    return aligned ? 0 : N < 64 ? 300 : N <= 192 ? (fp64 ? 256 : 160) : half ? 160 : 32;
+  if (N <= 96) return fp64 && !aligned ? 512 : 256;
+  if (N <= 192) return aligned ? 512 : half ? 384 : fp64 ? 300 : 224;
+  if (half) return 160;
+  return fp64 ? (aligned ? 0 : 64) : aligned ? 384 : 128;
 }
 
 // Whether contiguous systems take the fewest rows per lane that keep a system in one
@@ -402,13 +421,23 @@ static int64_t adjoint_plain_most(int64_t N, bool grads) {
 // 25, 24 x 16384 7.9 / 7.4, 100 x 65536 58 / 64, 100 x 8192 10.7 / 9.2, 64 x 2048 5.5 / 5.9, 64 x
 // 4096 6.6 / 6.1; FP64: 16 x 65536 17.9 / 19.7, 16 x 16384 7.9 / 6.8. lambda alone, FP32, 8 x
 // 16384 4.1 / 4.6.
+// Rows or planes apart from each other have more lines: sooner there (FP64, 8 / 16 rows, 600000
+// elements, 2 apart, as at 750000: 0.70 / 0.77 of the time; FP32 12 rows, 400000, 0.76).
 template <typename REAL>
 static bool adjoint_fewest_rows(const Geom &g, bool grads) {
   const int64_t N = g.N, n = N * g.nsys();
-  if (sizeof(REAL) == 8) return grads && N <= 24 && n >= 750000;
+  const bool apart = g.st0 != N || (g.n1 > 1 && g.st1 != g.n0 * N), pow2 = (N & (N - 1)) == 0;
+  if (sizeof(REAL) == 8) {
+    if (!grads) return false;
+    if (N <= 24) return n >= 750000 || (apart && g.nsys() >= 30000);
+    return apart && N <= 50 && n >= (N <= 32 ? 750000 : 2500000);
+  }
   if (!grads) return N == 8;
-  if ((N & (N - 1)) == 0 || N < 4) return N <= 32 || (N <= 128 && n <= 200000);
-  return N <= 24 ? n >= 750000 : N <= 100 && n >= 2500000;
+  if (N < 4 || (pow2 && N <= 32)) return true;
+  if (N <= 16) return g.nsys() >= 16500;
+  if (N <= 24) return n >= 750000;
+  if (pow2) return N <= 128 && (n <= 200000 || (g.st0 % 4 != 0 && n >= 2500000));
+  return N <= 100 && n >= (N <= 64 && g.st0 % 4 != 0 ? 750000 : 2500000);
 }
 
 template <typename REAL>
@@ -417,8 +446,10 @@ bool adjoint_default_cfg(const Geom &g, bool grads, HybridCfg *cfg) {
   // (adjoint_plain_most). Otherwise the same shapes as the forward solve where
   // they fit the adjoint's register budget, else the next valid one.
   HybridCfg c;
-  const int64_t rows = (g.n0 * g.n1 * (int64_t)sizeof(REAL) + 127) / 128;
-  if (g.stride != 1 && rows > adjoint_plain_most<REAL>(g.N, grads) &&
+  // (128-byte groups of the lines; two lines of at most half a group count as one)
+  const int64_t line = g.n0 * (int64_t)sizeof(REAL);
+  const int64_t rows = line <= 64 ? (g.n1 * line + 127) / 128 : (line + 127) / 128 * g.n1;
+  if (g.stride != 1 && rows > adjoint_plain_most<REAL>(g, grads) &&
       hybrid_wide_default_cfg<REAL>(g, &c) && adjoint_wide<REAL>(g, c)) {
     if (sizeof(REAL) == 4 && g.N <= 512 && wide::wide_many_groups<REAL>(g) &&
         wide::wide_whole_segments<REAL>(g)) {
@@ -429,6 +460,17 @@ bool adjoint_default_cfg(const Geom &g, bool grads, HybridCfg *cfg) {
       c.W = 64;
       c.P = (int)((g.N + c.M - 1) / c.M);
     }
+    if (sizeof(REAL) == 8 && g.N > 192 && g.N <= 512 && wide::wide_many_groups<REAL>(g, 160) &&
+        wide::wide_whole_segments<REAL>(g)) {
+      // 256-byte rows of long systems from fewer workgroups on than in the solve (64 x 256
+      // x 80 y 17.9 against 22.7 us, lambda alone, x 128 14.9 / 15.5; 64 x 400 x 64, 128
+      // workgroups, 26.8 against 23.3)
+      c.W = 32;
+      c.P = (int)(g.N + 31) / 32 * 2;
+    }
+    // plain workgroup order for short ones on aligned lines (64 x 128 x 1024 y 94.7 against
+    // 104.3 us, 192^3 y 86.8 / 90.0; 512 x 512 x 64 y the other way, 230.6 / 216.9)
+    if (sizeof(REAL) == 8 && g.N <= 192 && wide::wide_rows_aligned<REAL>(g, 0)) c.G = 1;
     *cfg = c;
     return true;
   }
