@@ -309,12 +309,12 @@ def test_small_contiguous_batches(N, systems, dtype, M, inc):
     ([16, 32, 400], 1, np.float64, 256),  # short systems: half the lanes at 128 bytes
     # three: the same; two: whole 256-byte segments
     ([40, 200, 192], 1, np.float64, 128), ([96, 300, 520], 1, np.float32, 128),
-    ([32, 200, 384], 1, np.float64, 256), ([64, 300, 1030], 1, np.float32, 256),
+    ([32, 200, 384], 1, np.float64, 256), ([64, 321, 1030], 1, np.float32, 256), ([64, 320, 1030], 1, np.float32, 128),
     # five and more: by the systems' length, until the empty half is small
     ([80, 320, 128], 1, np.float64, 256), ([80, 321, 128], 1, np.float64, 128),
     ([144, 384, 342], 1, np.float32, 128), ([144, 385, 342], 1, np.float32, 256),
     ([400, 400, 31], 1, np.float64, 256), ([368, 400, 33], 1, np.float64, 128),
-    ([288, 300, 206], 1, np.float32, 256)])
+    ([288, 330, 206], 1, np.float32, 256)])
 def test_rows_of_lines_that_end_in_half_a_segment(dims, sd, dtype, seg):
     """Strided batches whose lines are an odd number of 128-byte segments: the row
     width of the default shape, and the results of the smaller ones."""

@@ -383,10 +383,10 @@ bool adjoint_cfg_valid(const Geom &g, const HybridCfg &c) {
 // 23.2, 512 56 / 49; 1000 rows, 64 groups 22.3 / 28.2, 128 39.6 / 34.7; lambda alone, 64 rows
 // 5.8 / 5.0 at 256 groups, 1000 rows 23.2 / 24.4 at 128, 32.3 / 24.5 at 192. FP32, all
 // gradients, 40 rows, 512 groups 7.9 / 8.5, 768 11.6 / 9.1; 800 rows, 32 groups 20.2 / 22.7,
-// 64 32.8 / 27.8.
+// 64 32.8 / 27.8; 592 rows of a z line of 56 18.5 / 22.5, 32 rows of 312 7.8 / 9.1.
 // By the lines' shape too: on lines of at most half a segment the wide kernel leaves half
 // its systems out (half: 8 x 1000 x 512 FP64 y, lambda alone, 38 against 50; 16 x 512 x 512
-// FP32 20.5 against 23.0), and whole waves count for less where rows are misaligned
+// FP32 20.5 against 23.0; a quarter, lambda alone, 8 x 621 x 309 FP32 17.5 / 23.4), and whole waves count for less where rows are misaligned
 // (33 x 128 x 62 FP64 y, lambda alone, 5.9 against 6.9, on aligned lines 5.8 against 5.1).
 // One long misaligned line of FP64 systems of up to 256 rows stays with adjoint_kernel,
 // all gradients (32763 x 256 z 151 against 165, 601 x 404 x 136 z 580 against 597; 16379 x
@@ -400,15 +400,16 @@ static int64_t adjoint_plain_most(const Geom &g, bool grads) {
   if (N <= 16) return fp64 ? INT64_MAX : 16384 / N;
   if (half && (fp64 ? N > 512 : N > 256 && N <= 512)) return INT64_MAX;
   if (fp64 && grads && !aligned && g.n1 == 1 && N <= 256 && g.n0 > 28000) return INT64_MAX;
-  if (N > 512) return fp64 ? (grads ? 96 : 128) : grads ? 48 : 64;
+  if (!fp64 && N > 512 && g.n0 <= 8) return grads ? 80 : 256;
+  if (N > 512) return fp64 ? (grads ? 96 : 128) : grads ? 60 : 64;
   if (N > 256) return !fp64 ? 128 : !whole ? 256 : half ? 160 : 0;
   if (!whole) {
     if (!grads) return N < 64 ? 512 : aligned ? 256 : 300;
-    return fp64 && N < 64 ? 1024 : fp64 || N <= 192 ? 512 : 384;
+    return N < (fp64 ? 64 : 32) ? 1024 : fp64 || N <= 192 ? 512 : 384;
   }
   if (!grads)
     return aligned ? 0 : N < 64 ? 300 : N <= 192 ? (fp64 ? 256 : 160) : half ? 160 : 32;
-  if (N <= 96) return fp64 && !aligned ? 512 : 256;
+  if (N <= 96) return (fp64 ? !aligned : N < 64) ? 512 : 256;
   if (N <= 192) return aligned ? 512 : half ? 384 : fp64 ? 300 : 224;
   if (half) return 160;
   return fp64 ? (aligned ? 0 : 64) : aligned ? 384 : 128;

@@ -401,8 +401,9 @@ bool hybrid_wide_default_cfg(const Geom &g, HybridCfg *cfg) {
   //    256-byte ones would leave too many systems out (wide_whole_segments).
   //  - FP64 at 16 rows per lane (512^3 z 0.94 against 0.95 ms at 32, 251 x
   //    300 x 300 y 213 against 222 us). FP32 at 32 rows per lane on 256-byte
-  //    rows of 257-512 (512^3 y 0.466 against 0.484 ms for 16 on 128-byte
-  //    rows, given 1024 such workgroups: 200 x 300 x 150 y, 600, 56 against 48
+  //    rows of 321-512 (512^3 y 0.466 against 0.484 ms for 16 on 128-byte
+  //    rows, 592 x 320 x 128 y 108.7 against 107.2 us, 320 x 272 x 256 y 83.6 against
+  //    77.8; given 1024 such workgroups: 200 x 300 x 150 y, 600, 56 against 48
   //    us) and above 512, else at 16 on 128-byte rows (203 x 170 x 300 y 52
   //    against 55 us).
   //  - workgroups dealt to the XCDs in 8 ranges (G), so that neighbouring
@@ -415,7 +416,7 @@ bool hybrid_wide_default_cfg(const Geom &g, HybridCfg *cfg) {
   const int64_t row_bytes = g.stride * (int64_t)sizeof(REAL);
   const bool wide = g.N <= 512 && wide::wide_whole_segments<REAL>(g) &&
                     (fp64 ? wide::wide_many_groups<REAL>(g)
-                          : g.N > 256 && wide::wide_many_groups<REAL>(g, 1024));
+                          : g.N > 320 && wide::wide_many_groups<REAL>(g, 1024));
   c.M = fp64 || (!wide && g.N <= 512) ? 16 : 32;
   c.W = (wide ? 256 : 128) / (int)sizeof(REAL);
   const int per_wave = std::max(1, 64 / c.W);
