@@ -52,7 +52,9 @@ EXTERN_C tridStatus_t tridAdiRunS(const TridParams *ctx, float lambda, float *u,
  * position, :59-73). The ADI coefficients depend only on the grid position,
  * so each sweep computes a, b, c from (i, j, k), and the x sweep computes its
  * right-hand side from u: 56 B per point per step at FP64 instead of 168 with
- * arrays read back, same results bit for bit as tridAdiStep. du is workspace. */
+ * arrays read back, the results of tridAdiStep: bit for bit where that takes
+ * the matrix-free sweeps too, to rounding where it takes the array solves (opts 1 or 2, a
+ * forced shape, lines longer than a workgroup holds). du is workspace. */
 EXTERN_C tridStatus_t tridAdiStepFusedD(double lambda, double *u, double *du, int nx, int ny,
                                         int nz);
 EXTERN_C tridStatus_t tridAdiStepFusedS(float lambda, float *u, float *du, int nx, int ny,

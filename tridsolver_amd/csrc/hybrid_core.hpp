@@ -125,9 +125,8 @@ __device__ __forceinline__ int64_t fetch_row(const Lane &L, int r) {
 }
 
 // Element access with the nontemporal hint (NT) or without. NT marks data
-// that a kernel reads or writes once. The strided-batch kernels use it:
-// 512^3 FP64 x / y / z took 0.89 / 0.98 / 1.14 ms with it against 1.01 /
-// 1.04 / 1.19 without. Kernels whose data a caller reuses across calls from
+// that a kernel reads or writes once. The strided-batch kernels use it
+// (512^3 FP64 x 0.89 ms with it against 1.01 without, before x took 0.85). Kernels whose data a caller reuses across calls from
 // the 256 MB Infinity Cache (the FP32 ragged solve, the fused ADI steps) ran
 // slower with it and keep plain access.
 template <bool NT, typename T>

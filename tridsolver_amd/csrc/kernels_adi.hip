@@ -256,7 +256,7 @@ __global__ __launch_bounds__((AdiBounds<REAL, M>::threads)) void adi_solve_kerne
 // ---- sweeps along y and z, several lines per lane ----------------------------
 // Every line away from the grid's boundary has the same coefficients, and the lines
 // on it have a right-hand side of zeros (the x sweep leaves du = 0 there), which any
-// coefficients solve to zeros. So a lane takes V neighbouring lines, one 16-byte
+// regular coefficients solve to zeros. So a lane takes V neighbouring lines, one 16-byte
 // vector per row, and forms the pivots, the forward factors and the reduced
 // system's coefficients once for all of them: per point, the right-hand side's
 // four multiply-adds and 1/V of the rest (one division per row). Against a line per
@@ -393,8 +393,10 @@ __global__ __launch_bounds__(ADI_VEC_T) void adi_vec_kernel(Geom g, int P, int W
 // not apply: lines in whole vectors, 16-byte aligned, arrays below 4 GiB, a line
 // within a workgroup. Eight lanes' vectors a row are a 128-byte line (four: 200 x 168 x
 // 147 FP64 66 against 68 us a step, 300^3 412 against 389; sixteen 409). 16 rows per lane
-// for the longer lines (300^3 FP64 389 against 418 us; 256^3 FP64 166 against 170, FP32
-// 82 against 81; 200 x 168 x 147 FP32 39 against 37).
+// for the longer lines (us a step at 16 / 8 rows: FP64 300^3 389 / 413, 256^3 150 / 153, 128 x
+// 320^2 120 / 133, 64 x 400^2 98 / 110, 128 x 480 x 200 113 / 119; FP32 300^3 139 / 143, 128 x 448
+// x 256 71.5 / 73.1, 64 x 400^2 55.5 / 56.5; below the line FP32 256 x 176^2 45.6 / 44.1, 512 x
+// 144^2 58.7 / 56.2, FP64 256 x 160^2 70.0 / 70.0).
 template <typename REAL>
 bool adi_vec_cfg(const REAL *d, const REAL *u, int nx, int ny, int nz, int sd, Geom *g,
                  HybridCfg *cfg) {
@@ -611,8 +613,8 @@ bool adi_cfg(int dev, const Geom &g, HybridCfg *cfg) {
   return hybrid_cfg_valid<REAL>(g, *cfg) || hybrid_plain_cfg<REAL>(g, cfg);
 }
 
-// Shape of the ADI x sweeps, shared by the array step's x solve and the
-// matrix-free x sweep so that the two steps agree bit for bit. An x line
+// Shape of the array step's x solve and of the matrix-free x sweep that takes the lines
+// adi_xvec_kernel does not. An x line
 // fits one workgroup easily; what costs is the PCR across its lanes (a
 // division per step and lane), so fewer lanes of more rows than the general
 // contiguous default (up to 64 lanes of 4 rows at 256 rows) pay off. Measured
@@ -931,8 +933,8 @@ tridStatus_t run(const TridParams *ctx, REAL lambda, REAL *u, REAL *du, REAL *a,
   // a == NULL selects the matrix-free step. The array step's coefficient
   // arrays do not change from step to step: where its sweeps are matrix-free,
   // they are written once before the steps. 256^3, per step, against
-  // preproc and the array solves in every step: FP64 0.178 against 0.605 ms,
-  // FP32 0.104 against 0.276; a call of 20 FP64 steps 3.75 against 12.3 ms.
+  // preproc and the array solves in every step: FP64 0.150 against 0.605 ms,
+  // FP32 0.081 against 0.276; a call of 20 FP64 steps 3.10 against 12.3 ms.
   if (iters < 0) return TRID_STATUS_INVALID_VALUE;
   hipStream_t st = current_stream();
   tridStatus_t s = TRID_STATUS_SUCCESS;

@@ -118,8 +118,8 @@ __global__ __launch_bounds__((AdjBounds<REAL, M>::threads)) void adjoint_kernel(
 // come in two registers. The four outputs are written one array after the other
 // (256^3 FP64 y 231 against 237 us with all four row by row). Every output
 // stream is as long as an input's: with all gradients, nine streams at 256^3
-// FP64, y / z run at 5.2 / 4.9 TB/s, 231 / 246 us, against 251 / 261 with every
-// operand in registers (adjoint_kernel); lam alone at 5.9 TB/s (z 115 us).
+// FP64, y / z run at 5.3 / 5.0 TB/s, 227 / 241 us, against 234 / 262 with every
+// operand in registers (adjoint_kernel); lam alone at 6.2 TB/s (z 108 us against 147).
 template <typename REAL, int M, int SEG, bool GRAD, bool NT>
 __global__ __launch_bounds__((wide::WideBounds<REAL, M>::threads)) void adjoint_wide_kernel(
     Geom g, int P, int G, int slots, const REAL *__restrict__ a, const REAL *__restrict__ b,

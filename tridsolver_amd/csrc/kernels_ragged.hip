@@ -464,8 +464,9 @@ __device__ __forceinline__ void rg_item_segments(const RgMeta &cur, unsigned cha
 // HBM: with the plan's four launches (19 us), FP64, 40 M unknowns in systems of
 // 4096 rows 291 us, of 2048 (M = 8) 286; lengths of 2049-4096 at random 153 us for
 // 17.7 M unknowns, of 4097-8192 206 us for 23.6 M. What is left over the floor is
-// the last class's idle lanes (a system fills its power of two of lanes to 3/4
-// on average) and the plan. One 512- or 1024-thread workgroup per CU that took items
+// idle lanes (a system fills its power of two of lanes to 3/4 on average; 40 M FP64
+// unknowns in systems of 4096 / 3072 / 2064 rows, max_len 8192: 291 / 334 / 457 us)
+// and the plan. One 512- or 1024-thread workgroup per CU that took items
 // from an atomic counter: 412 and 406 us for the first two.
 template <typename REAL, int M, bool LONG32>
 constexpr size_t rg_each_lds_bytes() {
@@ -902,8 +903,6 @@ hipError_t launch_ragged_mixed(int M, const double *a, const double *b, const do
 size_t ragged_workspace_bytes(int64_t S) {
   return RAGGED_PLAN_HEADER_BYTES + sizeof(int) * (size_t)std::max<int64_t>(S, 1);
 }
-
-
 
 int ragged_max_len(int fp64, int M) {
   (void)fp64;  // the same shapes at both precisions

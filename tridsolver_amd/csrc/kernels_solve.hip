@@ -402,8 +402,8 @@ bool hybrid_wide_default_cfg(const Geom &g, HybridCfg *cfg) {
   //  - FP64 at 16 rows per lane (512^3 z 0.94 against 0.95 ms at 32, 251 x
   //    300 x 300 y 213 against 222 us). FP32 at 32 rows per lane on 256-byte
   //    rows of 321-512 (512^3 y 0.466 against 0.484 ms for 16 on 128-byte
-  //    rows, 592 x 320 x 128 y 108.7 against 107.2 us, 320 x 272 x 256 y 83.6 against
-  //    77.8; given 1024 such workgroups: 200 x 300 x 150 y, 600, 56 against 48
+  //    rows, but at 320 rows, 592 x 128 y, 108.7 against 107.2 us, at 272, 320 x 256 y,
+  //    83.6 against 77.8; given 1024 such workgroups: 200 x 300 x 150 y, 600, 56 against 48
   //    us) and above 512, else at 16 on 128-byte rows (203 x 170 x 300 y 52
   //    against 55 us).
   //  - workgroups dealt to the XCDs in 8 ranges (G), so that neighbouring

@@ -186,8 +186,7 @@ __device__ __forceinline__ void mixed_chunk_acc(const hyb::Lane &L, hyb::Ring &r
   }
 }
 
-// All four operands in registers.
-// The same for FP32 operands and at most one refinement, which keeps x0 in FP32
+// mixed_chunk_acc for FP32 operands and at most one refinement, which keeps x0 in FP32
 // registers (its FP64 value is exact) and forms x = x0 + dx in FP64 only at the
 // end. Factorisation and the first solve are one sweep in row order, so that it can
 // follow loads in flight (hyb::sweep_carry's form: the chunk's first unknown is carried
@@ -313,6 +312,7 @@ __device__ __forceinline__ void mixed_solve(const hyb::Lane &L, hyb::Ring &ring,
   else mixed_chunk_acc<M, STEPS, false, true>(L, ring, Aof, B, Cof, D, refine, X);
 }
 
+// All four operands in registers.
 template <int M>
 __device__ __forceinline__ void mixed_chunk(const hyb::Lane &L, hyb::Ring &ring,
                                             const double (&A)[M], const double (&B)[M],
